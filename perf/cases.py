@@ -144,3 +144,42 @@ def tolerance(case):
     1.6e-6 elementwise (coefficients near one), fp16 2.1e-4 and 4.9e-4, bf16 1.7e-3 and 3.9e-3 (one rounding)."""
     rel, largest = {"f32": (6e-7, 6e-6), "f16": (8e-4, 2e-3), "bf16": (7e-3, 1.6e-2)}[case["dtype"]]
     return {"rel": rel, "max": largest}
+
+
+def _scan64(inputs, coeffs):
+    """The recurrence along the last axis in float64, by doubling: after the step of distance d every position
+    holds the map from 2d positions before it."""
+    b, a = inputs.clone(), coeffs.clone()
+    a[..., 0] = 0.0
+    d = 1
+    while d < b.shape[-1]:
+        step = a[..., d:] * b[..., :-d]
+        b[..., d:] += step
+        step = a[..., d:] * a[..., :-d]
+        a[..., d:] = step
+        d *= 2
+    return b
+
+
+def exact(case, seed):
+    """Outputs and gradients by the recurrence in float64, from the inputs in their storage type."""
+    state = prepare(case, seed)
+    scan_axis = state["dim"]
+
+    def rows(t):  # the scan axis last and running forward
+        t = t.detach().double().movedim(scan_axis, -1)
+        return t.flip(-1) if case["reverse"] else t
+
+    def back(t):
+        return (t.flip(-1) if case["reverse"] else t).movedim(-1, scan_axis)
+
+    inputs, coeffs = rows(state["inputs"]), rows(state["coeffs"])
+    outputs = _scan64(inputs, coeffs)
+    if not case["grad"]:
+        return back(outputs)
+    # position l of the gradient's recurrence runs backward and takes the coefficient of l + 1
+    shifted = torch.cat([coeffs[..., 1:], torch.zeros_like(coeffs[..., :1])], -1)
+    d_inputs = _scan64(rows(state["d_outputs"]).flip(-1), shifted.flip(-1)).flip(-1)
+    d_coeffs = torch.zeros_like(d_inputs)
+    d_coeffs[..., 1:] = d_inputs[..., 1:] * outputs[..., :-1]
+    return back(outputs), back(d_inputs), back(d_coeffs)
