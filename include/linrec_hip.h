@@ -59,7 +59,10 @@ extern "C" {
 #define LINREC_FAMILY_SEGMENT 8 /* as COLUMN for few rows: the scan axis is cut into segments that run side by
                                   side (reduce, carry, apply: three launches).  Tuning: `waves` = rows per
                                   lane, `slots` = timesteps in flight, `tasks` = segments (at most 4096).
-                                  In the plan, `tiles_per_row` = segments, `tasks` = positions per segment */
+                                  In the plan, `tiles_per_row` = segments, `tasks` = positions per segment.
+                                  `carry` = 1: in one launch, the segments of a row chained by look-back.
+                                  Tuning: `waves` = rows per lane, `slots` = positions per run, `tasks` = waves
+                                  per workgroup; a segment is waves * run positions of 64 lanes' rows */
 #define LINREC_FAMILY_FLAT 9    /* dense short rows (row stride == row length <= 240 floats, 16-byte aligned
                                   bases): the tensor as one flat array of full slots, the scan cut at the row
                                   starts by the unused coefficient there.  Tuning: `slots` = rows of 64 slots

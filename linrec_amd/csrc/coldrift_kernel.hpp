@@ -73,10 +73,15 @@ __device__ __forceinline__ Lanes<VEC> widen(const Held<T, VEC>& h) {
 // compiler would rather keep the widened values, two registers for one).
 template <typename T, int VEC>
 __device__ __forceinline__ Held<T, VEC> held_again(Held<T, VEC> h) {
-  if constexpr (!std::is_same_v<T, float> && sizeof(typename Pack<T, VEC>::type) == 4) {
+  using V = typename Pack<T, VEC>::type;
+  if constexpr (!std::is_same_v<T, float> && sizeof(V) == 4) {
     uint32_t bits = __builtin_bit_cast(uint32_t, h.q);
     asm volatile("" : "+v"(bits));
-    h.q = __builtin_bit_cast(typename Pack<T, VEC>::type, bits);
+    h.q = __builtin_bit_cast(V, bits);
+  } else if constexpr (!std::is_same_v<T, float> && sizeof(V) == 8) {
+    uint64_t bits = __builtin_bit_cast(uint64_t, h.q);
+    asm volatile("" : "+v"(bits));
+    h.q = __builtin_bit_cast(V, bits);
   }
   return h;
 }

@@ -1,0 +1,276 @@
+// Segments of a strided scan axis in one launch: the scan axis is cut into segments of NW * U positions, a
+// workgroup takes one segment of 64 * VEC adjacent rows (wave w the run [w*U, w*U + U) of every row), and the
+// segments of a row are chained by decoupled look-back, row by row, through descriptors in global memory.
+//   1. every lane loads its run, folds it into an affine map value_out = a * value_in + b, the maps go to LDS;
+//   2. waves 0 .. VEC-1 (wave e: row e of every lane) compose the NW maps of a row, publish them, walk back over
+//      the segments before until one has published the value that leaves it, and publish what leaves their own;
+//   3. every wave composes the maps of the waves before it onto that value, walks its run again and stores.
+// The data stays in registers (packed in 16-bit storage) between 1 and 3, so every tensor is read and written
+// once: 12 / 20 bytes per element where the three launches (reduce, carry, apply: column_kernel.hpp) move 20 / 28.
+//
+// What bounds it: memory, and for a launch of a few microseconds the chain load -> publish -> look back -> store.
+// Workgroups are numbered segment by segment, all blocks of rows of one segment next to each other: the launch
+// sweeps the tensors in the order of their addresses (a matrix with its scan axis strided is stored segment after
+// segment), and the segment a workgroup looks back to was started one whole round of blocks earlier.
+//
+// Measured (bf16, 4096 positions x 2048 rows, forward / backward): 12.6 / 18.8 us, 4.0 / 4.5 TB/s, where the three
+// launches take 26.3 / 36.0; 8 x 4096 x 1024: 38 / 60 us, 5.3 / 5.6 TB/s, where the column drift kernels take 54 / 76.5;
+// fp32 16 x 2048 x 512: 38 / 63 us, 5.3 / 5.3 TB/s, where column blocks / drift take 43 / 69.  The same kernel without
+// the look-back takes 11.7 / 18.1, 37.9 / 60.8 and 38.1 / 62.8 us: what is left to the rate of a plain stream is the
+// width of the accesses (two rows to a lane instead of four: 46 / 73 us on the second shape) and the one workgroup
+// per CU, whose loads and stores do not overlap.  16 waves and runs as long as the registers hold beat smaller
+// workgroups of which several share a CU (8 waves, the second shape: 47 / 77 us): descriptors per byte halve.
+//
+// A segment only waits for segments with smaller numbers, which are started first; every wait is bounded, and a
+// lane whose wait runs out computes what enters its row from the row's own data.
+//
+// The reference has no strided kernel (linrec/impl/cuda/linrec_pipe.cu:35) and never splits a row.
+#pragma once
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include <type_traits>
+
+#include "coldrift_kernel.hpp"  // ColDriftArgs, Held
+
+namespace linrec {
+
+constexpr int PHASE_LOOKBACK = 3;  // the kernel table's code beside PHASE_REDUCE and PHASE_APPLY
+
+// (of args.chain: tasks = blocks of rows, num_tiles = workgroups)
+template <typename T, int VEC, int U, int NW, int MODE, bool DESC>
+__global__ __launch_bounds__(64 * NW) void collook_kernel(ColDriftArgs args) {
+  static_assert(VEC <= NW, "a wave per row of a lane looks back");
+  const ColumnArgs& p = args.col;
+  const TileArgs& ch = args.chain;
+  constexpr int RPB = 64 * VEC;  // rows of a block
+  constexpr int STEP = NW * U;   // positions of a segment
+  constexpr bool NEED_Y = MODE == 1;
+  // segments asked for in one round trip: one where the run itself takes most of the 128 registers there are
+  constexpr int LOOK = U * VEC * int(sizeof(T)) / 4 * (NEED_Y ? 3 : 2) <= 48 ? 4 : 1;
+  __shared__ float sh_a[NW][RPB];
+  __shared__ float sh_b[NW][RPB];
+  __shared__ float sh_in[RPB];  // the value entering the segment
+
+  const T* in0 = static_cast<const T*>(p.in0);
+  const T* coef = static_cast<const T*>(p.coef);
+  const T* aux = static_cast<const T*>(p.aux);
+  T* out0 = static_cast<T*>(p.out0);
+  T* out1 = static_cast<T*>(p.out1);
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int blocks = ch.tasks;
+  const int k = int(blockIdx.x / unsigned(blocks));  // segment
+  const int block = int(blockIdx.x - unsigned(k) * unsigned(blocks));
+  auto base_of = [&](long long row) __attribute__((always_inline)) {
+    if (p.rows_per_batch >= p.numseq) return row * p.row_stride;
+    const long long batch = row / p.rows_per_batch;
+    return batch * p.batch_stride + (row - batch * p.rows_per_batch) * p.row_stride;
+  };
+  long long r0 = ((long long)block * 64 + lane) * VEC;
+  const bool active = r0 < p.numseq;
+  if (!active) r0 = p.numseq - VEC;  // lanes beyond the last row read the last rows again and store nothing
+  // A wave's accesses are a scalar address plus 32 bits per lane (the planner sees to it that a block's rows span
+  // less than 2^31 bytes): 64-bit addresses per lane took 30 to 40 registers, and with them a workgroup per CU.
+  const long long base = base_of(r0);
+  const long long wbase = (long long)(uint32_t)__builtin_amdgcn_readfirstlane(int(base)) |
+                          ((long long)__builtin_amdgcn_readfirstlane(int(base >> 32)) << 32);
+  const uint32_t lane_bytes = uint32_t(base - wbase) * uint32_t(sizeof(T));
+  const int L = p.seqlen;
+  auto at = [&](auto* tensor, int l) __attribute__((always_inline)) {
+    using P = decltype(tensor);
+    using C = std::conditional_t<std::is_const_v<std::remove_pointer_t<P>>, const char*, char*>;
+    return reinterpret_cast<P>(reinterpret_cast<C>(tensor + (wbase + (long long)l * p.elem_stride)) + lane_bytes);
+  };
+  const int ksteps = (L + STEP - 1) / STEP;
+  const uint32_t seq = load_seq_through_caches(ch.ws);
+  const uint32_t want = (seq << 2) | STATUS_AGGREGATE, done = (seq << 2) | STATUS_INCLUSIVE;
+  // descriptors of segment s of this block: the first words of all rows, then the second words (a wave stores whole
+  // lines of them), row e of lane i in place e * 64 + i
+  auto desc_of = [&](int s) __attribute__((always_inline)) { return ch.desc + 2 * ((long long)s * blocks + block) * RPB; };
+
+  struct Batch {
+    Held<T, VEC> x[U], c[U], yn[NEED_Y ? U : 1];
+  };
+  const int n0 = k * STEP + wave * U;
+  // FULL: all positions of the segment exist and, for the backward, so does the last one's successor.
+  auto segment = [&](auto full_tag) __attribute__((always_inline)) {
+    constexpr bool FULL = decltype(full_tag)::value;
+    Batch bt;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int n = n0 + u;  // position in scan order
+      const int l = DESC ? L - 1 - n : n;
+      if (FULL || n < L) {
+        bt.x[u] = ld_held<VEC>(at(in0, l));
+        bt.c[u] = ld_held<VEC>(at(coef, l));
+        if constexpr (NEED_Y) {
+          const int ln = DESC ? l - 1 : l + 1;  // saved output one step further along this scan
+          if (FULL || (ln >= 0 && ln < L)) {
+            bt.yn[u] = ld_held<VEC>(at(aux, ln));
+          } else {
+            bt.yn[u] = held_zero<T, VEC>();
+          }
+        }
+      }
+    }
+    Lanes<VEC> ma, mb;
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) {
+      ma.v[e] = 1.0f;
+      mb.v[e] = 0.0f;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int n = n0 + u;
+      if (FULL || n < L) {
+        const Lanes<VEC> x = widen(bt.x[u]), c = widen(bt.c[u]);
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) {
+          if constexpr (MODE == 0) {
+            // the coefficient of the first position takes no part (linrec_ref.cuh:63)
+            mb.v[e] = n == 0 ? x.v[e] : fmaf(mb.v[e], c.v[e], x.v[e]);
+            ma.v[e] = n == 0 ? 0.0f : ma.v[e] * c.v[e];
+          } else {
+            mb.v[e] = (mb.v[e] + x.v[e]) * c.v[e];
+            ma.v[e] *= c.v[e];
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) {
+      sh_a[wave][e * 64 + lane] = ma.v[e];
+      sh_b[wave][e * 64 + lane] = mb.v[e];
+    }
+    __syncthreads();
+    if (wave < VEC) {
+      const int i = wave * 64 + lane;
+      float ta = sh_a[0][i], tb = sh_b[0][i];
+#pragma unroll 4
+      for (int w = 1; w < NW; ++w) {
+        tb = fmaf(tb, sh_a[w][i], sh_b[w][i]);
+        ta *= sh_a[w][i];
+      }
+      uint64_t* mine = desc_of(k) + i;
+      float entering = 0.0f;
+      if (k == 0) {
+        if (ksteps > 1) st_desc(mine + RPB, pack_desc(done, tb));
+      } else {
+        if (k + 1 < ksteps) {
+          st_desc(mine, pack_desc(want, ta));
+          st_desc(mine + RPB, pack_desc(want, tb));
+        }
+        // (acc_a, acc_b): the segments j+1 .. k-1 composed.  The wave walks back as one, so the words' addresses
+        // are scalar; a lane that has found its value ignores what else is read.
+        float acc_a = 1.0f, acc_b = 0.0f;
+        int j = k - 1, polls = 0;
+        bool found = false;
+        for (;;) {
+          uint64_t w0[LOOK], w1[LOOK];
+#pragma unroll
+          for (int q = 0; q < LOOK; ++q) {
+            const uint64_t* d = desc_of(j >= q ? j - q : 0);  // (beyond segment 0: asked for again, not used)
+            w0[q] = ld_desc(d + i);
+            w1[q] = ld_desc(d + RPB + i);
+          }
+          int moved = 0;
+#pragma unroll
+          for (int q = 0; q < LOOK; ++q) {
+            const uint32_t f1 = uint32_t(w1[q] >> 32);
+            const bool there = f1 == done || (f1 == want && uint32_t(w0[q] >> 32) == want);
+            if (moved == q && __ballot(!found && !there) == 0) {
+              const float b = __builtin_bit_cast(float, uint32_t(w1[q]));
+              if (!found) {
+                if (f1 == done) {  // (segment 0 always publishes what leaves it, so the walk never goes past it)
+                  entering = fmaf(b, acc_a, acc_b);
+                  found = true;
+                } else {
+                  acc_b = fmaf(b, acc_a, acc_b);
+                  acc_a *= __builtin_bit_cast(float, uint32_t(w0[q]));
+                }
+              }
+              ++moved;
+            }
+          }
+          if (__ballot(!found) == 0) break;
+          j -= moved;
+          if (moved > 0) {
+            polls = 0;
+          } else {
+            if (++polls >= ch.spin_limit) break;
+            __builtin_amdgcn_s_sleep(1);
+          }
+        }
+        const uint64_t late = __ballot(!found);
+        if (late) {
+          if (lane == 0) __hip_atomic_fetch_add(&ch.ws->gave_up, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          if (!found) {
+            // what enters the segment from the row's own data: the plain sequential walk
+            const long long row = r0 + (VEC > 1 ? wave : 0);
+            const long long rb = base_of(row);
+            float val = 0.0f;
+            for (int n = 0; n < k * STEP; ++n) {
+              const int l = DESC ? L - 1 - n : n;
+              const long long off = rb + (long long)l * p.elem_stride;
+              const float x = float(in0[off]), c = float(coef[off]);
+              if constexpr (MODE == 0) val = n == 0 ? x : fmaf(val, c, x);
+              else val = (val + x) * c;
+            }
+            entering = val;
+          }
+        }
+        if (k + 1 < ksteps) st_desc(mine + RPB, pack_desc(done, fmaf(entering, ta, tb)));
+      }
+      sh_in[i] = entering;
+    }
+    __syncthreads();
+    Lanes<VEC> val;
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) val.v[e] = sh_in[e * 64 + lane];
+    for (int w = 0; w < wave; ++w) {
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) {
+        const float a = sh_a[w][e * 64 + lane], b = sh_b[w][e * 64 + lane];
+        // before the first map of a row there is nothing: its b is taken as it is, so that 0 * inf can never arise
+        val.v[e] = (k == 0 && w == 0) ? b : fmaf(val.v[e], a, b);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int n = n0 + u;
+      const int l = DESC ? L - 1 - n : n;
+      if (FULL || n < L) {
+        const Lanes<VEC> x = widen(held_again(bt.x[u])), c = widen(held_again(bt.c[u]));
+        if constexpr (MODE == 0) {
+#pragma unroll
+          for (int e = 0; e < VEC; ++e) val.v[e] = n == 0 ? x.v[e] : fmaf(val.v[e], c.v[e], x.v[e]);
+          if (active) st_rows<VEC>(at(out0, l), val);
+        } else {
+          const Lanes<VEC> yn = widen(held_again(bt.yn[u]));
+          Lanes<VEC> dx, dc;
+#pragma unroll
+          for (int e = 0; e < VEC; ++e) {
+            dx.v[e] = val.v[e] + x.v[e];
+            dc.v[e] = dx.v[e] * yn.v[e];
+            val.v[e] = dx.v[e] * c.v[e];
+          }
+          if (active) {
+            st_rows<VEC>(at(out0, l), dx);
+            st_rows<VEC>(at(out1, l), dc);
+          }
+        }
+      }
+    }
+  };
+  if ((k + 1) * (long long)STEP <= (NEED_Y ? L - 1 : L)) segment(std::true_type{});
+  else segment(std::false_type{});
+
+  // (the look-back waves are past the last barrier: no descriptor of this launch is touched by this workgroup again)
+  if (threadIdx.x == 0) {
+    const uint32_t leaf_count = signal_tile_done_begin(ch, blockIdx.x);
+    signal_tile_done_end(ch, blockIdx.x, seq, leaf_count);
+  }
+}
+
+}  // namespace linrec

@@ -149,6 +149,16 @@ KernelGroup kernels_bf16_cols();
   SEGMENT_PHASES(TT, DT, PFX, VEC, U, MODE_FWD, 0), SEGMENT_PHASES(TT, DT, PFX, VEC, U, MODE_FWD, 1), \
   SEGMENT_PHASES(TT, DT, PFX, VEC, U, MODE_BWD, 0), SEGMENT_PHASES(TT, DT, PFX, VEC, U, MODE_BWD, 1)
 
+// ... in one launch, the segments of a row chained by look-back
+#define COLLOOK_ENTRY(TT, DT, PFX, NW, VEC, U, MODE, DESC)                                     \
+  {PFX "segment_lookback_w" #NW "_v" #VEC "_u" #U "_" #MODE "_" #DESC,                         \
+   (const void*)&linrec::collook_kernel<TT, VEC, U, NW, linrec::MODE, DESC != 0>, DT,          \
+   LINREC_FAMILY_SEGMENT, NW, U, VEC, linrec::MODE, DESC, linrec::PHASE_LOOKBACK}
+#define COLLOOK_FWD_DIRS(TT, DT, PFX, NW, VEC, U)                                              \
+  COLLOOK_ENTRY(TT, DT, PFX, NW, VEC, U, MODE_FWD, 0), COLLOOK_ENTRY(TT, DT, PFX, NW, VEC, U, MODE_FWD, 1)
+#define COLLOOK_BWD_DIRS(TT, DT, PFX, NW, VEC, U)                                              \
+  COLLOOK_ENTRY(TT, DT, PFX, NW, VEC, U, MODE_BWD, 0), COLLOOK_ENTRY(TT, DT, PFX, NW, VEC, U, MODE_BWD, 1)
+
 #define F32 float, LINREC_DTYPE_F32, ""
 #define F16 _Float16, LINREC_DTYPE_F16, "f16_"
 #define BF16 __bf16, LINREC_DTYPE_BF16, "bf16_"
@@ -169,8 +179,15 @@ KernelGroup kernels_bf16_cols();
 #define SEGMENT_(...) SEGMENT_ALL_DIRS(__VA_ARGS__)
 #define COLDRIFT_FWD_(...) COLDRIFT_FWD_DIRS(__VA_ARGS__)
 #define COLDRIFT_BWD_(...) COLDRIFT_BWD_DIRS(__VA_ARGS__)
+#define COLLOOK_FWD_(...) COLLOOK_FWD_DIRS(__VA_ARGS__)
+#define COLLOOK_BWD_(...) COLLOOK_BWD_DIRS(__VA_ARGS__)
 #define COLBLOCK_FWD_(...) COLBLOCK_FWD_DIRS(__VA_ARGS__)
 #define COLBLOCK_BWD_(...) COLBLOCK_BWD_DIRS(__VA_ARGS__)
+
+// (one row to a lane: odd row counts, and too few rows for anything wider; sixteen waves instead of eight: less
+// than 5 % either way on a dozen shapes, not kept)
+#define COLLOOK_NARROW_KERNELS(...)                                                            \
+  COLLOOK_FWD_(__VA_ARGS__, 8, 1, 16), COLLOOK_BWD_(__VA_ARGS__, 8, 1, 16)
 
 // The 16-bit storage types get the geometries the planner picks for them (their register tiles are
 // twice as wide as fp32's, so two slots of eight elements per lane is the rule; the forward team
@@ -187,7 +204,8 @@ KernelGroup kernels_bf16_cols();
   COLUMN_(TY, 8, 4), COLUMN_(TY, 4, 8), COLUMN_(TY, 2, 8), COLUMN_(TY, 2, 16), COLUMN_(TY, 1, 8), COLUMN_(TY, 1, 16), \
   SEGMENT_(TY, 4, 8), SEGMENT_(TY, 2, 8), SEGMENT_(TY, 1, 8),                                   \
   COLBLOCK_FWD_(TY, 2, 8, 1), COLBLOCK_BWD_(TY, 2, 4, 1), COLBLOCK_FWD_(TY, 2, 8, 2), COLBLOCK_BWD_(TY, 2, 4, 2), \
-  COLDRIFT_FWD_(TY, 16, 2, 8), COLDRIFT_BWD_(TY, 8, 2, 16), COLDRIFT_FWD_(TY, 8, 2, 16), COLDRIFT_BWD_(TY, 16, 2, 4)
+  COLDRIFT_FWD_(TY, 16, 2, 8), COLDRIFT_BWD_(TY, 8, 2, 16), COLDRIFT_FWD_(TY, 8, 2, 16), COLDRIFT_BWD_(TY, 16, 2, 4), \
+  COLLOOK_NARROW_KERNELS(TY), COLLOOK_FWD_(TY, 16, 2, 16), COLLOOK_BWD_(TY, 16, 2, 16), COLLOOK_FWD_(TY, 16, 4, 16), COLLOOK_BWD_(TY, 16, 4, 16)
 
 #define LINREC_KERNEL_GROUP(NAME, ...)                                                          \
   namespace linrec {                                                                            \

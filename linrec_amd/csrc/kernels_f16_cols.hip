@@ -6,6 +6,7 @@
 #include "column_kernel.hpp"
 #include "colblock_kernel.hpp"
 #include "coldrift_kernel.hpp"
+#include "collook_kernel.hpp"
 #include "kernel_table.hpp"
 
 LINREC_KERNEL_GROUP(kernels_f16_cols,

@@ -6,6 +6,7 @@
 #include "column_kernel.hpp"
 #include "colblock_kernel.hpp"
 #include "coldrift_kernel.hpp"
+#include "collook_kernel.hpp"
 #include "kernel_table.hpp"
 
 LINREC_KERNEL_GROUP(kernels_f32_cols,
@@ -30,5 +31,7 @@ LINREC_KERNEL_GROUP(kernels_f32_cols,
     // (nor two rows per lane with runs of 4 positions in 16 waves, whose 512-byte accesses a memory-only kernel
     // likes better by 14 %: twice the team and half the positions per step make four times the exchange,
     // 4096 x 16384 forward 187 against 157 us, 2048 x 16384 124 against 85.3 us, 8192 x 4096 89.6 against 82.7 us)
-    COLDRIFT_FWD_(F32, 16, 1, 8), COLDRIFT_BWD_(F32, 16, 1, 4), COLDRIFT_FWD_(F32, 8, 1, 16), COLDRIFT_BWD_(F32, 8, 1, 16)
+    COLDRIFT_FWD_(F32, 16, 1, 8), COLDRIFT_BWD_(F32, 16, 1, 4), COLDRIFT_FWD_(F32, 8, 1, 16), COLDRIFT_BWD_(F32, 8, 1, 16),
+    // segments in one launch, chained by look-back
+    COLLOOK_NARROW_KERNELS(F32), COLLOOK_FWD_(F32, 16, 2, 16), COLLOOK_BWD_(F32, 16, 2, 8), COLLOOK_BWD_(F32, 16, 4, 8)
 )

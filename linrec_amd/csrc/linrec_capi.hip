@@ -14,6 +14,7 @@
 #include "kernel_table.hpp"
 #include "colblock_kernel.hpp"
 #include "coldrift_kernel.hpp"
+#include "collook_kernel.hpp"
 #include "column_kernel.hpp"
 #include "flat_kernel.hpp"
 #include "drift_kernel.hpp"
@@ -60,7 +61,8 @@ int find_kernel(int dtype, int family, int waves, int slots, int vec, int mode, 
     const KernelEntry& k = kKernels[i];
     const bool waves_matter = family == LINREC_FAMILY_TILE || family == LINREC_FAMILY_STREAM ||
                               family == LINREC_FAMILY_TEAM || family == LINREC_FAMILY_SWEEP || family == LINREC_FAMILY_DRIFT || family == LINREC_FAMILY_GROUP ||
-                              family == LINREC_FAMILY_FLAT || family == LINREC_FAMILY_COLDRIFT;
+                              family == LINREC_FAMILY_FLAT || family == LINREC_FAMILY_COLDRIFT ||
+                              (family == LINREC_FAMILY_SEGMENT && carry == linrec::PHASE_LOOKBACK);
     if (k.dtype == dtype && k.family == family && k.slots == slots && k.vec == vec && k.mode == mode &&
         k.desc == desc && k.carry == carry && (!waves_matter || k.waves == waves))
       return i;
@@ -618,6 +620,89 @@ bool coldrift_applies(const Problem& q) {
   if (team > 8) return blocks * team * 8 >= 7 * q.cus;
   return blocks * team * 20 >= 13 * q.cus;
 }
+// The plan of a segmented launch whose segments are chained by look-back (one launch): `waves` waves per workgroup
+// with runs of `depth` positions, `vec` rows to a lane.
+int lookback_segments_plan(const Problem& q, int vec, int waves, int depth, int mode, int desc, linrec_plan_t* out) {
+  if (vec < 1 || colblock_rows_per_lane(q, vec) != vec) return LINREC_E_UNSUPPORTED;
+  // (a lane's offset from its wave's first row is 32 bits of bytes: strides forward, a block's rows within 2^31 bytes)
+  {
+    const int64_t rpb = q.batched() ? q.rows_per_batch : q.numseq, rows = 64 * int64_t(vec);
+    if (q.row_stride < 0 || (q.batched() && q.batch_stride < rpb * q.row_stride)) return LINREC_E_UNSUPPORTED;
+    const int64_t bound = (int64_t(1) << 31) / elem_size_of(q.dtype);
+    if (q.row_stride > bound / rows || (q.batched() && q.batch_stride > bound / 2 / (rows / rpb + 2)) || q.row_stride * rows > bound / 2)
+      return LINREC_E_UNSUPPORTED;
+  }
+  const int id = find_kernel(q.dtype, LINREC_FAMILY_SEGMENT, waves, depth, vec, mode, desc, linrec::PHASE_LOOKBACK);
+  if (id < 0) return LINREC_E_UNSUPPORTED;
+  const int64_t rows_per_block = int64_t(64) * vec;
+  const int64_t blocks = ceil_div(q.numseq, rows_per_block);
+  const int64_t segments = ceil_div(q.seqlen, int64_t(waves) * depth);
+  if (blocks * segments * rows_per_block > 2147483647LL) return LINREC_E_TOO_LARGE;
+  out->family = LINREC_FAMILY_SEGMENT;
+  out->waves = waves; out->slots = depth; out->vec = vec; out->carry = 1;
+  out->tiles_per_row = int32_t(segments);
+  out->tasks = waves * depth;
+  out->grid = blocks * segments;
+  out->block = 64 * waves;
+  out->kernel_id = id;
+  out->workspace_bytes = linrec_workspace_bytes_for_tiles(blocks * segments * rows_per_block);
+  return LINREC_OK;
+}
+
+// Whether the planner takes look-back segments for this problem (`family`: what the rules above chose), and with
+// which geometry.  One pass over the tensors, no three launches, and workgroups that need not divide the chip: they
+// win wherever the alternative reads its inputs twice, leaves part of the chip without a workgroup, or takes narrow
+// accesses that straddle lines.  Forward / backward in us against what was chosen before:
+//   few rows, a launch of microseconds: bf16 1 x 4096 x 2048 (batch x time x channels) 12.6 / 18.8 against 26.3 /
+//     36.0 (segments in three launches), fp32 8 x 1024 x 256 10.4 / 11.9 against 14.8 / 18.1, bf16 5 x 777 x 1001
+//     13.9 / 20.5 against 25.3 / 31.8;
+//   up to 8192 rows (16-bit storage: 16384): fp32 16 x 2048 x 512 39.7 / 64.2 against 43.2 / 70.0 (column blocks,
+//     column drift), 2 x 8192 x 700 38.7 / 56.7 against 47.5 / 72.7, bf16 8 x 4096 x 1024 43.2 / 61.6 against 55.0 /
+//     76.7 (column drift), 4 x 4096 x 4096 82.3 / 142.6 against 86.9 / 151.5 (column blocks);
+//   more rows: where a position's rows do not start on a 128-byte line, fp32 30 x 1024 x 1500 136.1 / 198.0 against
+//     168.9 / 291.4, bf16 7 x 4096 x 3500 161.7 / 280.7 against 218.0 / 404.1, 30 x 1111 x 2000 104.2 / 177.6 against
+//     118.8 / 221.2; where it does, the column blocks are as good or better (fp32 4 x 4096 x 4096 145.6 / 238.8 against
+//     135.6 / 239.0, 7 x 2048 x 4000 130.9 / 197.8 against 124.1 / 193.1, bf16 32 x 1024 x 1024 43.1 / 64.2 against 37.0 /
+//     63.9), and with one row to a lane they are from 16384 rows on (fp32 31 x 600 x 777 64.7 / 112.2 against 61.4 /
+//     111.4; 16-bit storage, which has no column block for that, from 32768: bf16 8 x 1024 x 4097 95.7 against 91.8);
+//   a forward of less than 1024 positions stays with the column blocks (fp32 8 x 700 x 1024 16.2 against 16.2) and one
+//     of less than 4096 with the column drift teams where those apply (fp32 3 x 2100 x 1344 25.5 against 26.3; bf16
+//     3 x 2100 x 2688 would gain, 25.4 against 31.5).
+// One matrix (not a batch of them): 16-bit storage where the three launches were chosen, up to 8192 positions; the
+// rest stays with the teams and the three launches.
+bool lookback_segments_choose(const Problem& q, int family, bool colblock, int mode, int desc, linrec_plan_t* out) {
+  const bool half = q.dtype != LINREC_DTYPE_F32;
+  if (q.row_stride != 1 || q.seqlen < kSegmentMinLen) return false;
+  if (!q.batched()) {
+    if (!half || family != LINREC_FAMILY_SEGMENT || q.seqlen > 8192) return false;
+  } else {
+    if (!q.is_bwd && colblock && q.seqlen < 1024) return false;
+    if (!q.is_bwd && family == LINREC_FAMILY_COLDRIFT && q.seqlen < 4096) return false;
+    const bool pairs = colblock_rows_per_lane(q, 2) == 2;
+    const bool on_lines = q.elem_stride * elem_size_of(q.dtype) % 128 == 0;
+    const int64_t most = !pairs ? (half ? 32767 : 16384) : on_lines ? (half ? 16384 : 8192) : 65536;
+    if (q.numseq > q.at(most)) return false;
+  }
+  // The widest access that makes a workgroup for 5 of 8 CUs: it needs the fewest descriptors and the memory system
+  // likes it best (bf16 8 x 4096 x 1024 forward: 43.2 us with four rows to a lane, 47.6 with two, 51.7 with one), but
+  // half a chip is worse than a narrower access (bf16 1 x 4096 x 2048: 128 workgroups of four rows to a lane 17.4 us,
+  // 256 of two 13.7; fp32 2 x 4096 x 256 backward: 128 of two 14.4, 256 of one 12.9).
+  // {rows per lane, waves, positions per run}: the run as long as its tensors fit the registers
+  static const int shapes[2][2][3][3] = {{{{2, 16, 16}, {1, 8, 16}, {0, 0, 0}}, {{4, 16, 8}, {2, 16, 8}, {1, 8, 16}}},
+                                         {{{4, 16, 16}, {2, 16, 16}, {1, 8, 16}}, {{4, 16, 16}, {2, 16, 16}, {1, 8, 16}}}};
+  for (const auto& s : shapes[half][q.is_bwd != 0]) {
+    linrec_plan_t p;
+    std::memset(&p, 0, sizeof(p));
+    if (s[0] == 0 || lookback_segments_plan(q, s[0], s[1], s[2], mode, desc, &p) != LINREC_OK) continue;
+    if (s[0] > 1 && p.grid * 8 < 5 * q.cus) continue;
+    // (a caller that can only give so much workspace is served by the kernels that need less)
+    if (q.workspace_cap && p.workspace_bytes > q.workspace_cap) return false;
+    *out = p;
+    return true;
+  }
+  return false;
+}
+
 // The rows a second launch serves: the last `tail_rows` rows of `q`, as a problem of their own.
 Problem tail_problem(const Problem& q, int64_t tail_rows) {
   Problem t = q;
@@ -727,6 +812,7 @@ int make_plan(const Problem& q, const linrec_tuning_t* tune, linrec_plan_t* out)
         family = LINREC_FAMILY_COLDRIFT;
         use_colblock = 0;
       }
+      if (lookback_segments_choose(q, family, use_colblock != 0, mode, desc, out)) return LINREC_OK;
     } else {
       family = LINREC_FAMILY_NAIVE;
     }
@@ -992,6 +1078,9 @@ int make_plan(const Problem& q, const linrec_tuning_t* tune, linrec_plan_t* out)
   if (family == LINREC_FAMILY_SEGMENT) {
     if (q.elem_stride == 1 && q.seqlen != 1) return LINREC_E_UNSUPPORTED;
     const bool given = tune && tune->family == LINREC_FAMILY_SEGMENT;
+    // in one launch (tuning: `carry` = 1, `waves` = rows per lane, `slots` = positions per run, `tasks` = waves)
+    if (given && tune->carry == 1)
+      return lookback_segments_plan(q, tune->waves, tune->tasks, tune->slots, mode, desc, out);
     // rows per lane: 8 bytes' worth when that leaves at least a wave of lanes, fewer otherwise; fp32 from 512
     // rows on: four rows (16-byte accesses, a wave reads 1 KiB of every position), which the backward likes
     // (forward / backward in us, four rows against two at their best segment counts: 700 x 100000 278 / 409
@@ -1283,6 +1372,29 @@ int launch(const linrec_plan_t& plan, const Problem& q, const void* in0, const v
     d.col = a;
     d.chain.num_tiles = plan.grid;
     d.chain.tasks = plan.tasks;
+    d.chain.ws = static_cast<linrec::CarryHeader*>(workspace);
+    d.chain.counters = reinterpret_cast<uint32_t*>(static_cast<char*>(workspace) + lay.counters_offset);
+    d.chain.desc = reinterpret_cast<uint64_t*>(static_cast<char*>(workspace) + lay.desc_offset);
+    d.chain.ws_tiles = lay.tiles;
+    d.chain.spin_limit = g_spin_limit.load(std::memory_order_relaxed);
+    void* dargs[] = {&d};
+    hipError_t e = hipLaunchKernel(k.fn, dim3((unsigned)plan.grid), dim3((unsigned)plan.block), dargs, 0, stream);
+    return e == hipSuccess ? int(hipGetLastError()) : int(e);
+  }
+  if (plan.family == LINREC_FAMILY_SEGMENT && plan.carry == 1) {
+    const int64_t rows_per_block = int64_t(64) * k.vec;
+    const int64_t blocks = ceil_div(q.numseq, rows_per_block);
+    if (plan.block != 64 * k.waves || k.carry != linrec::PHASE_LOOKBACK || plan.tiles_per_row != ceil_div(q.seqlen, int64_t(k.waves) * k.slots) ||
+        plan.grid != blocks * plan.tiles_per_row)
+      return LINREC_E_INVALID;  // (what the kernel is compiled for)
+    if (!workspace || (reinterpret_cast<uintptr_t>(workspace) & 15u) || workspace_bytes < plan.workspace_bytes)
+      return LINREC_E_WORKSPACE;
+    const WorkspaceLayout lay = workspace_layout(workspace_bytes);
+    if (lay.tiles < plan.grid * rows_per_block) return LINREC_E_WORKSPACE;
+    linrec::ColDriftArgs d{};
+    d.col = a;
+    d.chain.num_tiles = plan.grid;
+    d.chain.tasks = int(blocks);
     d.chain.ws = static_cast<linrec::CarryHeader*>(workspace);
     d.chain.counters = reinterpret_cast<uint32_t*>(static_cast<char*>(workspace) + lay.counters_offset);
     d.chain.desc = reinterpret_cast<uint64_t*>(static_cast<char*>(workspace) + lay.desc_offset);

@@ -94,6 +94,9 @@ def candidates(t):
         for width in (1, 2, 4):
             for segments in (8, 32, 128, 512):
                 out.append((f"segment rows {width} x{segments}", nat.Tuning(nat.FAMILY_SEGMENT, width, 8, -1, segments)))
+        # ... in one launch, chained by look-back: rows per lane, positions per run, waves per workgroup
+        for width, run, w in ((4, 16, 16), (4, 8, 16), (2, 16, 16), (2, 8, 16), (1, 16, 8)):
+            out.append((f"segment look-back w{w} run {run} rows {width}", nat.Tuning(nat.FAMILY_SEGMENT, width, run, 1, w)))
     return out
 
 
