@@ -525,7 +525,8 @@ def _few_rows_on_strided_axis(t, lay, tuning):
 # everything that only depends on those: validation, the layout, the workspace size; what is left is the
 # pointers (which must be 16-byte aligned, as the results then are), the stream and one library call that takes
 # its arguments in one block of memory.  On a 64 x 4096 tensor, whose kernel takes 3 us, this halves the time
-# the host needs per launch.  Everything else takes the general path below.
+# the host needs per launch.  Batches of matrices ((batch, time, channels) data) are remembered likewise: working out
+# their layout and planning the workspace anew in every call cost as much as their kernels (8 x 4096 x 1024: 40 us a step).  Everything else takes the general path below.
 _repeat = threading.local()
 _REPEAT_MAX = 256
 
@@ -538,14 +539,20 @@ def _repeat_table():
 
 
 def _remember(table, key, lay, t, is_bwd, reverse):
-    """What a repeat of the call `key` needs: (Call, reference to it, workspace bytes), or None if calls of
-    this kind take the general path."""
+    """What a repeat of the call `key` needs, or None if calls of this kind take the general path.  `lay`: row_layout's
+    four numbers ((Call, reference to it, workspace bytes) is kept), or batched_layout's six ((None, the arguments before
+    the workspace, workspace bytes) is kept: one library call with the arguments spelled out)."""
     entry = None
-    if lay is not None:
+    if lay is not None and len(lay) == 4:
         call = Call(dtype=DTYPES[t.dtype], reverse=int(bool(reverse)), numseq=lay[0], seqlen=lay[1], row_stride=lay[2],
                     elem_stride=lay[3])
         need = lib().linrec_workspace_bytes_dtype(DTYPES[t.dtype], *lay, 0, int(is_bwd), None)
         entry = (call, ctypes.byref(call), int(need))
+    elif lay is not None:
+        p = Plan()  # (planned for 16-byte aligned bases, which a repeat has)
+        check(lib().linrec_plan_batched(DTYPES[t.dtype], None, *lay, int(bool(reverse)), int(is_bwd), None, ctypes.byref(p)),
+              "linrec_plan_batched")
+        entry = (None, (*lay, int(bool(reverse))), int(p.workspace_bytes))
     if len(table) >= _REPEAT_MAX:
         table.clear()
     table[key] = entry
@@ -574,12 +581,27 @@ def _repeat_launch(entry, fn, t, what):
         check(rc, what)
 
 
-def _plain_rows(t, lay, *same):
-    """The layout if a call on `t` (and tensors `same`, which must lie in memory like it) can be repeated
-    from remembered arguments, else None."""
-    if lay is None or not t.is_cuda or t.dtype not in DTYPES or not t.numel() or _few_rows_on_strided_axis(t, lay, None):
+def _repeat_batched(entry, fn, t, pointers, what):
+    """A remembered call on a batch of matrices: `fn` is linrec_fwd_batched or linrec_bwd_batched."""
+    _, layout, need = entry
+
+    def go(stream):
+        ws = workspace(t.device, stream, need) if need else None
+        return fn(DTYPES[t.dtype], *pointers, *layout, ws.data_ptr() if need else None, ws.numel() if need else 0, None, stream)
+    rc = _on_device(t, go)
+    if rc:
+        check(rc, what)
+
+
+def _repeatable(t, *same):
+    """The layout (rows, or a batch of matrices) if a call on `t` (and tensors `same`, which must lie in memory like
+    it) can be repeated from remembered arguments, else None."""
+    if not t.is_cuda or t.dtype not in DTYPES or not t.numel() or not _same_layout(t, *same):
         return None
-    return lay if _same_layout(t, *same) else None
+    lay = row_layout(t)
+    if lay is None:
+        return batched_layout(t)
+    return None if _few_rows_on_strided_axis(t, lay, None) else lay
 
 
 def fwd(inputs, coeffs, reverse=False, tuning=None, out=None):
@@ -592,7 +614,7 @@ def fwd(inputs, coeffs, reverse=False, tuning=None, out=None):
         entry = table.get(key, False)
         if entry is False:
             _validate(inputs, coeffs, names=("inputs", "coeffs"))
-            entry = _remember(table, key, _plain_rows(inputs, row_layout(inputs), coeffs), inputs, False, reverse)
+            entry = _remember(table, key, _repeatable(inputs, coeffs), inputs, False, reverse)
         if entry is not None:
             px, pc = inputs.data_ptr(), coeffs.data_ptr()
             if not (px | pc) & 15:
@@ -605,6 +627,9 @@ def fwd(inputs, coeffs, reverse=False, tuning=None, out=None):
                 po = res.data_ptr()
                 if not po & 15:
                     call = entry[0]
+                    if call is None:
+                        _repeat_batched(entry, lib().linrec_fwd_batched, inputs, (px, pc, po), "linrec_fwd_batched")
+                        return res
                     call.in0, call.coef, call.out0 = px, pc, po
                     _repeat_launch(entry, lib().linrec_fwd_call, inputs, "linrec_fwd")
                     return res
@@ -622,7 +647,7 @@ def bwd(d_outputs, coeffs, outputs, reverse=False, tuning=None, out=None):
         entry = table.get(key, False)
         if entry is False:
             _validate(outputs, coeffs, d_outputs, names=("outputs", "coeffs", "d_outputs"))
-            entry = _remember(table, key, _plain_rows(outputs, row_layout(outputs), coeffs, d_outputs), outputs, True, reverse)
+            entry = _remember(table, key, _repeatable(outputs, coeffs, d_outputs), outputs, True, reverse)
         if entry is not None:
             pd, pc, py = d_outputs.data_ptr(), coeffs.data_ptr(), outputs.data_ptr()
             if not (pd | pc | py) & 15:
@@ -637,6 +662,9 @@ def bwd(d_outputs, coeffs, outputs, reverse=False, tuning=None, out=None):
                 p0, p1 = dx.data_ptr(), dc.data_ptr()
                 if not (p0 | p1) & 15:
                     call = entry[0]
+                    if call is None:
+                        _repeat_batched(entry, lib().linrec_bwd_batched, outputs, (pd, pc, py, p0, p1), "linrec_bwd_batched")
+                        return dx, dc
                     call.in0, call.coef, call.aux, call.out0, call.out1 = pd, pc, py, p0, p1
                     _repeat_launch(entry, lib().linrec_bwd_call, outputs, "linrec_bwd")
                     return dx, dc

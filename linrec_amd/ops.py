@@ -68,18 +68,33 @@ class _LinrecFn(torch.autograd.Function):
     times the kernels' own launch time on small inputs; traced and compiled calls use the operator."""
 
     @staticmethod
-    def forward(ctx, inputs, coeffs, reverse):
-        outputs = _native.fwd(inputs, coeffs, reverse)
+    def forward(ctx, inputs, coeffs, reverse, dim):
+        if dim is None:
+            outputs = _native.fwd(inputs, coeffs, reverse)
+        else:
+            # The scan axis is moved here, out of autograd's sight: three views recorded by autograd, and their three
+            # counterparts in the backward, took 40 us of host time a step, as long as the kernels of 2^23 elements.
+            moved = _native.fwd(inputs.transpose(dim, -1), coeffs.transpose(dim, -1), reverse)
+            view = moved.transpose(dim, -1)
+            # (the result itself, not a view of a tensor autograd has not seen)
+            outputs = torch.empty(0, dtype=moved.dtype, device=moved.device).set_(
+                moved.untyped_storage(), view.storage_offset(), view.size(), view.stride())
         ctx.save_for_backward(coeffs, outputs)
-        ctx.reverse = reverse
+        ctx.reverse, ctx.dim = reverse, dim
         return outputs
 
     @staticmethod
     @torch.autograd.function.once_differentiable
     def backward(ctx, d_outputs):
         coeffs, outputs = ctx.saved_tensors
-        d_inputs, d_coeffs = _native.bwd(d_outputs, coeffs, outputs, ctx.reverse)
-        return d_inputs, d_coeffs, None
+        dim = ctx.dim
+        if dim is None:
+            d_inputs, d_coeffs = _native.bwd(d_outputs, coeffs, outputs, ctx.reverse)
+        else:
+            d_inputs, d_coeffs = _native.bwd(d_outputs.transpose(dim, -1), coeffs.transpose(dim, -1),
+                                             outputs.transpose(dim, -1), ctx.reverse)
+            d_inputs, d_coeffs = d_inputs.transpose(dim, -1), d_coeffs.transpose(dim, -1)
+        return d_inputs, d_coeffs, None, None
 
 
 def linrec(inputs: torch.Tensor, coeffs: torch.Tensor, reverse: bool = False, *, logc: bool = False,
@@ -98,12 +113,13 @@ def linrec(inputs: torch.Tensor, coeffs: torch.Tensor, reverse: bool = False, *,
     """
     if logc:
         coeffs = torch.exp(coeffs)
-    if dim != -1 and dim != inputs.dim() - 1:
-        return linrec(inputs.transpose(dim, -1), coeffs.transpose(dim, -1), reverse).transpose(dim, -1)
+    last = dim == -1 or dim == inputs.dim() - 1
     plain = (torch.Tensor, torch.nn.Parameter)  # tensor subclasses (fake, functional, ...) take the operator
     if torch.compiler.is_compiling() or type(inputs) not in plain or type(coeffs) not in plain:
-        return linrec_fwd(inputs, coeffs, reverse)
-    return _LinrecFn.apply(inputs, coeffs, reverse)
+        if last:
+            return linrec_fwd(inputs, coeffs, reverse)
+        return linrec_fwd(inputs.transpose(dim, -1), coeffs.transpose(dim, -1), reverse).transpose(dim, -1)
+    return _LinrecFn.apply(inputs, coeffs, reverse, None if last else dim)
 
 
 # The reference exports three variants of the same function (ops.py:60,81,101); here one set of
