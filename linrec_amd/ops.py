@@ -69,7 +69,7 @@ class _LinrecFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, inputs, coeffs, reverse, dim):
-        if dim is None:
+        if dim == -1:
             outputs = _native.fwd(inputs, coeffs, reverse)
         else:
             # The scan axis is moved here, out of autograd's sight: three views recorded by autograd, and their three
@@ -88,7 +88,7 @@ class _LinrecFn(torch.autograd.Function):
     def backward(ctx, d_outputs):
         coeffs, outputs = ctx.saved_tensors
         dim = ctx.dim
-        if dim is None:
+        if dim == -1:
             d_inputs, d_coeffs = _native.bwd(d_outputs, coeffs, outputs, ctx.reverse)
         else:
             d_inputs, d_coeffs = _native.bwd(d_outputs.transpose(dim, -1), coeffs.transpose(dim, -1),
@@ -120,9 +120,9 @@ def linrec(inputs: torch.Tensor, coeffs: torch.Tensor, reverse: bool = False, *,
             return linrec_fwd(inputs, coeffs, reverse)
         return linrec_fwd(inputs.transpose(dim, -1), coeffs.transpose(dim, -1), reverse).transpose(dim, -1)
     if last or (torch.is_grad_enabled() and (inputs.requires_grad or coeffs.requires_grad)):
-        return _LinrecFn.apply(inputs, coeffs, reverse, None if last else dim)
+        return _LinrecFn.apply(inputs, coeffs, reverse, -1 if last else dim)
     # (nothing to record: the views are cheaper here, bf16 1 x 4096 x 2048 forward 14.4 us against 16.2 inside)
-    return _LinrecFn.apply(inputs.transpose(dim, -1), coeffs.transpose(dim, -1), reverse, None).transpose(dim, -1)
+    return _LinrecFn.apply(inputs.transpose(dim, -1), coeffs.transpose(dim, -1), reverse, -1).transpose(dim, -1)
 
 
 # The reference exports three variants of the same function (ops.py:60,81,101); here one set of

@@ -30,6 +30,15 @@ def test_same_as_moving_the_axis_outside(dim, reverse):
     assert torch.autograd.gradcheck(lambda a, b: linrec_amd.linrec(a, b, reverse, dim=dim), (x, c))
 
 
+@pytest.mark.parametrize("requires_grad", [False, True])
+def test_what_is_no_axis_is_refused(requires_grad):
+    """A scan axis that is none raises the same error whether or not a gradient is recorded."""
+    x, c = (torch.rand(3, 6, 4, requires_grad=requires_grad) for _ in range(2))
+    for dim, error in ((None, TypeError), (1.5, TypeError), ("1", (TypeError, RuntimeError)), (3, IndexError), (-4, IndexError)):
+        with pytest.raises(error):
+            linrec_amd.linrec(x, c, dim=dim)
+
+
 def test_saved_tensor_hooks_and_in_place_changes():
     x, c, dy = _case("cpu")
     packed = []
