@@ -232,6 +232,7 @@ def output_like(t, fake=False):
 _workspaces = collections.OrderedDict()  # (device index, stream handle) -> buffer, least recently used first
 _ws_pinned = set()           # keys whose workspace a graph capture has been given: never dropped
 _ws_retired = []             # buffers a captured graph may still write to, outgrown since
+_ws_cleared_in = {}          # keys whose workspace was allocated under capture -> the capture that cleared it last
 _ws_gave_up_of_dropped = {}  # device index -> waits that ran out, counted in workspaces since dropped
 _ws_lock = threading.Lock()
 _WS_MIN_BYTES = 1 << 20
@@ -243,23 +244,41 @@ def _capturing():
     return torch.cuda.is_available() and torch.cuda.is_current_stream_capturing()
 
 
+def _capture_id(stream_ptr):
+    """A number that tells the capture `stream_ptr` is in from all others of the process (streams forked into it
+    share it), None if the runtime names none.  torch has no such call; the HIP runtime the library is linked to has."""
+    status, number = ctypes.c_int(), ctypes.c_ulonglong()
+    rc = lib().hipStreamGetCaptureInfo(ctypes.c_void_p(stream_ptr), ctypes.byref(status), ctypes.byref(number))
+    return number.value if rc == 0 and status.value == 1 else None  # 1: hipStreamCaptureStatusActive
+
+
 def workspace(device, stream_ptr, nbytes):
     """Zero-initialised scratch owned by the kernels' look-back chain.  Kept per stream because two
     launches that overlap in time must not share descriptors; grown (and re-zeroed) on demand.
     A workspace handed out while its stream is being captured into a graph stays for good: the graph has
     its address baked in and every replay writes descriptors there, so such a buffer is neither dropped with
-    the least recently used ones nor freed when a later launch on the stream needs a larger one."""
+    the least recently used ones nor freed when a later launch on the stream needs a larger one.
+    The clearing of a buffer that is allocated under capture is itself a node of that graph, which runs when (and if)
+    the graph is replayed.  Such a buffer only serves captures, each of which records a clearing of its own before its
+    first use; the next eager launch on the stream gets a buffer that is cleared there and then."""
     key = (device.index, stream_ptr)
     with _ws_lock:
         capturing = _capturing()
         ws = _workspaces.get(key)
-        if ws is None or ws.numel() < nbytes:
+        of_captures = key in _ws_cleared_in
+        if ws is None or ws.numel() < nbytes or (of_captures and not capturing):
             size = max(_WS_MIN_BYTES, 1 << (int(nbytes) - 1).bit_length())
+            if of_captures:
+                size = max(size, ws.numel())  # (large enough for the next capture as well: no more buffers than sizes)
             if ws is not None and key in _ws_pinned:
                 _ws_retired.append(ws)
                 _ws_pinned.discard(key)
             ws = torch.zeros(size, dtype=torch.uint8, device=device)
             _workspaces[key] = ws
+            if capturing:
+                _ws_cleared_in[key] = _capture_id(stream_ptr)
+            else:
+                _ws_cleared_in.pop(key, None)
             # Streams come and go (their handles are even reused); the workspaces of the ones not
             # launched from for longest are dropped.  A dropped buffer goes back to torch's allocator,
             # which hands it out again in the order of the stream it was allocated on: the one its
@@ -272,6 +291,11 @@ def workspace(device, stream_ptr, nbytes):
                     # (what it counted is kept; reading it synchronises, which is allowed outside a capture)
                     if gone.is_cuda:
                         _ws_gave_up_of_dropped[old[0]] = _ws_gave_up_of_dropped.get(old[0], 0) + int(gone[:16].view(torch.int32)[1].item())
+        elif of_captures:
+            capture = _capture_id(stream_ptr)
+            if capture is None or _ws_cleared_in[key] != capture:
+                ws.zero_()
+                _ws_cleared_in[key] = capture
         if capturing:
             _ws_pinned.add(key)
         _workspaces.move_to_end(key)
@@ -498,7 +522,10 @@ def gave_up_count(device=None):
         total = sum(n for idx, n in _ws_gave_up_of_dropped.items() if want in (None, idx))
     for key, ws in items:
         if want in (None, key[0]):
-            total += int(ws[:16].view(torch.int32)[1].item())
+            header = ws[:16].view(torch.int32).tolist()
+            # (a buffer of captures holds anything until the first replay; its two reserved words are zero from then on)
+            if not (key in _ws_cleared_in and (header[2] or header[3])):
+                total += header[1]
     return total
 
 

@@ -173,3 +173,47 @@ def test_graph_replays_match_the_oracle(nat):
         check_close(dc, dc_t, f"replay {rep} d_coeffs")
         nat.fwd(dy, c)  # the program's own eager work between the replays
     assert nat.gave_up_count() == 0
+
+
+def test_graphs_captured_on_a_cold_stream_clear_their_own_workspace(nat, monkeypatch):
+    """Two graphs captured on a stream that has not launched before: the second one is replayed first, on a workspace
+    that holds what an earlier graph of a shared memory pool may have left there, and an eager launch comes between."""
+    for name in ("_workspaces", "_ws_pinned", "_ws_retired", "_ws_cleared_in"):
+        monkeypatch.setattr(nat, name, type(getattr(nat, name))())
+    x, c, dy = (t.transpose(1, 2) for t in draw((4, 1500, 96), torch.float32, 1))
+    nat.fwd(x, c)  # (the kernels are loaded, the call is remembered)
+    nat.bwd(dy, c, x)
+    torch.cuda.synchronize()
+    side, graphs, ids = torch.cuda.Stream(), [], []
+    key = (0, side.cuda_stream)
+    for i in range(2):
+        y, dx, dc = nan_like(x), nan_like(x), nan_like(x)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            nat.fwd(x, c, out=y)
+            ids.append(nat._capture_id(side.cuda_stream))
+            nat.bwd(dy, c, y, out=(dx, dc))
+        graphs.append((graph, y, dx, dc, nat._workspaces[key]))
+    assert None not in ids and ids[0] != ids[1], ids
+    nat._workspaces[key].fill_(0x5a)
+    assert nat.gave_up_count() == 0  # (nothing has been launched: what the buffer holds is no count)
+    for rep, which in enumerate((1, 1, 0, 1, 0)):
+        graph, y, dx, dc, ws = graphs[which]
+        for dst, src in zip((x, c, dy), draw((4, 1500, 96), torch.float32, 30 + rep)):
+            dst.copy_(src.transpose(1, 2))
+        for t in (y, dx, dc):
+            t.fill_(float("nan"))
+        ws.fill_(0x5a)
+        print("replay", rep, "of graph", which, flush=True)
+        graph.replay()
+        torch.cuda.synchronize()
+        check_close(y, oracle.fwd(f64(x), f64(c), False, dtype=np.float64), f"replay {rep} outputs")
+        dx_t, dc_t = oracle.bwd(f64(dy), f64(c), f64(y), False, dtype=np.float64)
+        check_close(dx, dx_t, f"replay {rep} d_inputs")
+        check_close(dc, dc_t, f"replay {rep} d_coeffs")
+        if rep:
+            with torch.cuda.stream(side):
+                eager = nat.fwd(x, c)
+            torch.cuda.synchronize()
+            assert torch.equal(eager, y) and all(nat._workspaces[key] is not g[4] for g in graphs)

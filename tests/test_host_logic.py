@@ -990,3 +990,66 @@ def test_caches_of_the_binding_stay_bounded(monkeypatch):
         t = torch.empty(600, L)
         nat._workspace_for(t, 0, nat.row_layout(t), False, None, 0)
     assert len(nat._need_cache) == 8
+
+
+def test_workspaces_under_graph_capture_are_cleared_by_the_graph_that_uses_them(monkeypatch):
+    """A buffer first allocated while a stream is captured is only cleared when that graph is replayed.  So another
+    graph captured on the stream records a clearing of its own (once), an eager launch gets a buffer that is cleared
+    for it, and a capture on a stream with such a buffer needs none."""
+    clearings, state = [], {"capture": None}
+
+    class Buffer:
+        def __init__(self, size):
+            self.size, self.is_cuda = size, False
+            clearings.append((self, state["capture"]))
+
+        def numel(self):
+            return self.size
+
+        def zero_(self):
+            clearings.append((self, state["capture"]))
+
+    monkeypatch.setattr(nat.torch, "zeros", lambda size, dtype, device: Buffer(size))
+    monkeypatch.setattr(nat, "_workspaces", type(nat._workspaces)())
+    for name, empty in (("_ws_pinned", set()), ("_ws_retired", []), ("_ws_cleared_in", {})):
+        monkeypatch.setattr(nat, name, empty)
+    monkeypatch.setattr(nat, "_capturing", lambda: state["capture"] is not None)
+    monkeypatch.setattr(nat, "_capture_id", lambda stream: state["capture"])
+    dev, stream = torch.device("cuda", 0), 7
+
+    def cleared_for(ws, capture):
+        return [c for b, c in clearings if b is ws].count(capture)
+
+    state["capture"] = 1
+    first = nat.workspace(dev, stream, 100)
+    assert nat.workspace(dev, stream, 200) is first and cleared_for(first, 1) == 1
+    state["capture"] = 2
+    second = nat.workspace(dev, stream, 100)
+    assert nat.workspace(dev, stream, 100) is second and cleared_for(second, 2) == 1  # the same buffer or not
+    state["capture"] = None
+    eager = nat.workspace(dev, stream, 100)
+    assert eager is not first and eager is not second and cleared_for(eager, None) == 1
+    assert nat.workspace(dev, stream, 100) is eager
+    assert any(b is first for b in nat._ws_retired)  # the graphs still write there
+    state["capture"] = 3
+    assert nat.workspace(dev, stream, 100) is eager and cleared_for(eager, 3) == 0  # cleared long before
+    larger = nat.workspace(dev, stream, eager.numel() + 1)
+    assert larger is not eager and cleared_for(larger, 3) == 1
+    state["capture"] = None
+    again = nat.workspace(dev, stream, 100)
+    assert again is not larger and cleared_for(again, None) == 1
+    # alternating sizes do not allocate for ever: what serves eager launches is as large as what it takes the place of
+    made = len(clearings)
+    for capture in (4, None, 5, None):
+        state["capture"] = capture
+        assert nat.workspace(dev, stream, larger.numel() if capture else 100) is again
+    assert len(clearings) == made
+    # a capture the runtime tells nothing about: cleared for every launch
+    monkeypatch.setattr(nat, "_capture_id", lambda stream: None)
+    state["capture"] = 6
+    unknown = nat.workspace(dev, 8, 100)
+    assert nat.workspace(dev, 8, 100) is unknown and cleared_for(unknown, 6) == 2
+
+
+def test_capture_id_outside_a_capture():
+    assert nat._capture_id(0) is None
