@@ -673,6 +673,23 @@ int lookback_segments_plan(const Problem& q, int vec, int waves, int depth, int 
 bool lookback_segments_choose(const Problem& q, int family, bool colblock, int mode, int desc, linrec_plan_t* out) {
   const bool half = q.dtype != LINREC_DTYPE_F32;
   if (q.row_stride != 1 || q.seqlen < kSegmentMinLen) return false;
+  if (q.batched()) {
+    // Batches of two or three channels: the lanes' accesses share no lines to speak of, and the three launches, which
+    // number their lanes segment by segment, bring more of them (forward / backward: fp32 100 x 2000 x 2 21.3 / 37.9
+    // against 16.7 / 22.7, 500 x 300 x 3 20.9 / 29.5 against 13.9 / 21.5, bf16 32 x 4096 x 2 22.6 / 30.0 against 16.0 /
+    // 18.8, 32 x 65536 x 2 backward 229 against 187); not up to 24 rows (fp32 12 x 51982 x 2 31.7 / 51.8 against 39.7 /
+    // 73.2) nor on the longest axes (fp32 64 x 262144 x 2 1285 / 2197 against 2049 / 3436).  The same on short axes up
+    // to seven channels in fp32, or an odd number of them (fp32 30 x 1000 x 6 14.1 / 19.8 against 12.2 / 15.0, 188 x 2587 x
+    // 6 35.4 / 68.6 against 31.5 / 60.8, bf16 186 x 310 x 5 15.5 / 20.7 against 13.1 / 18.0; but fp32 62 x 5831 x 5 24.2 /
+    // 46.6 against 26.8 / 50.7, bf16 64 x 300 x 6 11.4 / 15.6 against 13.4 / 16.2).
+    const int64_t few = q.rows_per_batch < 4 ? 131072 : q.rows_per_batch < 8 && (!half || q.rows_per_batch % 2) ? 4096 : 0;
+    if (q.numseq > q.at(24) && q.seqlen < few) return false;
+    // Fewer rows than a wave has lanes, in few batches, over the longest axes: thousands of segments that look back,
+    // mostly of lanes without a row (2 x 2^20 x 16 fp32 172 / 236 with one row to a lane against 149 / 231, bf16 160 / 215
+    // against 128 / 232; 4 x 2^20 x 8 fp32 forward 219 against 206; 2 x 2^18 x 2 fp32 46.3 / 63.4 against 43.8 / 58.3; but
+    // 2 x 2^18 x 16 51.2 / 68.5 against 56.0 / 80.5, 8 x 2^20 x 2 362 / 687 against 734 / 1523).
+    if (q.numseq < 64 && q.numseq < 8 * q.rows_per_batch && q.seqlen > (q.numseq <= 8 ? 131072 : 524288)) return false;
+  }
   if (!q.batched()) {
     if (!half || family != LINREC_FAMILY_SEGMENT || q.seqlen > 8192) return false;
   } else {
@@ -686,7 +703,12 @@ bool lookback_segments_choose(const Problem& q, int family, bool colblock, int m
   // The widest access that makes a workgroup for 5 of 8 CUs: it needs the fewest descriptors and the memory system
   // likes it best (bf16 8 x 4096 x 1024 forward: 43.2 us with four rows to a lane, 47.6 with two, 51.7 with one), but
   // half a chip is worse than a narrower access (bf16 1 x 4096 x 2048: 128 workgroups of four rows to a lane 17.4 us,
-  // 256 of two 13.7; fp32 2 x 4096 x 256 backward: 128 of two 14.4, 256 of one 12.9).
+  // 256 of two 13.7; fp32 2 x 4096 x 256 backward: 128 of two 14.4, 256 of one 12.9).  More than one row to a lane needs
+  // rows for three quarters of the lanes, or a workgroup's accesses and descriptors are mostly padding (fp32 2 x 262144 x
+  // 32: 78 / 131 with two rows to a lane in the forward and four in the backward, 57 / 78 with one, 78 / 102 in three
+  // launches; bf16 2 x 262144 x 16 72 / 93, 48 / 58 and 50 / 76), and lanes that lie next to each other: batches of at
+  // least 32 channels (fp32 500 x 2000 x 8 47.5 / 114.9, 41.7 / 87.4 and 53.5 / 101.6; bf16 8 x 262144 x 16 127 / 206,
+  // 106 / 161 and 147 / 264).
   // {rows per lane, waves, positions per run}: the run as long as its tensors fit the registers
   static const int shapes[2][2][3][3] = {{{{2, 16, 16}, {1, 8, 16}, {0, 0, 0}}, {{4, 16, 8}, {2, 16, 8}, {1, 8, 16}}},
                                          {{{4, 16, 16}, {2, 16, 16}, {1, 8, 16}}, {{4, 16, 16}, {2, 16, 16}, {1, 8, 16}}}};
@@ -694,7 +716,8 @@ bool lookback_segments_choose(const Problem& q, int family, bool colblock, int m
     linrec_plan_t p;
     std::memset(&p, 0, sizeof(p));
     if (s[0] == 0 || lookback_segments_plan(q, s[0], s[1], s[2], mode, desc, &p) != LINREC_OK) continue;
-    if (s[0] > 1 && p.grid * 8 < 5 * q.cus) continue;
+    const int64_t lanes = ceil_div(q.numseq, int64_t(64) * s[0]) * 64;  // of a segment, with and without a row
+    if (s[0] > 1 && (p.grid * 8 < 5 * q.cus || q.numseq * 4 < lanes * s[0] * 3 || (q.batched() && q.rows_per_batch < 32))) continue;
     // (a caller that can only give so much workspace is served by the kernels that need less)
     if (q.workspace_cap && p.workspace_bytes > q.workspace_cap) return false;
     *out = p;

@@ -1,0 +1,68 @@
+"""What the planner decides about segments of a strided scan axis chained by look-back, for 256 compute units.  No GPU."""
+import ctypes
+
+import pytest
+import torch
+
+from linrec_amd import _native as nat
+
+S = nat.FAMILY_SEGMENT
+
+
+@pytest.fixture(autouse=True)
+def full_part():
+    old = nat.set_compute_units(256)
+    yield
+    nat.set_compute_units(old)
+
+
+def plan(dtype, batch, time, channels, is_bwd=False, reverse=False, row_stride=1, batch_stride=None, elem_stride=None, tuning=None):
+    """The plan of a dense (batch, time, channels) tensor with the bases on 16 bytes, or of other strides; None if refused."""
+    es = elem_stride or channels * row_stride
+    p = nat.Plan()
+    args = (channels, time, row_stride, es)
+    tun = ctypes.byref(tuning) if tuning is not None else None
+    if batch > 1:
+        rc = nat.lib().linrec_plan_batched(nat.DTYPES[dtype], None, batch, channels, time, batch_stride or time * es, row_stride, es,
+                                           int(reverse), int(is_bwd), tun, ctypes.byref(p))
+    else:
+        rc = nat.lib().linrec_plan(nat.DTYPES[dtype], None, *args, int(reverse), int(is_bwd), tun, ctypes.byref(p))
+    if rc == -3:
+        return None
+    assert rc == 0, rc
+    return p.asdict()
+
+
+def chained(p):
+    return p["family"] == S and p["carry"] == 1
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+def test_a_lane_takes_several_rows_only_where_all_lanes_have_some_next_to_each_other(dtype):
+    size = torch.empty(0, dtype=dtype).element_size()
+    for batch, time, channels in [(2, 262144, 32), (4, 262144, 16), (2, 65536, 16), (3, 100000, 4), (8, 262144, 16), (2, 262144, 48),
+                                  (2, 262144, 64), (2, 262144, 128), (500, 16384, 8), (500, 2000, 8), (7, 67656, 48), (16, 8192, 512)]:
+        for is_bwd in (False, True):
+            p = plan(dtype, batch, time, channels, is_bwd)
+            assert chained(p), (batch, time, channels, p)
+            rows = batch * channels
+            assert p["vec"] == 1 or (rows >= 0.75 * -(-rows // (64 * p["vec"])) * 64 * p["vec"] and channels >= 32), (rows, time, p)
+            # workgroups of 64 lanes' rows, and a workspace that does not outgrow the tensors
+            assert p["grid"] == -(-batch * channels // (64 * p["vec"])) * p["tiles_per_row"]
+            assert p["workspace_bytes"] <= max(1 << 16, batch * time * channels * size), (batch, time, channels, p)
+    assert plan(dtype, 16, 8192, 512)["vec"] > 1 and plan(dtype, 2, 262144, 64)["vec"] == 2
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+def test_few_channels_and_few_very_long_rows_stay_with_the_three_launches(dtype):
+    half = dtype != torch.float32
+    for is_bwd in (False, True):
+        for batch, time, channels, want in [(32, 4096, 2, False), (500, 300, 3, False), (13, 131071, 2, False), (13, 131072, 2, True),
+                                            (12, 65535, 2, True), (32, 4096, 4, True), (8, 65535, 3, True), (9, 65535, 3, False),
+                                            (7, 4095, 4, half), (6, 4095, 4, True), (7, 4096, 4, True), (60, 4095, 7, False), (60, 4095, 6, half),
+                                            (60, 300, 8, True),
+                                            (2, 524289, 16, False), (2, 524288, 16, True), (2, 524289, 31, False), (2, 524289, 32, True),
+                                            (7, 524289, 8, False), (8, 524289, 2, True), (2, 131072, 4, True), (2, 131073, 4, False),
+                                            (2, 131073, 5, True)]:
+            p = plan(dtype, batch, time, channels, is_bwd)
+            assert chained(p) == want and p["family"] == S, (batch, time, channels, is_bwd, p)
