@@ -670,7 +670,7 @@ int lookback_segments_plan(const Problem& q, int vec, int waves, int depth, int 
 //     3 x 2100 x 2688 would gain, 25.4 against 31.5).
 // One matrix (not a batch of them): 16-bit storage where the three launches were chosen, up to 8192 positions; the
 // rest stays with the teams and the three launches.
-bool lookback_segments_choose(const Problem& q, int family, bool colblock, int mode, int desc, linrec_plan_t* out) {
+bool lookback_segments_choose(const Problem& q, int family, int colblock, int mode, int desc, linrec_plan_t* out) {
   const bool half = q.dtype != LINREC_DTYPE_F32;
   if (q.row_stride != 1 || q.seqlen < kSegmentMinLen) return false;
   if (q.batched()) {
@@ -695,6 +695,10 @@ bool lookback_segments_choose(const Problem& q, int family, bool colblock, int m
   } else {
     if (!q.is_bwd && colblock && q.seqlen < 1024) return false;
     if (!q.is_bwd && family == LINREC_FAMILY_COLDRIFT && q.seqlen < 4096) return false;
+    // The column blocks of two lane groups keep the shortest axes in the backward as well (fp32 8 x 256 x 1024 12.0 against
+    // 10.3, 8 x 352 x 832 15.4 against 13.0, 4000 x 300 x 4 160 against 131; bf16 8 x 300 x 1536 16.1 against 14.3, 2000 x
+    // 300 x 8 66.7 against 49.3; but fp32 8 x 448 x 768 13.5 against 16.3, bf16 8 x 512 x 1536 20.1 against 21.5).
+    if (q.is_bwd && colblock && q.seqlen < (half ? 384 : 448) && (colblock == 2 || q.rows_per_batch < 32)) return false;
     const bool pairs = colblock_rows_per_lane(q, 2) == 2;
     const bool on_lines = q.elem_stride * elem_size_of(q.dtype) % 128 == 0;
     const int64_t most = !pairs ? (half ? 32767 : 16384) : on_lines ? (half ? 16384 : 8192) : 65536;
@@ -718,6 +722,22 @@ bool lookback_segments_choose(const Problem& q, int family, bool colblock, int m
     if (s[0] == 0 || lookback_segments_plan(q, s[0], s[1], s[2], mode, desc, &p) != LINREC_OK) continue;
     const int64_t lanes = ceil_div(q.numseq, int64_t(64) * s[0]) * 64;  // of a segment, with and without a row
     if (s[0] > 1 && (p.grid * 8 < 5 * q.cus || q.numseq * 4 < lanes * s[0] * 3 || (q.batched() && q.rows_per_batch < 32))) continue;
+    // A few workgroups more than there are CUs, which hold one of sixteen waves each: the rest of them runs on a chip that
+    // is mostly idle.  Column blocks of two lane groups that fill most of it in one round are left in place there: fp32
+    // forwards from 11/16 of the CUs up to 7/4 workgroups per CU (6656 rows, 8 x 1200 x 832 28.1 against 22.5; 7680 x 1700
+    // 34.8 against 32.2; 8192 x 1200 30.0 against 27.4; but 8192 x 1700 35.7 against 37.3, 5120 x 1800 30.8 against 31.7),
+    // fp32 backwards of two rows to a lane alike (6656 x 640 25.7 against 19.9), of four up to 3/2 workgroups per CU where
+    // positions are not whole KiB apart (16 x 1200 x 416 36.0 against 32.1, 8 x 1400 x 960 47.8 against 44.5; but 2 x 1200 x
+    // 3328 35.7 against 39.5, 8 x 1536 x 768 44.7 against 51.0: there the blocks, which read position after position, do
+    // worse), 16-bit storage from 7/8 of the CUs up to 11/8 (14336 x 1280 30.8 / 48.2 against 26.8 / 43.3; but 12288 x 1400
+    // 28.1 / 41.8 against 33.4 / 46.6).
+    if (q.batched() && colblock == 2 && p.waves == 16 && p.grid > q.cus) {
+      const int64_t blocks = ceil_div(q.numseq / colblock_rows_per_lane(q, 0), 32);
+      if (half ? blocks * 8 >= 7 * q.cus && p.grid * 8 < 11 * q.cus
+               : blocks * 16 >= 11 * q.cus &&
+                     (s[0] <= 2 ? p.grid * 4 < 7 * q.cus : q.elem_stride * 4 % 1024 != 0 && p.grid * 2 < 3 * q.cus))
+        return false;
+    }
     // (a caller that can only give so much workspace is served by the kernels that need less)
     if (q.workspace_cap && p.workspace_bytes > q.workspace_cap) return false;
     *out = p;
@@ -835,7 +855,7 @@ int make_plan(const Problem& q, const linrec_tuning_t* tune, linrec_plan_t* out)
         family = LINREC_FAMILY_COLDRIFT;
         use_colblock = 0;
       }
-      if (lookback_segments_choose(q, family, use_colblock != 0, mode, desc, out)) return LINREC_OK;
+      if (lookback_segments_choose(q, family, use_colblock, mode, desc, out)) return LINREC_OK;
     } else {
       family = LINREC_FAMILY_NAIVE;
     }

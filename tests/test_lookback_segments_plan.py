@@ -66,3 +66,17 @@ def test_few_channels_and_few_very_long_rows_stay_with_the_three_launches(dtype)
                                             (2, 131073, 5, True)]:
             p = plan(dtype, batch, time, channels, is_bwd)
             assert chained(p) == want and p["family"] == S, (batch, time, channels, is_bwd, p)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+def test_column_blocks_keep_short_backwards_and_launches_a_little_beyond_one_round(dtype):
+    half = dtype != torch.float32
+    f32 = [(256, 1024, True, False), (447, 768, True, False), (448, 768, True, True), (1023, 1024, False, False), (1024, 1024, False, True),
+           (1200, 832, False, False), (1700, 960, False, False), (1200, 640, False, True), (1800, 1024, False, True), (640, 832, True, False),
+           (1200, 832, True, False), (1400, 960, True, False), (1900, 832, True, True), (1536, 768, True, True)]
+    f16 = [(256, 1280, True, False), (383, 2048, True, False), (384, 1536, True, True), (1280, 1792, False, False), (1280, 1792, True, False),
+           (1280, 2048, True, False), (1400, 1536, True, True), (1400, 2048, False, True)]
+    for time, channels, is_bwd, want in f16 if half else f32:
+        p = plan(dtype, 8, time, channels, is_bwd)
+        assert chained(p) == want, (time, channels, is_bwd, p)
+        assert want or (p["family"], p["carry"]) == (nat.FAMILY_COLUMN, 2), (time, channels, is_bwd, p)
