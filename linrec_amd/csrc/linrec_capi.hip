@@ -699,7 +699,8 @@ bool lookback_segments_choose(const Problem& q, int family, int colblock, int mo
     // 10.3, 8 x 352 x 832 15.4 against 13.0, 4000 x 300 x 4 160 against 131; bf16 8 x 300 x 1536 16.1 against 14.3, 2000 x
     // 300 x 8 66.7 against 49.3; but fp32 8 x 448 x 768 13.5 against 16.3, bf16 8 x 512 x 1536 20.1 against 21.5).
     if (q.is_bwd && colblock && q.seqlen < (half ? 384 : 448) && (colblock == 2 || q.rows_per_batch < 32)) return false;
-    const bool pairs = colblock_rows_per_lane(q, 2) == 2;
+    // (fp32 1862 x 632 x 20 with one row to a lane 105 / 220 against 101 / 181 for the plain column kernels)
+    const bool pairs = q.rows_per_batch >= 32 && colblock_rows_per_lane(q, 2) == 2;
     const bool on_lines = q.elem_stride * elem_size_of(q.dtype) % 128 == 0;
     const int64_t most = !pairs ? (half ? 32767 : 16384) : on_lines ? (half ? 16384 : 8192) : 65536;
     if (q.numseq > q.at(most)) return false;

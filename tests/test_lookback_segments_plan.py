@@ -54,6 +54,17 @@ def test_a_lane_takes_several_rows_only_where_all_lanes_have_some_next_to_each_o
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+def test_row_limits_follow_the_rows_a_lane_takes(dtype):
+    """One row to a lane up to 16384 rows (16-bit storage: 32767), more of them up to 8192 (16384) where a position's rows
+    start on a 128-byte line and up to 65536 where they do not."""
+    one, lines = (32767, 16384) if dtype != torch.float32 else (16384, 8192)
+    for channels, limit in ((31, one), (77, one), (30, one), (128, lines), (1024, lines), (100, 65536), (1000, 65536)):
+        for batch in (limit // channels, limit // channels + 1):
+            p = plan(dtype, batch, 3000, channels, True)
+            assert chained(p) == (batch * channels <= limit), (batch, channels, p)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 def test_few_channels_and_few_very_long_rows_stay_with_the_three_launches(dtype):
     half = dtype != torch.float32
     for is_bwd in (False, True):
