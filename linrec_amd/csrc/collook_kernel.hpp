@@ -21,6 +21,11 @@
 // per CU, whose loads and stores do not overlap.  16 waves and runs as long as the registers hold beat smaller
 // workgroups of which several share a CU (8 waves, the second shape: 47 / 77 us): descriptors per byte halve.
 //
+// A segment's map multiplies 128 or 256 coefficients, and the look-back composes several: the product can overflow where
+// the recurrence does not (nothing put in yet, or small values that grow and shrink again).  Where what leaves a segment
+// comes out non-finite, its row takes the value that leaves the segment before and goes through the waves' maps of U
+// positions one after the other.
+//
 // A segment only waits for segments with smaller numbers, which are started first; every wait is bounded, and a
 // lane whose wait runs out computes what enters its row from the row's own data.
 //
@@ -202,25 +207,44 @@ __global__ __launch_bounds__(64 * NW) void collook_kernel(ColDriftArgs args) {
             __builtin_amdgcn_s_sleep(1);
           }
         }
-        const uint64_t late = __ballot(!found);
-        if (late) {
-          if (lane == 0) __hip_atomic_fetch_add(&ch.ws->gave_up, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          if (!found) {
-            // what enters the segment from the row's own data: the plain sequential walk
-            const long long row = r0 + (VEC > 1 ? wave : 0);
-            const long long rb = base_of(row);
-            float val = 0.0f;
-            for (int n = 0; n < k * STEP; ++n) {
-              const int l = DESC ? L - 1 - n : n;
-              const long long off = rb + (long long)l * p.elem_stride;
-              const float x = float(in0[off]), c = float(coef[off]);
-              if constexpr (MODE == 0) val = n == 0 ? x : fmaf(val, c, x);
-              else val = (val + x) * c;
+        float leaving = fmaf(entering, ta, tb);
+        // (one test in the chain from segment to segment: what leaves cannot be finite if what enters is not)
+        const bool astray = found && !__builtin_isfinite(leaving);
+        if (__builtin_expect(__ballot(!found || astray) != 0, 0)) {
+          bool have = found && !astray, waits = astray;
+          const uint64_t* d = desc_of(k - 1) + RPB + i;
+          for (polls = 0; __ballot(waits) != 0 && polls < ch.spin_limit; ++polls) {
+            if (polls > 0) __builtin_amdgcn_s_sleep(1);
+            const uint64_t w = ld_desc(d);
+            if (waits && uint32_t(w >> 32) == done) {
+              entering = __builtin_bit_cast(float, uint32_t(w));
+              have = true;
+              waits = false;
             }
-            entering = val;
           }
+          if (__ballot(!have)) {
+            if (lane == 0) __hip_atomic_fetch_add(&ch.ws->gave_up, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (!have) {
+              // what enters the segment from the row's own data: the plain sequential walk
+              const long long row = r0 + (VEC > 1 ? wave : 0);
+              const long long rb = base_of(row);
+              float val = 0.0f;
+              for (int n = 0; n < k * STEP; ++n) {
+                const int l = DESC ? L - 1 - n : n;
+                const long long off = rb + (long long)l * p.elem_stride;
+                const float x = float(in0[off]), c = float(coef[off]);
+                if constexpr (MODE == 0) val = n == 0 ? x : fmaf(val, c, x);
+                else val = (val + x) * c;
+              }
+              entering = val;
+            }
+          }
+          float val = entering;
+#pragma unroll 1
+          for (int w = 0; w < NW; ++w) val = fmaf(val, sh_a[w][i], sh_b[w][i]);
+          if (!found || astray) leaving = val;
         }
-        if (k + 1 < ksteps) st_desc(mine + RPB, pack_desc(done, fmaf(entering, ta, tb)));
+        if (k + 1 < ksteps) st_desc(mine + RPB, pack_desc(done, leaving));
       }
       sh_in[i] = entering;
     }

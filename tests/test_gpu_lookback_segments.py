@@ -217,3 +217,50 @@ def test_graphs_captured_on_a_cold_stream_clear_their_own_workspace(nat, monkeyp
                 eager = nat.fwd(x, c)
             torch.cuda.synchronize()
             assert torch.equal(eager, y) and all(nat._workspaces[key] is not g[4] for g in graphs)
+
+
+def growing_rows(kind):
+    """Inputs and coefficients, (2, 68, 3000), whose running product overflows where the recurrence does not: nothing is
+    put in before position 1300 while the coefficients are 2 (batch 0), and values of 2^-60 grow by 2^130 and shrink
+    again (batch 1).  The first half of the rows is meant to be read forwards, the second half, its mirror image, backwards.
+    All values are positive, so that every result has a relative error of its own."""
+    g = torch.Generator().manual_seed(3)
+    x, c = 0.5 + torch.rand((2, 68, 3000), generator=g), 0.5 * torch.rand((2, 68, 3000), generator=g)
+    x[0, :, :1300] = 0
+    c[0, :, :1300] = 2.0
+    for pos in (200, 1300, 2400):
+        x[1, :, pos - 60:pos + 260] = 0
+        c[1, :, pos - 60:pos] = 0.5
+        c[1, :, pos:pos + 130] = 2.0
+        c[1, :, pos + 130:pos + 260] = 0.5
+    for t in (x, c):
+        t[:, 34:] = t[:, 34:].flip(-1)
+    return [t.to(DTYPES[kind]).transpose(1, 2).contiguous().to("cuda:0").transpose(1, 2) for t in (x, c)]
+
+
+@pytest.mark.parametrize("reverse", [False, True])
+@pytest.mark.parametrize("kind", ["f32", "bf16"])
+def test_products_of_a_segment_may_overflow_where_the_values_do_not(nat, kind, reverse):
+    """A segment publishes the product of its 128 or 256 coefficients before it knows what enters it."""
+    x, c = growing_rows(kind)
+    rows = [f64(t) for t in (x, c)]
+    saved = torch.ones_like(x)
+    fwd = [(2, 16, 16), (1, 8, 16)] if kind == "f32" else [(4, 16, 16), (2, 16, 16), (1, 8, 16)]
+    bwd = [(4, 16, 8), (2, 16, 8), (1, 8, 16)] if kind == "f32" else fwd
+    for is_bwd, geometries in ((False, fwd), (True, bwd)):
+        meant = slice(34, 68) if is_bwd != reverse else slice(0, 34)  # (the gradient's scan runs against the forward's)
+        want = oracle.bwd(rows[0], rows[1], f64(saved), reverse, dtype=np.float64)[0] if is_bwd else \
+            oracle.fwd(rows[0], rows[1], reverse, dtype=np.float64)
+        want = torch.from_numpy(want[:, meant])
+        assert want.min() >= 0 and 1e19 < want.max() < 1e30
+        for vec, waves, run in geometries:
+            tuning = nat.Tuning(nat.FAMILY_SEGMENT, vec, run, 1, waves)
+            got = nat.bwd(x, c, saved, reverse, tuning)[0] if is_bwd else nat.fwd(x, c, reverse, tuning)
+            torch.cuda.synchronize()
+            got = got[:, meant].cpu().double()
+            error = ((got - want).abs() / want.clamp_min(1e-30)).max().item()
+            what = f"{kind} reverse={reverse} {'backward' if is_bwd else 'forward'} rows/lane={vec} waves={waves} run={run}"
+            print(what, f"largest relative error {error:.2e}", flush=True)
+            # (a value holds about ten inputs, the powers of two are exact: far below the bar of the other tests)
+            assert error <= TOL[kind], what
+    assert nat.gave_up_count() == 0
