@@ -91,3 +91,38 @@ def test_column_blocks_keep_short_backwards_and_launches_a_little_beyond_one_rou
         p = plan(dtype, 8, time, channels, is_bwd)
         assert chained(p) == want, (time, channels, is_bwd, p)
         assert want or (p["family"], p["carry"]) == (nat.FAMILY_COLUMN, 2), (time, channels, is_bwd, p)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("channels", [2, 32, 48, 64, 100, 1024])
+def test_a_lane_is_less_than_2_31_bytes_from_its_wave(dtype, channels):
+    """The kernel adds 32 bits of bytes per lane to an address per wave: the largest batch stride that is accepted keeps
+    all rows of a block within them, the next one is refused and planned otherwise."""
+    size, time = torch.empty(0, dtype=dtype).element_size(), 4096
+    for vec, waves, run in ((1, 8, 16), (2, 16, 16), (4, 16, 16)):
+        tuning = nat.Tuning(S, vec, run, 1, waves)
+        if plan(dtype, 64, time, channels, tuning=tuning) is None:
+            assert (dtype == torch.float32 and vec == 4) or channels % vec  # (no such kernel; rows of a lane in two batches)
+            continue
+        low, high = time * channels // vec, 1 << 40  # in steps of the rows of a lane, which have to lie in one slot
+        while high - low > 1:
+            mid = (low + high) // 2
+            accepted = plan(dtype, 64, time, channels, batch_stride=mid * vec, tuning=tuning) is not None
+            low, high = (mid, high) if accepted else (low, mid)
+        rows, worst = 64 * vec, 0
+        offset = lambda r: (r // channels) * low * vec + r % channels
+        for block in range(64 * channels // rows + 1):
+            first, last = block * rows, min(block * rows + rows, 64 * channels) - vec
+            if first <= last:
+                worst = max(worst, (offset(last) - offset(first) + vec) * size)
+        assert worst < 1 << 31, (vec, low, worst)
+        assert channels >= rows or worst > 1 << 28, (vec, low, worst)  # (and the bound is no more than a few times too small)
+    wide = plan(dtype, 64, time, channels, batch_stride=(1 << 40) + 64)
+    assert wide is not None and not chained(wide)
+
+
+def test_strides_that_run_backwards_or_batches_that_overlap_are_refused():
+    tuning = nat.Tuning(S, 1, 16, 1, 8)
+    assert plan(torch.float32, 4, 4096, 64, tuning=tuning) is not None
+    assert plan(torch.float32, 4, 4096, 64, row_stride=-1, elem_stride=64, tuning=tuning) is None
+    assert plan(torch.float32, 4, 4096, 64, batch_stride=32, elem_stride=64, tuning=tuning) is None
