@@ -673,6 +673,7 @@ int lookback_segments_plan(const Problem& q, int vec, int waves, int depth, int 
 bool lookback_segments_choose(const Problem& q, int family, int colblock, int mode, int desc, linrec_plan_t* out) {
   const bool half = q.dtype != LINREC_DTYPE_F32;
   if (q.row_stride != 1 || q.seqlen < kSegmentMinLen) return false;
+  const bool on_lines = q.elem_stride * elem_size_of(q.dtype) % 128 == 0;
   if (q.batched()) {
     // Batches of two or three channels: the lanes' accesses share no lines to speak of, and the three launches, which
     // number their lanes segment by segment, bring more of them (forward / backward: fp32 100 x 2000 x 2 21.3 / 37.9
@@ -701,7 +702,6 @@ bool lookback_segments_choose(const Problem& q, int family, int colblock, int mo
     if (q.is_bwd && colblock && q.seqlen < (half ? 384 : 448) && (colblock == 2 || q.rows_per_batch < 32)) return false;
     // (fp32 1862 x 632 x 20 with one row to a lane 105 / 220 against 101 / 181 for the plain column kernels)
     const bool pairs = q.rows_per_batch >= 32 && colblock_rows_per_lane(q, 2) == 2;
-    const bool on_lines = q.elem_stride * elem_size_of(q.dtype) % 128 == 0;
     const int64_t most = !pairs ? (half ? 32767 : 16384) : on_lines ? (half ? 16384 : 8192) : 65536;
     if (q.numseq > q.at(most)) return false;
   }
@@ -723,6 +723,13 @@ bool lookback_segments_choose(const Problem& q, int family, int colblock, int mo
     if (s[0] == 0 || lookback_segments_plan(q, s[0], s[1], s[2], mode, desc, &p) != LINREC_OK) continue;
     const int64_t lanes = ceil_div(q.numseq, int64_t(64) * s[0]) * 64;  // of a segment, with and without a row
     if (s[0] > 1 && (p.grid * 8 < 5 * q.cus || q.numseq * 4 < lanes * s[0] * 3 || (q.batched() && q.rows_per_batch < 32))) continue;
+    // The backward's column drift teams give way to four rows to a lane, to fewer only where that is as good: not in 16-bit
+    // storage to two where positions do not start on a 128-byte line (2 x 3000 x 1750 46.3 against 36.7, 8 x 2100 x 504 37.9
+    // against 30.6; but 8 x 2048 x 512 21.4 against 23.5), nor in fp32 to one where the rows make teams of eight (8 x 4096 x
+    // 175 46.6 against 41.5, 2 x 8192 x 701 81.1 against 77.8; but 3 x 4096 x 1365 121 against 126).
+    if (q.is_bwd && family == LINREC_FAMILY_COLDRIFT && q.rows_per_batch >= 32 &&
+        (half ? s[0] == 2 && !on_lines : s[0] == 1 && q.numseq < q.at(2048)))
+      return false;
     // A few workgroups more than there are CUs, which hold one of sixteen waves each: the rest of them runs on a chip that
     // is mostly idle.  Column blocks of two lane groups that fill most of it in one round are left in place there: fp32
     // forwards from 11/16 of the CUs up to 7/4 workgroups per CU (6656 rows, 8 x 1200 x 832 28.1 against 22.5; 7680 x 1700

@@ -93,6 +93,17 @@ def test_column_blocks_keep_short_backwards_and_launches_a_little_beyond_one_rou
         assert want or (p["family"], p["carry"]) == (nat.FAMILY_COLUMN, 2), (time, channels, is_bwd, p)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+def test_column_drift_teams_keep_backwards_that_would_take_narrow_accesses(dtype):
+    f32 = [(8, 4096, 175, False), (2, 8192, 701, False), (3, 4096, 467, False), (3, 4096, 1365, True), (56, 3132, 47, True),
+           (2, 8192, 700, True), (16, 2048, 512, True)]
+    f16 = [(2, 3000, 1750, False), (8, 2100, 504, False), (8, 2048, 512, True), (8, 4096, 1024, True), (3, 4096, 1344, True)]
+    for batch, time, channels, want in f32 if dtype == torch.float32 else f16:
+        p = plan(dtype, batch, time, channels, True)
+        assert chained(p) == want and (want or p["family"] == nat.FAMILY_COLDRIFT), (batch, time, channels, p)
+        assert chained(plan(dtype, batch, max(time, 4096), channels))
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("channels", [2, 32, 48, 64, 100, 1024])
 def test_a_lane_is_less_than_2_31_bytes_from_its_wave(dtype, channels):
