@@ -13,13 +13,13 @@
 // sweeps the tensors in the order of their addresses (a matrix with its scan axis strided is stored segment after
 // segment), and the segment a workgroup looks back to was started one whole round of blocks earlier.
 //
-// Measured (bf16, 4096 positions x 2048 rows, forward / backward): 12.6 / 18.8 us, 4.0 / 4.5 TB/s, where the three
-// launches take 26.3 / 36.0; 8 x 4096 x 1024: 38 / 60 us, 5.3 / 5.6 TB/s, where the column drift kernels take 54 / 76.5;
-// fp32 16 x 2048 x 512: 38 / 63 us, 5.3 / 5.3 TB/s, where column blocks / drift take 43 / 69.  The same kernel without
-// the look-back takes 11.7 / 18.1, 37.9 / 60.8 and 38.1 / 62.8 us: what is left to the rate of a plain stream is the
-// width of the accesses (two rows to a lane instead of four: 46 / 73 us on the second shape) and the one workgroup
-// per CU, whose loads and stores do not overlap.  16 waves and runs as long as the registers hold beat smaller
-// workgroups of which several share a CU (8 waves, the second shape: 47 / 77 us): descriptors per byte halve.
+// Measured (medians of launches replayed from a graph over several buffer sets, forward / backward): bf16 1 x 4096 x 2048
+// (batch x time x channels) 15.1 / 21.9 us, 3.3 / 3.8 TB/s, where the three launches take 28.1 / 37.4; 8 x 4096 x 1024
+// 43.7 / 67.6 us, 4.6 / 5.0 TB/s, where the column drift kernels take 54.5 / 78.4; fp32 16 x 2048 x 512 40.7 / 69.3 us,
+// 4.9 / 4.8 TB/s, where column blocks / drift take 45.5 / 70.9.  What is left to the rate of a plain stream is the width
+// of the accesses (bf16 8 x 4096 x 1024 with two rows to a lane instead of four 49.2 / 76.9 us, with one in eight waves
+// 51.2 / 83.3) and the one workgroup per CU, whose loads and stores do not overlap.  Runs as long as the registers hold:
+// descriptors per byte halve.
 //
 // A segment's map multiplies 128 or 256 coefficients, and the look-back composes several: the product can overflow where
 // the recurrence does not (nothing put in yet, or small values that grow and shrink again).  Where what leaves a segment

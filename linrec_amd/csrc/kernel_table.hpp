@@ -186,7 +186,7 @@ KernelGroup kernels_bf16_cols();
 
 // (one row to a lane: odd row counts, and too few rows for anything wider.  Sixteen waves instead of eight: bf16
 // 2 x 4096 x 256 (batch x time x channels) 8.9 / 14.3 us against 9.7 / 10.8, 2 x 8192 x 701 34.5 / 61.5 against 33.6 /
-// 58.3, fp32 46.4 / 81.6 against 43.0 / 78.3: not kept)
+// 58.3, fp32 46.4 / 81.6 against 43.0 / 78.3, smallest times of graph replays: not kept)
 #define COLLOOK_NARROW_KERNELS(...)                                                            \
   COLLOOK_FWD_(__VA_ARGS__, 8, 1, 16), COLLOOK_BWD_(__VA_ARGS__, 8, 1, 16)
 

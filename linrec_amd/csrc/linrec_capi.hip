@@ -652,22 +652,23 @@ int lookback_segments_plan(const Problem& q, int vec, int waves, int depth, int 
 // Whether the planner takes look-back segments for this problem (`family`: what the rules above chose), and with
 // which geometry.  One pass over the tensors, no three launches, and workgroups that need not divide the chip: they
 // win wherever the alternative reads its inputs twice, leaves part of the chip without a workgroup, or takes narrow
-// accesses that straddle lines.  Forward / backward in us against what was chosen before:
-//   few rows, a launch of microseconds: bf16 1 x 4096 x 2048 (batch x time x channels) 12.6 / 18.8 against 26.3 /
-//     36.0 (segments in three launches), fp32 8 x 1024 x 256 10.4 / 11.9 against 14.8 / 18.1, bf16 5 x 777 x 1001
-//     13.9 / 20.5 against 25.3 / 31.8;
-//   up to 8192 rows (16-bit storage: 16384): fp32 16 x 2048 x 512 39.7 / 64.2 against 43.2 / 70.0 (column blocks,
-//     column drift), 2 x 8192 x 700 38.7 / 56.7 against 47.5 / 72.7, bf16 8 x 4096 x 1024 43.2 / 61.6 against 55.0 /
-//     76.7 (column drift), 4 x 4096 x 4096 82.3 / 142.6 against 86.9 / 151.5 (column blocks);
-//   more rows: where a position's rows do not start on a 128-byte line, fp32 30 x 1024 x 1500 136.1 / 198.0 against
-//     168.9 / 291.4, bf16 7 x 4096 x 3500 161.7 / 280.7 against 218.0 / 404.1, 30 x 1111 x 2000 104.2 / 177.6 against
-//     118.8 / 221.2; where it does, the column blocks are as good or better (fp32 4 x 4096 x 4096 145.6 / 238.8 against
-//     135.6 / 239.0, 7 x 2048 x 4000 130.9 / 197.8 against 124.1 / 193.1, bf16 32 x 1024 x 1024 43.1 / 64.2 against 37.0 /
-//     63.9), and with one row to a lane they are from 16384 rows on (fp32 31 x 600 x 777 64.7 / 112.2 against 61.4 /
-//     111.4; 16-bit storage, which has no column block for that, from 32768: bf16 8 x 1024 x 4097 95.7 against 91.8);
-//   a forward of less than 1024 positions stays with the column blocks (fp32 8 x 700 x 1024 16.2 against 16.2) and one
-//     of less than 4096 with the column drift teams where those apply (fp32 3 x 2100 x 1344 25.5 against 26.3; bf16
-//     3 x 2100 x 2688 would gain, 25.4 against 31.5).
+// accesses that straddle lines.  Forward / backward in us (medians of launches replayed from a graph over two to six
+// buffer sets, both sides in turn; all figures of this function) against what the rules above choose:
+//   few rows, a launch of microseconds: bf16 1 x 4096 x 2048 (batch x time x channels) 15.1 / 21.9 against 28.1 /
+//     37.4 (segments in three launches), fp32 8 x 1024 x 256 10.5 / 12.4 against 15.5 / 19.4, bf16 5 x 777 x 1001
+//     14.9 / 21.4 against 25.3 / 32.1;
+//   up to 8192 rows (16-bit storage: 16384): fp32 16 x 2048 x 512 40.7 / 69.3 against 45.5 / 70.9 (column blocks,
+//     column drift), 2 x 8192 x 700 39.9 / 58.4 against 48.9 / 74.1, bf16 8 x 4096 x 1024 43.7 / 67.6 against 54.5 /
+//     78.4 (column drift), 4 x 4096 x 4096 87 / 148 against 89 / 143 (column blocks);
+//   more rows: where a position's rows do not start on a 128-byte line, fp32 30 x 1024 x 1500 144 / 220 against
+//     186 / 337, bf16 7 x 4096 x 3500 162 / 281 against 219 / 397, 30 x 1111 x 2000 104 / 177 against 123 / 221; where it
+//     does, the column blocks are as good or better (fp32 4 x 4096 x 4096 146 / 244 against 138 / 242, 7 x 2048 x 4000
+//     131 / 220 against 124 / 210, bf16 32 x 1024 x 1024 45.2 / 64.7 against 39.1 / 64.3), and with one row to a lane
+//     they are from 16384 rows on (fp32 31 x 600 x 777 69.8 / 118 against 66.3 / 118; 16-bit storage, which has no
+//     column block for that, from 32768: bf16 8 x 1024 x 4097 96.8 / 183 against 93.3 / 187);
+//   a forward of less than 1024 positions stays with the column blocks (fp32 8 x 700 x 1024 17.0 against 17.7) and one
+//     of less than 4096 with the column drift teams where those apply (fp32 3 x 2100 x 1344 27.0 against 27.9; bf16
+//     3 x 2100 x 2688 would gain, 27.0 against 32.7).
 // One matrix (not a batch of them): 16-bit storage where the three launches were chosen, up to 8192 positions; the
 // rest stays with the teams and the three launches.
 bool lookback_segments_choose(const Problem& q, int family, int colblock, int mode, int desc, linrec_plan_t* out) {
@@ -706,9 +707,9 @@ bool lookback_segments_choose(const Problem& q, int family, int colblock, int mo
     if (q.numseq > q.at(most)) return false;
   }
   // The widest access that makes a workgroup for 5 of 8 CUs: it needs the fewest descriptors and the memory system
-  // likes it best (bf16 8 x 4096 x 1024 forward: 43.2 us with four rows to a lane, 47.6 with two, 51.7 with one), but
-  // half a chip is worse than a narrower access (bf16 1 x 4096 x 2048: 128 workgroups of four rows to a lane 17.4 us,
-  // 256 of two 13.7; fp32 2 x 4096 x 256 backward: 128 of two 14.4, 256 of one 12.9).  More than one row to a lane needs
+  // likes it best (bf16 8 x 4096 x 1024 43.7 / 67.6 with four rows to a lane, 49.2 / 76.9 with two, 51.2 / 83.3 with one), but
+  // half a chip is worse than a narrower access (bf16 1 x 4096 x 2048: 128 workgroups of four rows to a lane 18.4 / 25.6,
+  // 256 of two 15.1 / 21.9; fp32 2 x 4096 x 256 backward: 128 of two 15.4, 256 of one 13.7).  More than one row to a lane needs
   // rows for three quarters of the lanes, or a workgroup's accesses and descriptors are mostly padding (fp32 2 x 262144 x
   // 32: 78 / 131 with two rows to a lane in the forward and four in the backward, 57 / 78 with one, 78 / 102 in three
   // launches; bf16 2 x 262144 x 16 72 / 93, 48 / 58 and 50 / 76), and lanes that lie next to each other: batches of at
