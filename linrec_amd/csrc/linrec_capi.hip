@@ -707,9 +707,12 @@ bool lookback_segments_choose(const Problem& q, int family, int colblock, int mo
     if (q.numseq > q.at(most)) return false;
   }
   // The widest access that makes a workgroup for 5 of 8 CUs: it needs the fewest descriptors and the memory system
-  // likes it best (bf16 8 x 4096 x 1024 43.7 / 67.6 with four rows to a lane, 49.2 / 76.9 with two, 51.2 / 83.3 with one), but
-  // half a chip is worse than a narrower access (bf16 1 x 4096 x 2048: 128 workgroups of four rows to a lane 18.4 / 25.6,
-  // 256 of two 15.1 / 21.9; fp32 2 x 4096 x 256 backward: 128 of two 15.4, 256 of one 13.7).  More than one row to a lane needs
+  // likes it best (bf16 8 x 4096 x 1024 43.7 / 67.6 with four rows to a lane, 49.2 / 76.9 with two, 51.2 / 83.3 with one; fp32
+  // 4 x 4096 x 1024 41.1 / 66.0 with two in the forward and four in the backward, 44.6 / 73.9 with one, 8 x 4096 x 700 74 /
+  // 110 and 92 / 166; at 3 x 4200 x 2688, where positions are ten and a half KiB apart, one is ahead, 75.3 / 124.9 against
+  // 77.8 / 131.4: not told apart here), but half a chip is worse than a narrower access (bf16 1 x 4096 x 2048: 128 workgroups
+  // of four rows to a lane 18.4 / 25.6, 256 of two 15.1 / 21.9; fp32 2 x 4096 x 256 backward: 128 of two 15.4, 256 of one
+  // 13.7).  More than one row to a lane needs
   // rows for three quarters of the lanes, or a workgroup's accesses and descriptors are mostly padding (fp32 2 x 262144 x
   // 32: 78 / 131 with two rows to a lane in the forward and four in the backward, 57 / 78 with one, 78 / 102 in three
   // launches; bf16 2 x 262144 x 16 72 / 93, 48 / 58 and 50 / 76), and lanes that lie next to each other: batches of at
