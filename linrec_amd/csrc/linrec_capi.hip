@@ -697,12 +697,12 @@ bool lookback_segments_choose(const Problem& q, int family, int colblock, int mo
   } else {
     if (!q.is_bwd && colblock && q.seqlen < 1024) return false;
     if (!q.is_bwd && family == LINREC_FAMILY_COLDRIFT && q.seqlen < 4096) return false;
-    // The column blocks of two lane groups keep the shortest axes in the backward as well (fp32 8 x 256 x 1024 12.0 against
-    // 10.3, 8 x 352 x 832 15.4 against 13.0, 4000 x 300 x 4 160 against 131; bf16 8 x 300 x 1536 16.1 against 14.3, 2000 x
-    // 300 x 8 66.7 against 49.3; but fp32 8 x 448 x 768 13.5 against 16.3, bf16 8 x 512 x 1536 20.1 against 21.5).
-    if (q.is_bwd && colblock && q.seqlen < (half ? 384 : 448) && (colblock == 2 || q.rows_per_batch < 32)) return false;
+    // 16-bit storage: column blocks keep the shortest axes in the backward as well (8 x 300 x 1536 16.1 against 14.3, 2000 x
+    // 300 x 8 54.9 against 49.0; but 8 x 380 x 2048 17.9 against 18.4, and off the 128-byte lines 8 x 256 x 1368 17.5
+    // against 15.3 but 8 x 271 x 2042 20.8 against 22.9).
+    if (half && q.is_bwd && colblock == 2 && q.seqlen < (on_lines || q.rows_per_batch < 32 ? 352 : 264)) return false;
     // (fp32 1862 x 632 x 20 with one row to a lane 105 / 220 against 101 / 181 for the plain column kernels)
-    const bool pairs = q.rows_per_batch >= 32 && colblock_rows_per_lane(q, 2) == 2;
+    const bool pairs = q.rows_per_batch >= 24 && colblock_rows_per_lane(q, 2) == 2;
     const int64_t most = !pairs ? (half ? 32767 : 16384) : on_lines ? (half ? 16384 : 8192) : 65536;
     if (q.numseq > q.at(most)) return false;
   }
@@ -713,10 +713,10 @@ bool lookback_segments_choose(const Problem& q, int family, int colblock, int mo
   // 77.8 / 131.4: not told apart here), but half a chip is worse than a narrower access (bf16 1 x 4096 x 2048: 128 workgroups
   // of four rows to a lane 18.4 / 25.6, 256 of two 15.1 / 21.9; fp32 2 x 4096 x 256 backward: 128 of two 15.4, 256 of one
   // 13.7).  More than one row to a lane needs
-  // rows for three quarters of the lanes, or a workgroup's accesses and descriptors are mostly padding (fp32 2 x 262144 x
+  // rows for more than half of its lanes, or the accesses and descriptors are mostly padding (fp32 2 x 262144 x
   // 32: 78 / 131 with two rows to a lane in the forward and four in the backward, 57 / 78 with one, 78 / 102 in three
   // launches; bf16 2 x 262144 x 16 72 / 93, 48 / 58 and 50 / 76), and lanes that lie next to each other: batches of at
-  // least 32 channels (fp32 500 x 2000 x 8 47.5 / 114.9, 41.7 / 87.4 and 53.5 / 101.6; bf16 8 x 262144 x 16 127 / 206,
+  // least 24 channels (fp32 500 x 2000 x 8 47.5 / 114.9, 41.7 / 87.4 and 53.5 / 101.6; bf16 8 x 262144 x 16 127 / 206,
   // 106 / 161 and 147 / 264).
   // {rows per lane, waves, positions per run}: the run as long as its tensors fit the registers
   static const int shapes[2][2][3][3] = {{{{2, 16, 16}, {1, 8, 16}, {0, 0, 0}}, {{4, 16, 8}, {2, 16, 8}, {1, 8, 16}}},
@@ -726,7 +726,7 @@ bool lookback_segments_choose(const Problem& q, int family, int colblock, int mo
     std::memset(&p, 0, sizeof(p));
     if (s[0] == 0 || lookback_segments_plan(q, s[0], s[1], s[2], mode, desc, &p) != LINREC_OK) continue;
     const int64_t lanes = ceil_div(q.numseq, int64_t(64) * s[0]) * 64;  // of a segment, with and without a row
-    if (s[0] > 1 && (p.grid * 8 < 5 * q.cus || q.numseq * 4 < lanes * s[0] * 3 || (q.batched() && q.rows_per_batch < 32))) continue;
+    if (s[0] > 1 && (p.grid * 8 < 5 * q.cus || q.numseq * 2 <= lanes * s[0] || (q.batched() && q.rows_per_batch < 24))) continue;
     // The backward's column drift teams give way to four rows to a lane, to fewer only where that is as good: not in 16-bit
     // storage to two where positions do not start on a 128-byte line (2 x 3000 x 1750 46.3 against 36.7, 8 x 2100 x 504 37.9
     // against 30.6; but 8 x 2048 x 512 21.4 against 23.5), nor in fp32 to one where the rows make teams of eight (8 x 4096 x
@@ -734,21 +734,28 @@ bool lookback_segments_choose(const Problem& q, int family, int colblock, int mo
     if (q.is_bwd && family == LINREC_FAMILY_COLDRIFT && q.rows_per_batch >= 32 &&
         (half ? s[0] == 2 && !on_lines : s[0] == 1 && q.numseq < q.at(2048)))
       return false;
+    // fp32: column blocks keep the shortest axes in the backward, one row to a lane (8 x 256 x 1024 12.0 against 10.3, 8 x
+    // 352 x 832 15.4 against 13.0; with two 8 x 300 x 896 13.8 against 12.4, but 8 x 352 x 1024 13.6 against 15.5, 8 x 448 x
+    // 768 13.5 against 16.3).
+    if (!half && q.is_bwd && colblock == 2 && q.seqlen < (s[0] == 1 ? 448 : q.numseq < q.at(8192) ? 320 : 0)) return false;
     // A few workgroups more than there are CUs, which hold one of sixteen waves each: the rest of them runs on a chip that
-    // is mostly idle.  Column blocks of two lane groups that fill most of it in one round are left in place there: fp32
-    // forwards from 11/16 of the CUs up to 7/4 workgroups per CU (6656 rows, 8 x 1200 x 832 28.1 against 22.5; 7680 x 1700
-    // 34.8 against 32.2; 8192 x 1200 30.0 against 27.4; but 8192 x 1700 35.7 against 37.3, 5120 x 1800 30.8 against 31.7),
-    // fp32 backwards of two rows to a lane alike (6656 x 640 25.7 against 19.9), of four up to 3/2 workgroups per CU where
-    // positions are not whole KiB apart (16 x 1200 x 416 36.0 against 32.1, 8 x 1400 x 960 47.8 against 44.5; but 2 x 1200 x
-    // 3328 35.7 against 39.5, 8 x 1536 x 768 44.7 against 51.0: there the blocks, which read position after position, do
-    // worse), 16-bit storage from 7/8 of the CUs up to 11/8 (14336 x 1280 30.8 / 48.2 against 26.8 / 43.3; but 12288 x 1400
-    // 28.1 / 41.8 against 33.4 / 46.6).
-    if (q.batched() && colblock == 2 && p.waves == 16 && p.grid > q.cus) {
+    // is mostly idle.  Column blocks of two lane groups that fill most of it in one round are left in place there:
+    //   fp32 forwards and backwards of two rows to a lane from 11/16 of the CUs up to 7/4 workgroups per CU (6656 rows, 8 x
+    //     1200 x 832 28.1 against 22.5, backward 8 x 640 x 832 25.7 against 19.9; 7680 x 1700 34.8 against 32.2; but 5120 x
+    //     1800 30.8 against 31.7), where positions are whole KiB apart from 13/16 of the CUs up to 3/2 (8 x 1200 x 1024 30.0
+    //     against 27.4, 2 x 1200 x 3328 28.2 against 24.4; but 8 x 2048 x 768 32.4 against 36.8: there the blocks, which read
+    //     position after position, do worse);
+    //   fp32 backwards of four rows to a lane up to 3/2 workgroups per CU where positions are not whole KiB apart (16 x 1200 x
+    //     416 36.0 against 32.1, 8 x 1400 x 960 47.8 against 44.5; but 2 x 1200 x 3328 35.7 against 39.5);
+    //   16-bit storage from 7/8 of the CUs up to 9/8 workgroups per CU, in whole steps of the blocks up to 11/8 (8 x 1280 x
+    //     1792 30.8 / 48.2 against 26.8 / 43.3, 16 x 1200 x 896 29.2 / 43.5 against 27.0 / 39.4; but 16 x 1200 x 1024 29.9 /
+    //     45.1 against 33.0 / 48.0, 8 x 1400 x 1536 28.1 / 41.8 against 33.4 / 46.6).
+    if (q.batched() && colblock == 2 && on_lines && p.waves == 16 && p.grid > q.cus) {
       const int64_t blocks = ceil_div(q.numseq / colblock_rows_per_lane(q, 0), 32);
-      if (half ? blocks * 8 >= 7 * q.cus && p.grid * 8 < 11 * q.cus
-               : blocks * 16 >= 11 * q.cus &&
-                     (s[0] <= 2 ? p.grid * 4 < 7 * q.cus : q.elem_stride * 4 % 1024 != 0 && p.grid * 2 < 3 * q.cus))
-        return false;
+      const bool whole_kib = q.elem_stride * 4 % 1024 == 0;
+      const bool fills = blocks * 16 >= (half ? 14 : s[0] <= 2 && whole_kib ? 13 : 11) * q.cus;
+      const int64_t up_to = half ? (q.seqlen % 128 == 0 ? 11 : 9) : s[0] <= 2 ? (whole_kib ? 12 : 14) : whole_kib ? 0 : 12;
+      if (fills && p.grid * 8 < up_to * q.cus) return false;
     }
     // (a caller that can only give so much workspace is served by the kernels that need less)
     if (q.workspace_cap && p.workspace_bytes > q.workspace_cap) return false;
