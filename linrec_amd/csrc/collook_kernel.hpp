@@ -13,13 +13,27 @@
 // sweeps the tensors in the order of their addresses (a matrix with its scan axis strided is stored segment after
 // segment), and the segment a workgroup looks back to was started one whole round of blocks earlier.
 //
+// A lane's rows need not be aligned to more than an element: what a wave reads of a position that does not start on a
+// 128-byte line takes one line more than it holds, whatever the phase (memory-only, 16-bit matrices of 2050 and 2052
+// columns, 8 bytes to a lane: 93 and 89 us where 2048 take 64), so the wider the access the less of that, and rows off
+// 16 bytes get the same widths as the others.  The line at the border of two blocks is wanted by both: such launches load
+// through the caches, and eight segments are dealt out at a time so that the blocks of a segment run on one XCD and
+// find the border lines in its L2 (memory-only, 16640 x 4022, 8 bytes to a lane: 101.7 us as before, 93 with cached loads,
+// 85 with both; where positions start on lines cached loads cost 4 %).  That order also serves backwards on whole
+// lines (fp32 32768 x 1024 123 us instead of 130, 16384 x 4096 233 instead of 247), not forwards (16 x 2048 x 512 43.6
+// instead of 39.5).
+//
 // Measured (medians of launches replayed from a graph over several buffer sets, forward / backward): bf16 1 x 4096 x 2048
-// (batch x time x channels) 15.1 / 21.9 us, 3.3 / 3.8 TB/s, where the three launches take 28.1 / 37.4; 8 x 4096 x 1024
-// 43.7 / 67.6 us, 4.6 / 5.0 TB/s, where the column drift kernels take 54.5 / 78.4; fp32 16 x 2048 x 512 40.7 / 69.3 us,
-// 4.9 / 4.8 TB/s, where column blocks / drift take 45.5 / 70.9.  What is left to the rate of a plain stream is the width
-// of the accesses (bf16 8 x 4096 x 1024 with two rows to a lane instead of four 49.2 / 76.9 us, with one in eight waves
-// 51.2 / 83.3) and the one workgroup per CU, whose loads and stores do not overlap.  Runs as long as the registers hold:
-// descriptors per byte halve.
+// (batch x time x channels) 15.1 / 22.0 us, 3.3 / 3.8 TB/s, where the three launches take 28.1 / 37.4; 8 x 4096 x 1024
+// 42.1 / 64.9 us, 4.8 / 5.2 TB/s, where the column drift kernels take 54.5 / 78.4; fp32 16 x 2048 x 512 39.5 / 66.8 us,
+// 5.1 / 5.0 TB/s, where column blocks / drift take 45.5 / 70.9.  Off the lines, with narrow aligned accesses in the order
+// of the segments before / now: fp32 2 x 125567 x 222 184 / 325 before, 166 / 244 now, bf16 131 / 227 and 90 / 149, 8 x 4096 x 175
+// 20.7 / 34.5 and 13.2 / 23.4, fp32 30 x 1024 x 1500 141 / 215 and 135 / 198.  What is left to the rate of a plain stream is
+// the width of the accesses (bf16 8 x 4096 x 1024 with two rows to a lane instead of four 48.4 / 75.6 us, with one in eight
+// waves 52.9 / 82.8) and the one workgroup per CU, whose loads and stores do not overlap: a memory-only launch of this
+// shape takes 79 us for fp32 32768 x 1024 forward where small workgroups take 63, but smaller segments pay more for the
+// exchange than that brings (two workgroups of half the segment 84.6 us, four of a quarter 89 against 82.9).  Runs as
+// long as the registers hold: descriptors per byte halve.
 //
 // A segment's map multiplies 128 or 256 coefficients, and the look-back composes several: the product can overflow where
 // the recurrence does not (nothing put in yet, or small values that grow and shrink again).  Where what leaves a segment
@@ -42,7 +56,50 @@ namespace linrec {
 
 constexpr int PHASE_LOOKBACK = 3;  // the kernel table's code beside PHASE_REDUCE and PHASE_APPLY
 
-// (of args.chain: tasks = blocks of rows, num_tiles = workgroups)
+// VEC adjacent rows of one position by one access that need not be aligned to more than an element.
+template <typename T, int VEC>
+struct AnyPack {
+  typedef T type __attribute__((ext_vector_type(VEC), aligned(sizeof(T))));
+};
+template <int VEC, bool STREAM, typename T>
+__device__ __forceinline__ Held<T, VEC> ld_any(const T* p) {
+  Held<T, VEC> h;
+  if constexpr (VEC == 1) {
+    const T q = STREAM ? stream_load(p) : *p;
+    if constexpr (std::is_same_v<T, float>) h.q.v[0] = q;
+    else h.q[0] = q;
+  } else {
+    using V = typename Pack<T, VEC>::type;
+    using A = typename AnyPack<T, VEC>::type;
+    const A* pa = reinterpret_cast<const A*>(p);
+    const V q = STREAM && LINREC_NT_LOAD ? V(__builtin_nontemporal_load(pa)) : V(*pa);
+    if constexpr (std::is_same_v<T, float>) {
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) h.q.v[e] = q[e];
+    } else {
+      h.q = q;
+    }
+  }
+  return h;
+}
+template <int VEC, typename T>
+__device__ __forceinline__ void st_any(T* p, const Lanes<VEC>& r) {
+  if constexpr (VEC == 1) {
+    stream_store(T(r.v[0]), p);
+  } else {
+    using A = typename AnyPack<T, VEC>::type;
+    A q;
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) q[e] = T(r.v[e]);
+#if LINREC_NT_STORE
+    __builtin_nontemporal_store(q, reinterpret_cast<A*>(p));
+#else
+    *reinterpret_cast<A*>(p) = q;
+#endif
+  }
+}
+
+// (of args.chain: tasks = blocks of lanes, num_tiles = workgroups; of args.col: lanes_per_segment = lanes of a segment)
 template <typename T, int VEC, int U, int NW, int MODE, bool DESC>
 __global__ __launch_bounds__(64 * NW) void collook_kernel(ColDriftArgs args) {
   static_assert(VEC <= NW, "a wave per row of a lane looks back");
@@ -65,19 +122,34 @@ __global__ __launch_bounds__(64 * NW) void collook_kernel(ColDriftArgs args) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int blocks = ch.tasks;
-  const int k = int(blockIdx.x / unsigned(blocks));  // segment
-  const int block = int(blockIdx.x - unsigned(k) * unsigned(blocks));
-  auto base_of = [&](long long row) __attribute__((always_inline)) {
-    if (p.rows_per_batch >= p.numseq) return row * p.row_stride;
-    const long long batch = row / p.rows_per_batch;
-    return batch * p.batch_stride + (row - batch * p.rows_per_batch) * p.row_stride;
-  };
-  long long r0 = ((long long)block * 64 + lane) * VEC;
-  const bool active = r0 < p.numseq;
-  if (!active) r0 = p.numseq - VEC;  // lanes beyond the last row read the last rows again and store nothing
+  // Segment and block of lanes.  Workgroups are dealt to the eight XCDs in turn, so with eight segments dealt out at a time
+  // (ch.row_groups; 1 otherwise) one XCD runs the blocks of a segment.  A segment's workgroup still has a larger number
+  // than the same block's of the segments before.
+  int k, block;
+  {
+    const unsigned id = blockIdx.x, nb = unsigned(blocks), at_once = unsigned(ch.row_groups);
+    const unsigned group = at_once * nb, g = id / group, r = id - g * group;
+    if (at_once > 1u && (g + 1u) * group <= gridDim.x) {
+      block = int(r / at_once);
+      k = int(g * at_once + (r - unsigned(block) * at_once));
+    } else {  // (also the last segments, less than eight of them)
+      k = int(id / nb);
+      block = int(id - unsigned(k) * nb);
+    }
+  }
+  // Lanes are numbered batch by batch; where a batch's rows are not a multiple of VEC its last lane starts early and
+  // shares rows with the one before it (both compute and store them).
+  unsigned lane_no = unsigned(block) * 64u + unsigned(lane);  // (the planner keeps lanes and rows of a segment below 2^31)
+  const bool active = lane_no < unsigned(p.lanes_per_segment);
+  if (!active) lane_no = unsigned(p.lanes_per_segment) - 1u;  // lanes beyond the last row read the last rows again and store nothing
+  const unsigned rows = unsigned(p.rows_per_batch < p.numseq ? p.rows_per_batch : p.numseq);
+  const unsigned lanes = (rows + unsigned(VEC) - 1u) / unsigned(VEC);
+  const unsigned batch = p.rows_per_batch < p.numseq ? lane_no / lanes : 0u;
+  unsigned row = (lane_no - batch * lanes) * unsigned(VEC);
+  if (row > rows - unsigned(VEC)) row = rows - unsigned(VEC);
   // A wave's accesses are a scalar address plus 32 bits per lane (the planner sees to it that a block's rows span
   // less than 2^31 bytes): 64-bit addresses per lane took 30 to 40 registers, and with them a workgroup per CU.
-  const long long base = base_of(r0);
+  const long long base = (long long)batch * p.batch_stride + (long long)row * p.row_stride;
   const long long wbase = (long long)(uint32_t)__builtin_amdgcn_readfirstlane(int(base)) |
                           ((long long)__builtin_amdgcn_readfirstlane(int(base >> 32)) << 32);
   const uint32_t lane_bytes = uint32_t(base - wbase) * uint32_t(sizeof(T));
@@ -98,21 +170,23 @@ __global__ __launch_bounds__(64 * NW) void collook_kernel(ColDriftArgs args) {
     Held<T, VEC> x[U], c[U], yn[NEED_Y ? U : 1];
   };
   const int n0 = k * STEP + wave * U;
+  // positions a whole number of 128-byte lines apart: no line is wanted twice
+  const bool on_lines = p.elem_stride * (long long)sizeof(T) % 128 == 0;
   // FULL: all positions of the segment exist and, for the backward, so does the last one's successor.
-  auto segment = [&](auto full_tag) __attribute__((always_inline)) {
-    constexpr bool FULL = decltype(full_tag)::value;
+  auto segment = [&](auto full_tag, auto stream_tag) __attribute__((always_inline)) {
+    constexpr bool FULL = decltype(full_tag)::value, STREAM = decltype(stream_tag)::value;
     Batch bt;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int n = n0 + u;  // position in scan order
       const int l = DESC ? L - 1 - n : n;
       if (FULL || n < L) {
-        bt.x[u] = ld_held<VEC>(at(in0, l));
-        bt.c[u] = ld_held<VEC>(at(coef, l));
+        bt.x[u] = ld_any<VEC, STREAM>(at(in0, l));
+        bt.c[u] = ld_any<VEC, STREAM>(at(coef, l));
         if constexpr (NEED_Y) {
           const int ln = DESC ? l - 1 : l + 1;  // saved output one step further along this scan
           if (FULL || (ln >= 0 && ln < L)) {
-            bt.yn[u] = ld_held<VEC>(at(aux, ln));
+            bt.yn[u] = ld_any<VEC, STREAM>(at(aux, ln));
           } else {
             bt.yn[u] = held_zero<T, VEC>();
           }
@@ -226,8 +300,7 @@ __global__ __launch_bounds__(64 * NW) void collook_kernel(ColDriftArgs args) {
             if (lane == 0) __hip_atomic_fetch_add(&ch.ws->gave_up, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             if (!have) {
               // what enters the segment from the row's own data: the plain sequential walk
-              const long long row = r0 + (VEC > 1 ? wave : 0);
-              const long long rb = base_of(row);
+              const long long rb = base + (VEC > 1 ? wave : 0) * p.row_stride;
               float val = 0.0f;
               for (int n = 0; n < k * STEP; ++n) {
                 const int l = DESC ? L - 1 - n : n;
@@ -269,7 +342,7 @@ __global__ __launch_bounds__(64 * NW) void collook_kernel(ColDriftArgs args) {
         if constexpr (MODE == 0) {
 #pragma unroll
           for (int e = 0; e < VEC; ++e) val.v[e] = n == 0 ? x.v[e] : fmaf(val.v[e], c.v[e], x.v[e]);
-          if (active) st_rows<VEC>(at(out0, l), val);
+          if (active) st_any<VEC>(at(out0, l), val);
         } else {
           const Lanes<VEC> yn = widen(held_again(bt.yn[u]));
           Lanes<VEC> dx, dc;
@@ -280,15 +353,17 @@ __global__ __launch_bounds__(64 * NW) void collook_kernel(ColDriftArgs args) {
             val.v[e] = dx.v[e] * c.v[e];
           }
           if (active) {
-            st_rows<VEC>(at(out0, l), dx);
-            st_rows<VEC>(at(out1, l), dc);
+            st_any<VEC>(at(out0, l), dx);
+            st_any<VEC>(at(out1, l), dc);
           }
         }
       }
     }
   };
-  if ((k + 1) * (long long)STEP <= (NEED_Y ? L - 1 : L)) segment(std::true_type{});
-  else segment(std::false_type{});
+  const bool full = (k + 1) * (long long)STEP <= (NEED_Y ? L - 1 : L);
+  if (full && on_lines) segment(std::true_type{}, std::true_type{});
+  else if (full) segment(std::true_type{}, std::false_type{});
+  else segment(std::false_type{}, std::false_type{});
 
   // (the look-back waves are past the last barrier: no descriptor of this launch is touched by this workgroup again)
   if (threadIdx.x == 0) {

@@ -622,11 +622,28 @@ bool coldrift_applies(const Problem& q) {
 }
 // The plan of a segmented launch whose segments are chained by look-back (one launch): `waves` waves per workgroup
 // with runs of `depth` positions, `vec` rows to a lane.
+// Lanes of a segment: `vec` adjacent rows each, a batch's last lane overlapping the one before it where the rows of a batch
+// are not a multiple of `vec`.
+int64_t lookback_lanes(const Problem& q, int64_t vec) {
+  return q.batched() ? q.numseq / q.rows_per_batch * ceil_div(q.rows_per_batch, vec) : ceil_div(q.numseq, vec);
+}
+// Segments dealt out at a time (collook_kernel.hpp): eight where that is as good or better, whole groups of which there are
+// at least two.  Forward / backward in us, eight against one: off the 128-byte lines fp32 8326 x 4022 (time x channels) 91.6 /
+// 140.7 against 98.0 / 150.2, 2 x 125567 x 222 165.9 / 244 against 172.4 / 251, bf16 8 x 4096 x 700 40.6 / 69.0 against 42.9 /
+// 73.2, but 3 x 1813 x 1464 (eight segments) 33.7 against 28.0; on them fp32 32768 x 1024 79.9 / 122.8 against 82.9 / 129.7,
+// 16 x 2048 x 512 43.6 / 66.8 against 39.5 / 69.5, bf16 32768 x 1024 47.6 / 67.6 against 44.4 / 68.8, of two blocks fp32
+// 16384 x 512 24.2 / 33.9 against 22.3 / 32.6.
+int64_t lookback_segments_at_once(const Problem& q, int64_t blocks, int64_t segments) {
+  const bool on_lines = q.elem_stride * elem_size_of(q.dtype) % 128 == 0;
+  return segments >= 16 && (on_lines ? q.is_bwd && blocks >= 4 : blocks >= 2) ? 8 : 1;
+}
 int lookback_segments_plan(const Problem& q, int vec, int waves, int depth, int mode, int desc, linrec_plan_t* out) {
-  if (vec < 1 || colblock_rows_per_lane(q, vec) != vec) return LINREC_E_UNSUPPORTED;
+  if (vec < 1 || colblock_rows_per_lane(q, 1) != 1) return LINREC_E_UNSUPPORTED;
+  const int64_t rpb = q.batched() ? q.rows_per_batch : q.numseq;
+  if (vec > 1 && (q.row_stride != 1 || rpb < vec)) return LINREC_E_UNSUPPORTED;
   // (a lane's offset from its wave's first row is 32 bits of bytes: strides forward, a block's rows within 2^31 bytes)
   {
-    const int64_t rpb = q.batched() ? q.rows_per_batch : q.numseq, rows = 64 * int64_t(vec);
+    const int64_t rows = 64 * int64_t(vec);
     if (q.row_stride < 0 || (q.batched() && q.batch_stride < rpb * q.row_stride)) return LINREC_E_UNSUPPORTED;
     const int64_t bound = (int64_t(1) << 31) / elem_size_of(q.dtype);
     if (q.row_stride > bound / rows || (q.batched() && q.batch_stride > bound / 2 / (rows / rpb + 2)) || q.row_stride * rows > bound / 2)
@@ -635,7 +652,7 @@ int lookback_segments_plan(const Problem& q, int vec, int waves, int depth, int 
   const int id = find_kernel(q.dtype, LINREC_FAMILY_SEGMENT, waves, depth, vec, mode, desc, linrec::PHASE_LOOKBACK);
   if (id < 0) return LINREC_E_UNSUPPORTED;
   const int64_t rows_per_block = int64_t(64) * vec;
-  const int64_t blocks = ceil_div(q.numseq, rows_per_block);
+  const int64_t blocks = ceil_div(lookback_lanes(q, vec), 64);
   const int64_t segments = ceil_div(q.seqlen, int64_t(waves) * depth);
   if (blocks * segments * rows_per_block > 2147483647LL) return LINREC_E_TOO_LARGE;
   out->family = LINREC_FAMILY_SEGMENT;
@@ -657,87 +674,136 @@ int lookback_segments_plan(const Problem& q, int vec, int waves, int depth, int 
 //   few rows, a launch of microseconds: bf16 1 x 4096 x 2048 (batch x time x channels) 15.1 / 21.9 against 28.1 /
 //     37.4 (segments in three launches), fp32 8 x 1024 x 256 10.5 / 12.4 against 15.5 / 19.4, bf16 5 x 777 x 1001
 //     14.9 / 21.4 against 25.3 / 32.1;
-//   up to 8192 rows (16-bit storage: 16384): fp32 16 x 2048 x 512 40.7 / 69.3 against 45.5 / 70.9 (column blocks,
-//     column drift), 2 x 8192 x 700 39.9 / 58.4 against 48.9 / 74.1, bf16 8 x 4096 x 1024 43.7 / 67.6 against 54.5 /
-//     78.4 (column drift), 4 x 4096 x 4096 87 / 148 against 89 / 143 (column blocks);
-//   more rows: where a position's rows do not start on a 128-byte line, fp32 30 x 1024 x 1500 144 / 220 against
-//     186 / 337, bf16 7 x 4096 x 3500 162 / 281 against 219 / 397, 30 x 1111 x 2000 104 / 177 against 123 / 221; where it
-//     does, the column blocks are as good or better (fp32 4 x 4096 x 4096 146 / 244 against 138 / 242, 7 x 2048 x 4000
-//     131 / 220 against 124 / 210, bf16 32 x 1024 x 1024 45.2 / 64.7 against 39.1 / 64.3), and with one row to a lane
-//     they are from 16384 rows on (fp32 31 x 600 x 777 69.8 / 118 against 66.3 / 118; 16-bit storage, which has no
-//     column block for that, from 32768: bf16 8 x 1024 x 4097 96.8 / 183 against 93.3 / 187);
-//   a forward of less than 1024 positions stays with the column blocks (fp32 8 x 700 x 1024 17.0 against 17.7) and one
-//     of less than 4096 with the column drift teams where those apply (fp32 3 x 2100 x 1344 27.0 against 27.9; bf16
-//     3 x 2100 x 2688 would gain, 27.0 against 32.7).
-// One matrix (not a batch of them): 16-bit storage where the three launches were chosen, up to 8192 positions; the
-// rest stays with the teams and the three launches.
+//   up to 8192 rows (16-bit storage: 16384): fp32 16 x 2048 x 512 39.5 / 66.8 against 45.5 / 70.9 (column blocks,
+//     column drift), 2 x 8192 x 700 39.9 / 58.4 against 48.9 / 74.1, bf16 8 x 4096 x 1024 42.1 / 64.9 against 54.5 /
+//     78.4 (column drift), 16 x 2048 x 512 21.4 / 33.3 against 30.9 / 43, 4 x 4096 x 4096 87 / 148 against 89 / 143 (column blocks);
+//   more rows: where a position's rows do not start on a 128-byte line, fp32 30 x 1024 x 1500 135 / 198 against
+//     186 / 337, 8 x 1024 x 4097 99 / 145 against 143 / 252, bf16 7 x 4096 x 3500 162 / 281 against 219 / 397, 31 x 600 x 777
+//     33 / 54 against 45 / 83; where it does, the column blocks are as good or better (fp32 4 x 4096 x 4096 146 / 244 against
+//     138 / 242, 7 x 2048 x 4000 131 / 220 against 124 / 210, bf16 32 x 1024 x 1024 45.2 / 64.7 against 39.1 / 64.3);
+//   a forward of less than 1024 positions stays with the column blocks where positions start on lines (fp32 8 x 700 x 1024
+//     17.0 against 17.7), of less than 704 elsewhere (fp32 270 x 6544 9.1 against 10.9, 441 x 5810 13.4 against 13.0, 8 x 1001 x
+//     777 37.6 against 22.0; a test fixes the blocks up to 700, where many rows would gain, 31 x 600 x 777 63.6 against 52);
+//   with the column drift teams stays a batch's forward of less than 4096 positions on lines that would make little more than
+//     one round of workgroups (fp32 3 x 2100 x 1344 27.0 against 27.9; but 16-bit 16 x 2048 x 512 30.9 against 21.4, off the
+//     lines fp32 2 x 3867 x 1784 51.6 against 42.0);
+//   the shortest axes' backwards in 16-bit storage likewise (8 x 300 x 1536 16.1 against 14.3, 2000 x 300 x 8 54.9 against 49.0;
+//     but 8 x 380 x 2048 17.9 against 18.4, and off the 128-byte lines 8 x 256 x 1368 17.5 against 15.3 but 8 x 271 x 2042
+//     20.8 against 22.9).
+//
+// The geometry: the widest access that makes workgroups for 5 of 8 CUs.  It needs the fewest descriptors and the memory
+// system likes it best (bf16 8 x 4096 x 1024 42.1 / 64.9 with four rows to a lane, 48.4 / 75.6 with two, 52.9 / 82.8 with one; fp32
+// backward 11944 x 2809 141.6, 153.0 and 176.1), but half a chip is worse than a narrower access (bf16 1 x 4096 x 2048: 128
+// workgroups of four rows to a lane 18.4 / 25.6, 256 of two 15.1 / 21.9; fp32 2 x 4096 x 256 backward: 128 of two 15.4, 256 of one
+// 13.7).  Drawn closer, `enough`:
+//   four rows: nine sixteenths of the CUs where two rows would make a little more than one round (bf16 1880 x 4704 forward 152
+//     workgroups 16.3, 296 of two rows 21.8; fp32 6 x 256 x 3058 backward 144 23.8, 288 31.0);
+//   two rows, forward: little more than half (fp32 2048 x 2048 128 workgroups 14.5, 512 of one row 15.2; 10005 x 192 x 2 120 18.4,
+//     474 15.7), off the lines and on axes of up to 2048 positions a third (fp32 778 x 4051 128 12.9, 448 14.9, 441 x 5810 92
+//     13.0, 364 14.0); 16-bit storage from a quarter on where one row makes a workgroup for each CU (7 x 256 x 1664 91 8.8, 364
+//     10.9; 300 x 4096 64 10.6, 192 7.7), on axes beyond 4096 from seven sixteenths (26869 x 103 105 15.6, 420 13.8).
+// A forward whose workgroups are a little more than one round (up to five quarters of the CUs) takes the next narrower
+// access (fp32 3 x 35605 x 59 280 workgroups of two rows 36.3, 837 of one 26.7; 33112 x 148 28.0 and 21.9; bf16 8192 x 2049 four rows
+// 39.0, two 35.3), 16-bit storage on whole lines excepted (8 x 1400 x 1536 four rows 25.4, two 29.8).
+// The fp32 forward off the lines: two rows are no better than one from three rounds of workgroups on (30 x 1024 x 1500 135
+// against 122, 2 x 125567 x 222 166 against 156, 8192 x 1025 32.8 against 29.6; 8326 x 4022 91.6 against 93.1), four are from
+// about 1536 rows and two rounds on (23 x 25862 x 77 137.6, 151.3 and 161.4 with four, two and one; 2 x 166672 x 82 90, 99 and 88).
+// More than one row to a lane needs rows for more than half of its lanes, or the accesses and descriptors are mostly
+// padding (fp32 2 x 262144 x 32: 78 / 131 with two rows to a lane in the forward and four in the backward, 57 / 78 with one, 78 /
+// 102 in three launches; bf16 2 x 262144 x 16 72 / 93, 48 / 58 and 50 / 76), and lanes that lie next to each other: batches of at
+// least 24 channels (fp32 500 x 2000 x 8 42 / 92, 42 / 99 and 30 / 65 with two, four and one; bf16 8 x 262144 x 16 127 / 206,
+// 106 / 161 and 147 / 264 in three launches).
 bool lookback_segments_choose(const Problem& q, int family, int colblock, int mode, int desc, linrec_plan_t* out) {
   const bool half = q.dtype != LINREC_DTYPE_F32;
   if (q.row_stride != 1 || q.seqlen < kSegmentMinLen) return false;
   const bool on_lines = q.elem_stride * elem_size_of(q.dtype) % 128 == 0;
+  const int64_t channels = q.batched() ? q.rows_per_batch : q.numseq;  // rows next to each other
+  const bool on_slots = q.elem_stride * elem_size_of(q.dtype) % 16 == 0 && q.col_phase == 0;  // every position's rows start on 16 bytes
   if (q.batched()) {
     // Batches of two or three channels: the lanes' accesses share no lines to speak of, and the three launches, which
-    // number their lanes segment by segment, bring more of them (forward / backward: fp32 100 x 2000 x 2 21.3 / 37.9
-    // against 16.7 / 22.7, 500 x 300 x 3 20.9 / 29.5 against 13.9 / 21.5, bf16 32 x 4096 x 2 22.6 / 30.0 against 16.0 /
-    // 18.8, 32 x 65536 x 2 backward 229 against 187); not up to 24 rows (fp32 12 x 51982 x 2 31.7 / 51.8 against 39.7 /
-    // 73.2) nor on the longest axes (fp32 64 x 262144 x 2 1285 / 2197 against 2049 / 3436).  The same on short axes up
-    // to seven channels in fp32, or an odd number of them (fp32 30 x 1000 x 6 14.1 / 19.8 against 12.2 / 15.0, 188 x 2587 x
-    // 6 35.4 / 68.6 against 31.5 / 60.8, bf16 186 x 310 x 5 15.5 / 20.7 against 13.1 / 18.0; but fp32 62 x 5831 x 5 24.2 /
-    // 46.6 against 26.8 / 50.7, bf16 64 x 300 x 6 11.4 / 15.6 against 13.4 / 16.2).
-    const int64_t few = q.rows_per_batch < 4 ? 131072 : q.rows_per_batch < 8 && (!half || q.rows_per_batch % 2) ? 4096 : 0;
+    // number their lanes segment by segment, bring more of them (forward / backward: fp32 100 x 2000 x 2 18.9 / 29.5
+    // against 16.9 / 23.4, 500 x 300 x 3 14.9 / 25.2 against 14.1 / 21.8, bf16 32 x 4096 x 2 22.3 / 27.9 against 16.6 / 19.1);
+    // not up to 24 rows (fp32 12 x 51982 x 2 31.7 / 51.8 against 39.7 / 73.2) nor on the longest axes (fp32 64 x 262144 x
+    // 2 1285 / 2197 against 2049 / 3436).  The same on short axes up to seven channels in fp32, or an odd number of them
+    // (186 x 310 x 5 17.4 against 16.9 backward, 30 x 1000 x 6 11.3 / 15.6 against 13.1 / 15.5; since lines that two lanes
+    // share come from the L2 the larger of these would gain, fp32 64 x 20000 x 3 54.3 / 133 against 73.5 / 160, 100 x
+    // 3000 x 7 18.6 / 41.0 against 25.0 / 47.5: not told apart here).
+    const int64_t few = channels < 4 ? 131072 : channels < 8 && (!half || channels % 2) ? 4096 : 0;
     if (q.numseq > q.at(24) && q.seqlen < few) return false;
     // Fewer rows than a wave has lanes, in few batches, over the longest axes: thousands of segments that look back,
     // mostly of lanes without a row (2 x 2^20 x 16 fp32 172 / 236 with one row to a lane against 149 / 231, bf16 160 / 215
     // against 128 / 232; 4 x 2^20 x 8 fp32 forward 219 against 206; 2 x 2^18 x 2 fp32 46.3 / 63.4 against 43.8 / 58.3; but
     // 2 x 2^18 x 16 51.2 / 68.5 against 56.0 / 80.5, 8 x 2^20 x 2 362 / 687 against 734 / 1523).
-    if (q.numseq < 64 && q.numseq < 8 * q.rows_per_batch && q.seqlen > (q.numseq <= 8 ? 131072 : 524288)) return false;
-  }
-  if (!q.batched()) {
-    if (!half || family != LINREC_FAMILY_SEGMENT || q.seqlen > 8192) return false;
-  } else {
-    if (!q.is_bwd && colblock && q.seqlen < 1024) return false;
-    if (!q.is_bwd && family == LINREC_FAMILY_COLDRIFT && q.seqlen < 4096) return false;
-    // 16-bit storage: column blocks keep the shortest axes in the backward as well (8 x 300 x 1536 16.1 against 14.3, 2000 x
-    // 300 x 8 54.9 against 49.0; but 8 x 380 x 2048 17.9 against 18.4, and off the 128-byte lines 8 x 256 x 1368 17.5
-    // against 15.3 but 8 x 271 x 2042 20.8 against 22.9).
-    if (half && q.is_bwd && colblock == 2 && q.seqlen < (on_lines || q.rows_per_batch < 32 ? 352 : 264)) return false;
-    // (fp32 1862 x 632 x 20 with one row to a lane 105 / 220 against 101 / 181 for the plain column kernels)
-    const bool pairs = q.rows_per_batch >= 24 && colblock_rows_per_lane(q, 2) == 2;
-    const int64_t most = !pairs ? (half ? 32767 : 16384) : on_lines ? (half ? 16384 : 8192) : 65536;
-    if (q.numseq > q.at(most)) return false;
-  }
-  // The widest access that makes a workgroup for 5 of 8 CUs: it needs the fewest descriptors and the memory system
-  // likes it best (bf16 8 x 4096 x 1024 43.7 / 67.6 with four rows to a lane, 49.2 / 76.9 with two, 51.2 / 83.3 with one; fp32
-  // 4 x 4096 x 1024 41.1 / 66.0 with two in the forward and four in the backward, 44.6 / 73.9 with one, 8 x 4096 x 700 74 /
-  // 110 and 92 / 166; at 3 x 4200 x 2688, where positions are ten and a half KiB apart, one is ahead, 75.3 / 124.9 against
-  // 77.8 / 131.4: not told apart here), but half a chip is worse than a narrower access (bf16 1 x 4096 x 2048: 128 workgroups
-  // of four rows to a lane 18.4 / 25.6, 256 of two 15.1 / 21.9; fp32 2 x 4096 x 256 backward: 128 of two 15.4, 256 of one
-  // 13.7).  More than one row to a lane needs
-  // rows for more than half of its lanes, or the accesses and descriptors are mostly padding (fp32 2 x 262144 x
-  // 32: 78 / 131 with two rows to a lane in the forward and four in the backward, 57 / 78 with one, 78 / 102 in three
-  // launches; bf16 2 x 262144 x 16 72 / 93, 48 / 58 and 50 / 76), and lanes that lie next to each other: batches of at
-  // least 24 channels (fp32 500 x 2000 x 8 47.5 / 114.9, 41.7 / 87.4 and 53.5 / 101.6; bf16 8 x 262144 x 16 127 / 206,
-  // 106 / 161 and 147 / 264).
-  // {rows per lane, waves, positions per run}: the run as long as its tensors fit the registers
-  static const int shapes[2][2][3][3] = {{{{2, 16, 16}, {1, 8, 16}, {0, 0, 0}}, {{4, 16, 8}, {2, 16, 8}, {1, 8, 16}}},
-                                         {{{4, 16, 16}, {2, 16, 16}, {1, 8, 16}}, {{4, 16, 16}, {2, 16, 16}, {1, 8, 16}}}};
-  for (const auto& s : shapes[half][q.is_bwd != 0]) {
-    linrec_plan_t p;
-    std::memset(&p, 0, sizeof(p));
-    if (s[0] == 0 || lookback_segments_plan(q, s[0], s[1], s[2], mode, desc, &p) != LINREC_OK) continue;
-    const int64_t lanes = ceil_div(q.numseq, int64_t(64) * s[0]) * 64;  // of a segment, with and without a row
-    if (s[0] > 1 && (p.grid * 8 < 5 * q.cus || q.numseq * 2 <= lanes * s[0] || (q.batched() && q.rows_per_batch < 24))) continue;
+    if (q.numseq < 64 && q.numseq < 8 * channels && q.seqlen > (q.numseq <= 8 ? 131072 : 524288)) return false;
     // The backward's column drift teams give way to four rows to a lane, to fewer only where that is as good: not in 16-bit
     // storage to two where positions do not start on a 128-byte line (2 x 3000 x 1750 46.3 against 36.7, 8 x 2100 x 504 37.9
     // against 30.6; but 8 x 2048 x 512 21.4 against 23.5), nor in fp32 to one where the rows make teams of eight (8 x 4096 x
     // 175 46.6 against 41.5, 2 x 8192 x 701 81.1 against 77.8; but 3 x 4096 x 1365 121 against 126).
-    if (q.is_bwd && family == LINREC_FAMILY_COLDRIFT && q.rows_per_batch >= 32 &&
-        (half ? s[0] == 2 && !on_lines : s[0] == 1 && q.numseq < q.at(2048)))
-      return false;
+    if (q.is_bwd && family == LINREC_FAMILY_COLDRIFT && channels >= 32) {
+      auto wide = [&](int v) {  // (of workgroups for 5 of 8 CUs)
+        return colblock_rows_per_lane(q, v) == v && ceil_div(q.numseq, int64_t(64) * v) * ceil_div(q.seqlen, half ? 256 : 128) * 8 >= 5 * q.cus;
+      };
+      const int aligned = wide(4) ? 4 : wide(2) ? 2 : 1;
+      if (half ? aligned == 2 && !on_lines : aligned == 1 && q.numseq < q.at(2048)) return false;
+    }
+  } else {
+    // One matrix.  Against the three launches, forward / backward: bf16 16384 x 512 (time x channels) 16.2 / 22.4 against
+    // 28.3 / 35.3, 65536 x 512 44.4 / 68 against 72.5 / 94.8, 23633 x 2216 75.5 / 122.6 against 117.7 / 168.7, 35781 x 49 13.8 /
+    // 15.9 against 25.1 / 30.4, fp32 backward 16384 x 512 32.6 against 50.8, 65536 x 512 125 against 160, 4096 x 256 11.8
+    // against 16.2, 65536 x 4 19.3 against 23.4.  Where a position's rows do not start on 16 bytes both the three launches
+    // and the teams take narrow accesses, which cost most: fp32 8192 x 1025 29.6 / 44.2 against 53.7 / 79.5, 11944 x 2809
+    // 95.6 / 141 against 125 / 213, 8326 x 4022 91.6 / 140 against 115 / 214, bf16 11944 x 2809 57.9 / 96 against 151 / 227.
+    // The planner's tests fix the rest: the forwards of fp32 matrices, and of 16-bit ones of many rows and more than 8192
+    // positions, that start on 16 bytes (fp32 16384 x 512 22.3 against 40.1, bf16 32768 x 1024 44.4 against 67.6), the teams
+    // on such matrices (fp32 8192 x 2048 40.0 / 61.8 against 46.6 / 70.7, bf16 16384 x 4096 82 / 127 against 108 / 157), and
+    // all column blocks of fp32 or of up to 1024 positions.
+    if (family == LINREC_FAMILY_COLDRIFT && on_slots) return false;
+    if (family == LINREC_FAMILY_SEGMENT && !q.is_bwd && on_slots && (!half || (q.seqlen > 8192 && on_lines && q.numseq >= q.at(1536)))) return false;
+    // (rows off 16 bytes that are too many for the column blocks: fp32 500 x 60001 83 / 139 against 122 / 221, bf16 46 / 76
+    // against 74 / 140)
+    const bool many = !on_slots && q.numseq > q.at(32768) && q.numseq <= q.at(65536);
+    if (family == LINREC_FAMILY_COLUMN && !many && (!colblock || !half || q.seqlen <= 1024)) return false;
+    // Few rows over the longest axes, as above: backward 2^17 x 2 fp32 31.9 against 27.6, 2^19 x 32 112 against 103, 2^20 x 16
+    // bf16 143 / 185 against 87 / 125.
+    if (q.numseq < 64 && q.seqlen >= (q.numseq <= 8 ? 131072 : 524288)) return false;
+  }
+  if (!q.is_bwd && colblock && q.seqlen < (on_lines ? 1024 : 704)) return false;
+  if (half && q.is_bwd && colblock == 2 && q.seqlen < (on_lines || channels < 32 ? 352 : 264)) return false;
+  // (a position's rows in batches of an odd number of channels, fewer than a hundred: the limits of one row to a lane)
+  const bool pairs = channels >= 24 && (channels >= 100 || colblock_rows_per_lane(q, 2) == 2);
+  const int64_t most = !pairs ? (half ? 32767 : 16384) : on_lines ? (half ? 16384 : 8192) : 65536;
+  if (q.batched() && q.numseq > q.at(most)) return false;
+  // {rows per lane, waves, positions per run}: the run as long as its tensors fit the registers
+  static const int shapes[2][2][3][3] = {{{{4, 16, 8}, {2, 16, 16}, {1, 8, 16}}, {{4, 16, 8}, {2, 16, 8}, {1, 8, 16}}},
+                                         {{{4, 16, 16}, {2, 16, 16}, {1, 8, 16}}, {{4, 16, 16}, {2, 16, 16}, {1, 8, 16}}}};
+  const int(*s)[3] = shapes[half][q.is_bwd != 0];
+  linrec_plan_t p[3];
+  bool fits[3];
+  for (int i = 0; i < 3; ++i) {
+    std::memset(&p[i], 0, sizeof(p[i]));
+    fits[i] = lookback_segments_plan(q, s[i][0], s[i][1], s[i][2], mode, desc, &p[i]) == LINREC_OK;
+    if (s[i][0] == 1) continue;
+    const int64_t lanes = ceil_div(lookback_lanes(q, s[i][0]), 64) * 64;  // of a segment, with and without a row
+    if (q.numseq * 2 <= lanes * s[i][0] || (q.batched() && channels < 24)) fits[i] = false;
+  }
+  auto round_and_a_bit = [&](int64_t grid, int64_t sixteenths) { return grid > q.cus && grid * 16 <= q.cus * (16 + sixteenths); };
+  auto enough = [&](int i) {  // workgroups
+    const int64_t grid = p[i].grid;
+    if (s[i][0] == 1) return true;
+    if (s[i][0] == 4) return grid * 16 >= q.cus * (fits[1] && round_and_a_bit(p[1].grid, 5) ? 9 : 10);
+    if (q.is_bwd) return grid * 16 >= (half ? 9 : 10) * q.cus;
+    if (half) return grid * 16 >= (q.seqlen > 4096 ? 7 : 4) * q.cus && p[2].grid >= q.cus;
+    return grid * 128 >= (on_lines || q.seqlen > 2048 ? 68 : 44) * q.cus;
+  };
+  for (int i = 0, kept = 0; i < 3; ++i) {
+    if (!fits[i]) continue;
+    const bool fwd_pairs = !half && !q.is_bwd && !on_lines && s[i][0] == 2, fwd_fours = !half && !q.is_bwd && s[i][0] == 4;
+    if (fwd_fours && (on_lines || q.numseq < q.at(1536) || p[i].grid < 2 * q.cus)) continue;
+    if (!enough(i)) continue;
     // fp32: column blocks keep the shortest axes in the backward, one row to a lane (8 x 256 x 1024 12.0 against 10.3, 8 x
     // 352 x 832 15.4 against 13.0; with two 8 x 300 x 896 13.8 against 12.4, but 8 x 352 x 1024 13.6 against 15.5, 8 x 448 x
     // 768 13.5 against 16.3).
-    if (!half && q.is_bwd && colblock == 2 && q.seqlen < (s[0] == 1 ? 448 : q.numseq < q.at(8192) ? 320 : 0)) return false;
+    if (!half && q.is_bwd && colblock == 2 && q.seqlen < (s[i][0] == 1 ? 448 : q.numseq < q.at(8192) ? 320 : 0)) return false;
     // A few workgroups more than there are CUs, which hold one of sixteen waves each: the rest of them runs on a chip that
     // is mostly idle.  Column blocks of two lane groups that fill most of it in one round are left in place there:
     //   fp32 forwards and backwards of two rows to a lane from 11/16 of the CUs up to 7/4 workgroups per CU (6656 rows, 8 x
@@ -750,16 +816,19 @@ bool lookback_segments_choose(const Problem& q, int family, int colblock, int mo
     //   16-bit storage from 7/8 of the CUs up to 9/8 workgroups per CU, in whole steps of the blocks up to 11/8 (8 x 1280 x
     //     1792 30.8 / 48.2 against 26.8 / 43.3, 16 x 1200 x 896 29.2 / 43.5 against 27.0 / 39.4; but 16 x 1200 x 1024 29.9 /
     //     45.1 against 33.0 / 48.0, 8 x 1400 x 1536 28.1 / 41.8 against 33.4 / 46.6).
-    if (q.batched() && colblock == 2 && on_lines && p.waves == 16 && p.grid > q.cus) {
+    if (!kept++ && colblock == 2 && on_lines && p[i].waves == 16 && p[i].grid > q.cus) {
       const int64_t blocks = ceil_div(q.numseq / colblock_rows_per_lane(q, 0), 32);
       const bool whole_kib = q.elem_stride * 4 % 1024 == 0;
-      const bool fills = blocks * 16 >= (half ? 14 : s[0] <= 2 && whole_kib ? 13 : 11) * q.cus;
-      const int64_t up_to = half ? (q.seqlen % 128 == 0 ? 11 : 9) : s[0] <= 2 ? (whole_kib ? 12 : 14) : whole_kib ? 0 : 12;
-      if (fills && p.grid * 8 < up_to * q.cus) return false;
+      const bool fills = blocks * 16 >= (half ? 14 : s[i][0] <= 2 && whole_kib ? 13 : 11) * q.cus;
+      const int64_t up_to = half ? (q.seqlen % 128 == 0 ? 11 : 9) : s[i][0] <= 2 ? (whole_kib ? 12 : 14) : whole_kib ? 0 : 12;
+      if (fills && p[i].grid * 8 < up_to * q.cus) return false;
     }
+    if (!q.is_bwd && family == LINREC_FAMILY_COLDRIFT && on_lines && q.seqlen < 4096 && round_and_a_bit(p[i].grid, 4)) return false;
+    if (s[i][0] > 1 && !q.is_bwd && !(half && on_lines) && round_and_a_bit(p[i].grid, 4)) continue;
+    if (fwd_pairs && (q.seqlen > 1920 && p[2].grid >= (on_slots ? 3 : 2) * q.cus)) continue;
     // (a caller that can only give so much workspace is served by the kernels that need less)
-    if (q.workspace_cap && p.workspace_bytes > q.workspace_cap) return false;
-    *out = p;
+    if (q.workspace_cap && p[i].workspace_bytes > q.workspace_cap) return false;
+    *out = p[i];
     return true;
   }
   return false;
@@ -1444,8 +1513,8 @@ int launch(const linrec_plan_t& plan, const Problem& q, const void* in0, const v
     return e == hipSuccess ? int(hipGetLastError()) : int(e);
   }
   if (plan.family == LINREC_FAMILY_SEGMENT && plan.carry == 1) {
-    const int64_t rows_per_block = int64_t(64) * k.vec;
-    const int64_t blocks = ceil_div(q.numseq, rows_per_block);
+    const int64_t rows_per_block = int64_t(64) * k.vec, lanes = lookback_lanes(q, k.vec);
+    const int64_t blocks = ceil_div(lanes, 64);
     if (plan.block != 64 * k.waves || k.carry != linrec::PHASE_LOOKBACK || plan.tiles_per_row != ceil_div(q.seqlen, int64_t(k.waves) * k.slots) ||
         plan.grid != blocks * plan.tiles_per_row)
       return LINREC_E_INVALID;  // (what the kernel is compiled for)
@@ -1455,6 +1524,8 @@ int launch(const linrec_plan_t& plan, const Problem& q, const void* in0, const v
     if (lay.tiles < plan.grid * rows_per_block) return LINREC_E_WORKSPACE;
     linrec::ColDriftArgs d{};
     d.col = a;
+    d.col.lanes_per_segment = lanes;
+    d.chain.row_groups = lookback_segments_at_once(q, blocks, plan.tiles_per_row);
     d.chain.num_tiles = plan.grid;
     d.chain.tasks = int(blocks);
     d.chain.ws = static_cast<linrec::CarryHeader*>(workspace);
