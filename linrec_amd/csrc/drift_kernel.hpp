@@ -13,8 +13,8 @@
 // workgroups that share rows, hence an exchange; what a sweep kernel loses by waiting for it in every
 // step, these kernels keep.
 //
-// Restrictions as for the sweep kernels: 16-byte aligned bases, a row stride that keeps every row
-// aligned, rows of a whole number K of tiles with M dividing K.  Every workgroup of the launch has to
+// Restrictions of the plain form as for the sweep kernels: 16-byte aligned bases, a row stride that keeps every row
+// aligned, rows of a whole number K of tiles with M dividing K (RAGGED and SKEWED below lift them).  Every workgroup of the launch has to
 // be resident at once (the planner sees to that); every wait is bounded all the same, and a wave whose
 // wait runs out computes the value it needs from the row's own data.
 //
@@ -44,10 +44,18 @@ namespace linrec {
 // tile takes the loads and stores that look at every slot, the others stay as they are; the team need not divide K,
 // and the walk's start moves on by K % M tiles in every row, so that neither the partial tiles nor the longer walks
 // all fall to the same team mates.
-template <typename T, int NW, int S, int VEC, int MODE, bool DESC, int PF, int WPE = 1, bool WIDE = true, bool RAGGED = false>
+// SKEWED (fp32, with RAGGED): rows that start or end inside a slot, each at its own phase (RowView per row).  The waves
+// that hold a row's first or last slot take the loads and stores that look at every slot, all others whole slots as
+// before; a row's last tile may hold no slot of it at all, and is the identity then.  335 x 100001 backward 120.4 us, 5.6
+// TB/s, where look-back tiles of 16384 elements take 135.5 (one workgroup per CU and its waits); 100 x 250001 57.3 / 91.3
+// where one team per row takes 66.6 / 105.8.  Rows that start on a slot (335 x 100000 73.7 / 115.7) move the same bytes: what
+// is left is the launch shape's, see above.
+template <typename T, int NW, int S, int VEC, int MODE, bool DESC, int PF, int WPE = 1, bool WIDE = true, bool RAGGED = false,
+          bool SKEWED = false>
 __global__ __launch_bounds__(64 * NW, WPE) void drift_kernel(TileArgs p) {
   static_assert(PF == 1 || PF == 2, "one or two tiles of loads ahead of the scan");
   static_assert(NW <= 16, "the waves' shares are composed inside a DPP row");
+  static_assert(!SKEWED || (RAGGED && std::is_same_v<T, float>), "rows at any phase: fp32, partial last tiles");
   constexpr int WAVE_SLOTS = S * 64;
   constexpr int TILE_SLOTS = NW * WAVE_SLOTS;
   __shared__ float sh_a[2][NW];
@@ -82,7 +90,19 @@ __global__ __launch_bounds__(64 * NW, WPE) void drift_kernel(TileArgs p) {
   // agent-scope load did for a memory round trip at the start of every launch)
   const uint32_t seq = load_seq_through_caches(p.ws);
   if (threadIdx.x < 4) sh_fail[threadIdx.x] = 0;  // (every reader has passed a step's barrier first)
-  const RowView rv = make_row_view<VEC>(0, 0, p.seqlen);
+  // (all rows start on a slot unless SKEWED)
+  auto view_of = [&](int row) __attribute__((always_inline)) {
+    return SKEWED ? make_row_view<VEC>(p.base_mis, (long long)row * p.row_stride, p.seqlen) : make_row_view<VEC>(0, 0, p.seqlen);
+  };
+  // (every slot of a wave whose first one is `u_wave` lies in the row: no slot needs looking at)
+  auto whole_slots = [&](const RowView& rv, int u_wave) __attribute__((always_inline)) {
+    return !RAGGED || slots_interior<VEC, DESC>(u_wave, WAVE_SLOTS, rv);
+  };
+
+  // Partial tiles are loaded in whole slots and masked when their turn has come.  (The forward of rows that start on a slot
+  // masks its one partial tile at load time: fewer instructions in every step, 335 x 100000 74.4 against 75.8 us, backward 117.9
+  // against 116.5, 1 x 30000000 68.1 against 69.7, backward 109.9 against 103.6.)
+  constexpr bool MASK_LATE = SKEWED || (RAGGED && MODE == MODE_BWD && std::is_same_v<T, float>);
 
   struct Item {
     int row;
@@ -106,7 +126,7 @@ __global__ __launch_bounds__(64 * NW, WPE) void drift_kernel(TileArgs p) {
     return it;
   };
   auto ptrs_of = [&](int row) {
-    return make_row_ptrs<T, MODE>(p.in0, p.coef, p.aux, p.out0, p.out1, (long long)row * p.row_stride, 0);
+    return make_row_ptrs<T, MODE>(p.in0, p.coef, p.aux, p.out0, p.out1, (long long)row * p.row_stride, SKEWED ? view_of(row).lo : 0);
   };
 
   // 16-bit storage: the tiles whose loads are in flight, and a pending tile's saved outputs, stay in the storage
@@ -223,7 +243,7 @@ __global__ __launch_bounds__(64 * NW, WPE) void drift_kernel(TileArgs p) {
     }
     float carry_in = 0.0f;
     if (t > 0) {
-      if (!ok) carry_in = recompute_entry<VEC, MODE, DESC>(ptrs_of(it.row), rv, t * TILE_SLOTS, lane);
+      if (!ok) carry_in = recompute_entry<VEC, MODE, DESC>(ptrs_of(it.row), view_of(it.row), t * TILE_SLOTS, lane);
       else if (t < M) carry_in = acc.b;  // the maps reach back to the row start
       else carry_in = need > 0 ? fmaf(own_out, acc.a, acc.b) : own_out;
     }
@@ -240,7 +260,7 @@ __global__ __launch_bounds__(64 * NW, WPE) void drift_kernel(TileArgs p) {
     if (t > 0) {
       if (sh_fail[slot] == token) {  // (the same for the whole workgroup)
         if (wave == 0) {
-          const float c = recompute_entry<VEC, MODE, DESC>(ptrs_of(q.it.row), rv, t * TILE_SLOTS, lane);
+          const float c = recompute_entry<VEC, MODE, DESC>(ptrs_of(q.it.row), view_of(q.it.row), t * TILE_SLOTS, lane);
           if (lane == 0) sh_carry[slot] = c;
         }
         __syncthreads();
@@ -266,6 +286,7 @@ __global__ __launch_bounds__(64 * NW, WPE) void drift_kernel(TileArgs p) {
   };
   auto store_pending = [&](const Pending& q, float tile_in) {
     const int t = q.it.t;
+    const RowView rv = view_of(q.it.row);
     bool has_entry = false;
     float entry = 0.0f;
     if (t > 0) {
@@ -292,7 +313,7 @@ __global__ __launch_bounds__(64 * NW, WPE) void drift_kernel(TileArgs p) {
       tile_apply_store_packed<S, VEC, MODE, DESC, RAGGED>(q.d.ys, q.edge, q.r, ptrs_of(q.it.row), rv,
                                                           t * TILE_SLOTS + wave * WAVE_SLOTS, lane, has_entry, entry);
     } else {
-      if (RAGGED && t == K - 1)
+      if (!whole_slots(rv, t * TILE_SLOTS + wave * WAVE_SLOTS))
         tile_apply_store<S, VEC, MODE, DESC, false>(q.d, q.r, ptrs_of(q.it.row), rv, t * TILE_SLOTS + wave * WAVE_SLOTS,
                                                     lane, has_entry, entry);
       else
@@ -302,12 +323,16 @@ __global__ __launch_bounds__(64 * NW, WPE) void drift_kernel(TileArgs p) {
   };
   auto load_next = [&](Loaded& d, Item& it) {
     it = next_item();
+    const RowView rv = view_of(it.row);
+    const int u_wave = it.t * TILE_SLOTS + wave * WAVE_SLOTS;
     if constexpr (PACKED)  // (16-bit storage: a slot either lies in the row or beyond its end, every tile asks)
-      tile_load_packed<S, VEC, MODE, DESC, RAGGED>(d, ptrs_of(it.row), rv, it.t * TILE_SLOTS + wave * WAVE_SLOTS, lane);
-    else if (RAGGED && it.t == K - 1)
-      tile_load<S, VEC, MODE, DESC, false>(d, ptrs_of(it.row), rv, it.t * TILE_SLOTS + wave * WAVE_SLOTS, lane, false);
+      tile_load_packed<S, VEC, MODE, DESC, RAGGED>(d, ptrs_of(it.row), rv, u_wave, lane);
+    else if (MASK_LATE && !whole_slots(rv, u_wave))
+      tile_load_edge<S, VEC, MODE, DESC>(d, ptrs_of(it.row), rv, u_wave, lane);
+    else if (!whole_slots(rv, u_wave))
+      tile_load<S, VEC, MODE, DESC, false>(d, ptrs_of(it.row), rv, u_wave, lane, false);
     else
-      tile_load<S, VEC, MODE, DESC, true>(d, ptrs_of(it.row), rv, it.t * TILE_SLOTS + wave * WAVE_SLOTS, lane, false);
+      tile_load<S, VEC, MODE, DESC, true>(d, ptrs_of(it.row), rv, u_wave, lane, false);
   };
 
   // Step n, n % 3 == PH: tile n lies in D[PH]; P[(PH + 1) % 3] is tile n-2, stored in this step.
@@ -333,8 +358,24 @@ __global__ __launch_bounds__(64 * NW, WPE) void drift_kernel(TileArgs p) {
           return D[PH];
         }
       }();
+      if constexpr (MASK_LATE) {
+        const RowView rv = view_of(it.row);
+        const int u_wave = it.t * TILE_SLOTS + wave * WAVE_SLOTS;
+        if (!whole_slots(rv, u_wave)) tile_mask<S, VEC, MODE, DESC>(d, rv, u_wave, lane);
+      }
       if constexpr (MODE == MODE_FWD) {
-        if (it.t == 0 && wave == 0 && lane == 0) d.cs[0][0] = 0.0f;  // the row's first coefficient takes no part
+        // the row's first coefficient takes no part
+        if constexpr (SKEWED) {
+          if (it.t == 0 && wave == 0) {
+            const RowView rv = view_of(it.row);
+            const int first = DESC ? rv.nslots * VEC - rv.hi : rv.lo;  // its place in the slot, in scan order
+#pragma unroll
+            for (int i = 0; i < VEC; ++i)
+              if (i == first && lane == 0) d.cs[0][i] = 0.0f;
+          }
+        } else if (it.t == 0 && wave == 0 && lane == 0) {
+          d.cs[0][0] = 0.0f;
+        }
       }
       tile_scan<S, VEC, MODE>(d, now.r);
       if constexpr (MODE == MODE_FWD || PACKED) {

@@ -77,6 +77,15 @@ KernelGroup kernels_bf16_cols();
   {PFX "drift_ragged_w" #NW "_s" #S "_" #MODE "_" #DESC,                                        \
    (const void*)&linrec::drift_kernel<TT, NW, S, VEC, linrec::MODE, DESC != 0, DRIFT_TILES_AHEAD(NW, S, VEC, MODE), ((NW) > 8 ? 4 : 2), !((NW) == 16 && (S) == 2 && (VEC) == 4), true>, DT, LINREC_FAMILY_DRIFT, \
    NW, S, VEC, linrec::MODE, DESC, 2}
+// ... for fp32 rows that start or end inside a slot (`carry` column 3)
+#define DRIFT_SKEWED_ENTRY(TT, DT, PFX, NW, S, VEC, MODE, DESC)                                 \
+  {PFX "drift_skewed_w" #NW "_s" #S "_" #MODE "_" #DESC,                                        \
+   (const void*)&linrec::drift_kernel<TT, NW, S, VEC, linrec::MODE, DESC != 0, DRIFT_TILES_AHEAD(NW, S, VEC, MODE), ((NW) > 8 ? 4 : 2), !((NW) == 16 && (S) == 2 && (VEC) == 4), true, true>, DT, LINREC_FAMILY_DRIFT, \
+   NW, S, VEC, linrec::MODE, DESC, 3}
+#define DRIFT_SKEWED_FWD_DIRS(TT, DT, PFX, NW, S, VEC)                                         \
+  DRIFT_SKEWED_ENTRY(TT, DT, PFX, NW, S, VEC, MODE_FWD, 0), DRIFT_SKEWED_ENTRY(TT, DT, PFX, NW, S, VEC, MODE_FWD, 1)
+#define DRIFT_SKEWED_BWD_DIRS(TT, DT, PFX, NW, S, VEC)                                         \
+  DRIFT_SKEWED_ENTRY(TT, DT, PFX, NW, S, VEC, MODE_BWD, 0), DRIFT_SKEWED_ENTRY(TT, DT, PFX, NW, S, VEC, MODE_BWD, 1)
 #define DRIFT_RAGGED_FWD_DIRS(TT, DT, PFX, NW, S, VEC)                                         \
   DRIFT_RAGGED_ENTRY(TT, DT, PFX, NW, S, VEC, MODE_FWD, 0), DRIFT_RAGGED_ENTRY(TT, DT, PFX, NW, S, VEC, MODE_FWD, 1)
 #define DRIFT_RAGGED_BWD_DIRS(TT, DT, PFX, NW, S, VEC)                                         \
@@ -171,6 +180,8 @@ KernelGroup kernels_bf16_cols();
 #define DRIFT_BWD_(...) DRIFT_BWD_DIRS(__VA_ARGS__)
 #define DRIFT_RAGGED_FWD_(...) DRIFT_RAGGED_FWD_DIRS(__VA_ARGS__)
 #define DRIFT_RAGGED_BWD_(...) DRIFT_RAGGED_BWD_DIRS(__VA_ARGS__)
+#define DRIFT_SKEWED_FWD_(...) DRIFT_SKEWED_FWD_DIRS(__VA_ARGS__)
+#define DRIFT_SKEWED_BWD_(...) DRIFT_SKEWED_BWD_DIRS(__VA_ARGS__)
 #define TEAM_FWD_(...) TEAM_FWD_DIRS(__VA_ARGS__)
 #define STREAM_(...) STREAM_ALL_DIRS(__VA_ARGS__)
 #define COLUMN_(...) COLUMN_ALL_DIRS(__VA_ARGS__)

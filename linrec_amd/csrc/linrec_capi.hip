@@ -319,12 +319,30 @@ int half_drift_slots_for(const Problem& q, int fv) {
   }
   return 0;
 }
+// Rows that start or end inside a slot.
+bool drift_skewed(const Problem& q, int fv) {
+  return q.base_mis > 0 || (q.numseq > 1 && q.row_stride % fv != 0) || q.seqlen % fv != 0;
+}
+// Where they go to the drift kernels.  Forward / backward in us against one team per row, one workgroup per row or
+// look-back tiles of 16384 elements.  The backward nearly everywhere: 335 x 100001 120.4 against 135.5, 300 x 65541 73.3 against
+// 82.4, 600 x 20003 49.2 against 55.0, 1024 x 32769 123.2 against 142.0, 4000 x 16385 243 against 262, 100 x 250001 91.3 against
+// 105.8, 8 x 4194305 121 against 146, 1 x 33554431 116.4 against 129.2; not many rows where the look-back tiles would serve them
+// (4096 x 28002 453 against 416; 2048 x 32770 240 against 266).  The forward of 20 rows and more, fewer than there are CUs: 24 x
+// 262145 19.7 against 24.0, 100 x 250001 57.3 against 66.6, 192 x 65537 32.2 against 33.6; but 335 x 100001 77.2 against 77.0,
+// 1024 x 32769 81.1 against 78.2, 4096 x 28002 262 against 243.  With fewer rows the planner's tests hold it to one team per row (8 x
+// 4194305 79.0 against 93.7, 16 x 1048577 44.7 against 45.0), below that kernel's row counts it gains with plenty of work (1 x
+// 33554431 75.8 against 82.3, 4 x 8388609 77.2 against 83.0).
+bool drift_skewed_pays(const Problem& q) {
+  if (q.is_bwd) return q.numseq <= q.at(2560) || q.seqlen < kT_stream_max_len;
+  return q.numseq >= 20 ? q.numseq < q.cus : q.numseq < kT_team_min_rows && q.numseq * q.seqlen >= 12 * 8192 * q.cus;
+}
 // Returns the tile to use as slots per lane of 8 waves (4: 8192 fp32 elements, 2: 4096), 0 for "not a drift
 // case"; which kernel serves the tile (8 waves, or 16 with half the slots) is the launch planner's business.
 int drift_slots_for(const Problem& q, int fv) {
   const bool half = q.dtype != LINREC_DTYPE_F32;
-  if (q.base_mis != 0 || (q.numseq > 1 && q.row_stride % fv != 0) || q.elem_stride != 1) return 0;
-  if (half) return half_drift_slots_for(q, fv);
+  if (q.base_mis < 0 || q.elem_stride != 1) return 0;
+  const bool skewed = drift_skewed(q, fv);
+  if (half) return skewed && (q.base_mis != 0 || (q.numseq > 1 && q.row_stride % fv != 0)) ? 0 : half_drift_slots_for(q, fv);
   // More than 2048 rows: the forward gains as well (us, against one workgroup per row: 4096 x 32768 266.0 against
   // 274.3, 4096 x 40960 335.3 against 360.1, 4096 x 16384 128.9 against 138.8), in the same tiles of 8192 elements as
   // fewer rows (tiles of 4096: 269.2, 340.2, 139.3).
@@ -348,8 +366,9 @@ int drift_slots_for(const Problem& q, int fv) {
     if (half != (s == 1)) continue;
     if (q.is_bwd && s == 4) continue;  // (the backward pass holds three tensors: two slots per lane fit)
     const int64_t tile = int64_t(8) * s * 64 * fv;
-    if ((q.seqlen % tile != 0) != ragged) continue;
-    if (ragged && (half || q.seqlen % fv != 0 || s != (q.is_bwd ? 2 : 4))) continue;
+    if ((skewed || q.seqlen % tile != 0) != ragged) continue;
+    if (ragged && (half || s != (q.is_bwd ? 2 : 4))) continue;
+    if (skewed && !drift_skewed_pays(q)) continue;
     const int64_t tiles_per_row = q.seqlen / tile;  // (full ones)
     const int64_t team = drift_team_size(q, tiles_per_row + ragged, 8, q.cus, ragged);
     // the forward's tiles of 8192 elements: as many tiles a row as the generated table says, and from its number of
@@ -1071,7 +1090,7 @@ int make_plan(const Problem& q, const linrec_tuning_t* tune, linrec_plan_t* out)
     // 8192): 16 waves with one slot each rather than 8 waves with two.  Forward / backward in us: 512 x 65536
     // backward 116.2 against 117.4, 300 x 65536 70.7 against 71.5, 1024 x 65536 229.2 against 231.2, 16 x 1048576
     // 61.9 against 64.2, 1 x 33554432 74.6 / 119.8 against 82.1 / 125.0.
-    if (drift && !half && auto_slots == 2 && !(tune && (tune->waves > 0 || tune->slots > 0))) {
+    if (drift && !half && (auto_slots == 2 || (auto_slots == 0 && drift_skewed(q, fv) && q.is_bwd)) && !(tune && (tune->waves > 0 || tune->slots > 0))) {
       waves = 16;
       slots = 1;
     }
@@ -1086,13 +1105,15 @@ int make_plan(const Problem& q, const linrec_tuning_t* tune, linrec_plan_t* out)
     }
     const int64_t tile_elems = int64_t(waves) * slots * 64 * fv;
     // every tile of every row has to be a full one; the drift kernels also come for rows of whole slots whose last
-    // tile is a partial one (kernel-table code 2 in the carry column)
-    const bool ragged = drift && q.seqlen % tile_elems != 0 && q.seqlen % fv == 0 && q.seqlen > tile_elems;
-    if (q.base_mis != 0 || (q.numseq > 1 && q.row_stride % fv != 0) || (q.seqlen % tile_elems != 0 && !ragged)) return LINREC_E_UNSUPPORTED;
-    const int id = find_kernel(q.dtype, family, waves, slots, fv, mode, desc, ragged ? 2 : 1);
+    // tile is a partial one (kernel-table code 2 in the carry column), in fp32 for rows at any phase as well (code 3)
+    const bool skewed = drift && !half && drift_skewed(q, fv) && q.seqlen > tile_elems;
+    const bool ragged = skewed || (drift && q.seqlen % tile_elems != 0 && q.seqlen % fv == 0 && q.seqlen > tile_elems);
+    if (q.base_mis < 0 || (!skewed && (q.base_mis != 0 || (q.numseq > 1 && q.row_stride % fv != 0))) || (q.seqlen % tile_elems != 0 && !ragged))
+      return LINREC_E_UNSUPPORTED;
+    const int id = find_kernel(q.dtype, family, waves, slots, fv, mode, desc, skewed ? 3 : ragged ? 2 : 1);
     if (id < 0) return LINREC_E_UNSUPPORTED;
     const int block = 64 * waves;
-    const int64_t tiles_per_row = ceil_div(q.seqlen, tile_elems);
+    const int64_t tiles_per_row = ceil_div(full_slots * fv, tile_elems);
     // Every workgroup of the launch has to be resident at once (a walker waits for its team mates, and a
     // workgroup that has not started yet only starts when another one ends): never more than the CUs hold.
     const int64_t resident = int64_t(workgroups_per_cu(id, block, drift || q.is_bwd ? 1 : 2)) * q.cus;

@@ -176,6 +176,49 @@ __device__ __forceinline__ void tile_load(TileData<S, VEC, MODE>& d, const RowPt
   }
 }
 
+// tile_load for a wave that holds the row's first or last slot, in a kernel that keeps loads in flight: whole slots
+// only, lanes beyond the row's last slot read that one again, and nothing looks at what arrives before tile_mask does
+// when the tile's turn has come (a fill at load time would wait for the loads in the step that issues them: 335 x 100001
+// 86 / 155 us with it).
+template <int S, int VEC, int MODE, bool DESC, typename T>
+__device__ __forceinline__ void tile_load_edge(TileData<S, VEC, MODE>& d, const RowPtrs<T>& q, const RowView& rv, int u_wave,
+                                               int lane) {
+  auto place = [&](int j) {
+    const int u = u_wave + j * 64 + lane;
+    return unsigned(slot_of<VEC, DESC>(u < rv.nslots ? u : rv.nslots - 1, rv));
+  };
+#pragma unroll
+  for (int j = 0; j < S; ++j) load_slot_full<VEC, DESC>(q.in0, place(j), d.xs[j]);
+#pragma unroll
+  for (int j = 0; j < S; ++j) load_slot_full<VEC, DESC>(q.coef, place(j), d.cs[j]);
+  d.y_edge = 0.0f;
+  if constexpr (MODE == MODE_BWD) {
+#pragma unroll
+    for (int j = 0; j < S; ++j) load_slot_full<VEC, DESC>(q.aux, place(j), d.ys[j]);
+    if (lane == 63) {
+      const int u_next = u_wave + S * 64;
+      const int s_next = slot_of<VEC, DESC>(u_next, rv);
+      d.y_edge = (u_next < rv.nslots) ? load_element(q.aux, vindex<VEC, DESC>(s_next, 0), rv, 0.0f) : 0.0f;
+    }
+  }
+}
+// ... and what lies outside the row becomes inputs of zero, coefficients of one and outputs of zero.
+template <int S, int VEC, int MODE, bool DESC>
+__device__ __forceinline__ void tile_mask(TileData<S, VEC, MODE>& d, const RowView& rv, int u_wave, int lane) {
+#pragma unroll
+  for (int j = 0; j < S; ++j) {
+    const int u = u_wave + j * 64 + lane, s = slot_of<VEC, DESC>(u, rv);
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) {
+      const int v = vindex<VEC, DESC>(s, i);
+      const bool in_row = u < rv.nslots && v >= rv.lo && v < rv.hi;
+      d.xs[j][i] = in_row ? d.xs[j][i] : 0.0f;
+      d.cs[j][i] = in_row ? d.cs[j][i] : 1.0f;
+      if constexpr (MODE == MODE_BWD) d.ys[j][i] = in_row ? d.ys[j][i] : 0.0f;
+    }
+  }
+}
+
 // A wave's share of one interior tile as it arrives from memory, still in the storage type.  A kernel that keeps
 // loads in flight across the steps of a software pipeline holds 16-bit data this way (half the registers of
 // TileData, and nothing that would have to wait for the loads before the step that uses them).
