@@ -1090,7 +1090,7 @@ int make_plan(const Problem& q, const linrec_tuning_t* tune, linrec_plan_t* out)
     // 8192): 16 waves with one slot each rather than 8 waves with two.  Forward / backward in us: 512 x 65536
     // backward 116.2 against 117.4, 300 x 65536 70.7 against 71.5, 1024 x 65536 229.2 against 231.2, 16 x 1048576
     // 61.9 against 64.2, 1 x 33554432 74.6 / 119.8 against 82.1 / 125.0.
-    if (drift && !half && (auto_slots == 2 || (auto_slots == 0 && drift_skewed(q, fv) && q.is_bwd)) && !(tune && (tune->waves > 0 || tune->slots > 0))) {
+    if (drift && !half && auto_slots == 2 && !(tune && (tune->waves > 0 || tune->slots > 0))) {
       waves = 16;
       slots = 1;
     }
@@ -1106,7 +1106,8 @@ int make_plan(const Problem& q, const linrec_tuning_t* tune, linrec_plan_t* out)
     const int64_t tile_elems = int64_t(waves) * slots * 64 * fv;
     // every tile of every row has to be a full one; the drift kernels also come for rows of whole slots whose last
     // tile is a partial one (kernel-table code 2 in the carry column), in fp32 for rows at any phase as well (code 3)
-    const bool skewed = drift && !half && drift_skewed(q, fv) && q.seqlen > tile_elems;
+    // (the planner's choice only: a caller who names the family gets rows of whole slots)
+    const bool skewed = drift && !half && !(tune && tune->family != LINREC_FAMILY_AUTO) && drift_skewed(q, fv) && q.seqlen > tile_elems;
     const bool ragged = skewed || (drift && q.seqlen % tile_elems != 0 && q.seqlen % fv == 0 && q.seqlen > tile_elems);
     if (q.base_mis < 0 || (!skewed && (q.base_mis != 0 || (q.numseq > 1 && q.row_stride % fv != 0))) || (q.seqlen % tile_elems != 0 && !ragged))
       return LINREC_E_UNSUPPORTED;
@@ -1231,8 +1232,10 @@ int make_plan(const Problem& q, const linrec_tuning_t* tune, linrec_plan_t* out)
     if (q.elem_stride == 1 && q.seqlen != 1) return LINREC_E_UNSUPPORTED;
     const bool given = tune && tune->family == LINREC_FAMILY_SEGMENT;
     // in one launch (tuning: `carry` = 1, `waves` = rows per lane, `slots` = positions per run, `tasks` = waves)
+    // (a caller who names the rows per lane gets rows that start on a whole access, as in every strided family)
     if (given && tune->carry == 1)
-      return lookback_segments_plan(q, tune->waves, tune->tasks, tune->slots, mode, desc, out);
+      return tune->waves >= 1 && colblock_rows_per_lane(q, tune->waves) == tune->waves
+                 ? lookback_segments_plan(q, tune->waves, tune->tasks, tune->slots, mode, desc, out) : LINREC_E_UNSUPPORTED;
     // rows per lane: 8 bytes' worth when that leaves at least a wave of lanes, fewer otherwise; fp32 from 512
     // rows on: four rows (16-byte accesses, a wave reads 1 KiB of every position), which the backward likes
     // (forward / backward in us, four rows against two at their best segment counts: 700 x 100000 278 / 409

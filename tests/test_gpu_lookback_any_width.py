@@ -10,29 +10,34 @@ from tests.test_gpu_lookback_segments import DTYPES, TOL, check_bwd, check_fwd, 
 from tests.util import check_close
 
 
+@pytest.fixture
+def compute_units(nat):  # noqa: F811
+    yield nat.set_compute_units
+    nat.set_compute_units(0)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("reverse", [False, True])
 @pytest.mark.parametrize("kind", list(DTYPES))
-def test_several_rows_to_a_lane_at_any_alignment(nat, kind, reverse):  # noqa: F811
-    fwd = [(4, 16, 8), (2, 16, 16)] if kind == "f32" else [(4, 16, 16), (2, 16, 16)]
-    bwd = [(4, 16, 8), (2, 16, 8)] if kind == "f32" else fwd
-    for batch, time, channels in [(1, 300, 5), (1, 2049, 257), (1, 2100, 33), (3, 700, 129), (2, 2300, 66), (5, 257, 7), (1, 513, 1023)]:
+def test_several_rows_to_a_lane_at_any_alignment(nat, compute_units, kind, reverse):  # noqa: F811
+    """On fewer compute units than there are, so that small tensors get wide accesses: every width, both passes."""
+    seen = set()
+    for cus, batch, time, channels in [(2, 3, 1100, 129), (3, 2, 2300, 66), (16, 1, 2100, 203), (16, 1, 5000, 131), (8, 1, 1500, 101),
+                                       (9, 2, 2100, 257), (16, 2, 3000, 203), (20, 1, 2100, 257), (40, 3, 1100, 205)]:
+        compute_units(cus)
         for start in (0, 1):  # the bases on 16 bytes, and one element after
             wide = draw((batch, time, channels + start), DTYPES[kind], channels + start, near1=time > 1000)
             x, c, dy = (t[:, :, start:].transpose(1, 2) for t in wide)
-            y = None
-            for is_bwd, geometries in ((False, fwd), (True, bwd)):
-                for vec, waves, run in geometries:
-                    tuning = nat.Tuning(nat.FAMILY_SEGMENT, vec, run, 1, waves)
-                    what = f"{kind} {(batch, time, channels, start)} rows/lane={vec} run={run} rev={reverse}"
-                    print(what, "backward" if is_bwd else "forward", flush=True)
-                    p = nat.plan(x, reverse, is_bwd, tuning)
-                    assert (p["carry"], p["vec"], p["tiles_per_row"]) == (1, vec, -(-time // (waves * run))), p
-                    assert p["grid"] == -(-(batch * -(-channels // vec)) // 64) * p["tiles_per_row"]
-                    if is_bwd:
-                        check_bwd(nat, kind, dy, c, y, reverse, tuning, what)
-                    else:
-                        y = check_fwd(nat, kind, x, c, reverse, tuning, what)
+            plans = [nat.plan(x, reverse, b) for b in (False, True)]
+            what = f"{kind} {cus} CUs {(batch, time, channels, start)} rows/lane={[p['vec'] for p in plans]} rev={reverse}"
+            print(what, flush=True)
+            for is_bwd, p in enumerate(plans):
+                assert (p["family"], p["carry"]) == (nat.FAMILY_SEGMENT, 1) and p["tiles_per_row"] == -(-time // p["tasks"]), (what, p)
+                assert p["grid"] == -(-(batch * -(-channels // p["vec"])) // 64) * p["tiles_per_row"], (what, p)
+                seen.add((is_bwd, p["vec"]))
+            y = check_fwd(nat, kind, x, c, reverse, None, what)
+            check_bwd(nat, kind, dy, c, y, reverse, None, what)
+    assert {(0, 4), (0, 2), (1, 4), (1, 2)} <= seen, seen
     assert nat.gave_up_count() == 0
 
 
