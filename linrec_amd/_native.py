@@ -553,7 +553,9 @@ def _few_rows_on_strided_axis(t, lay, tuning):
 # pointers (which must be 16-byte aligned, as the results then are), the stream and one library call that takes
 # its arguments in one block of memory.  On a 64 x 4096 tensor, whose kernel takes 3 us, this halves the time
 # the host needs per launch.  Batches of matrices ((batch, time, channels) data) are remembered likewise: working out
-# their layout and planning the workspace anew in every call cost as much as their kernels (8 x 4096 x 1024: 40 us a step).  Everything else takes the general path below.
+# their layout and planning the workspace anew in every call cost as much as their kernels (8 x 4096 x 1024: 40 us a step).
+# A scan axis other than the last is part of what is remembered, so a repeat makes no views of its tensors.  Everything else
+# takes the general path below.
 _repeat = threading.local()
 _REPEAT_MAX = 256
 
@@ -631,17 +633,33 @@ def _repeatable(t, *same):
     return None if _few_rows_on_strided_axis(t, lay, None) else lay
 
 
-def fwd(inputs, coeffs, reverse=False, tuning=None, out=None):
+def _last(dim, *tensors):
+    """Views with axis `dim` in the last place."""
+    return tensors if dim == -1 else tuple(t.transpose(dim, -1) for t in tensors)
+
+
+def _back(dim, *moved):
+    """Results with their last axis back in place `dim`: tensors of their own on the same memory, not views (autograd
+    has to be handed the result itself)."""
+    if dim == -1:
+        return moved
+    views = [m.transpose(dim, -1) for m in moved]
+    return tuple(torch.empty(0, dtype=m.dtype, device=m.device).set_(m.untyped_storage(), v.storage_offset(), v.size(), v.stride())
+                 for m, v in zip(moved, views))
+
+
+def fwd(inputs, coeffs, reverse=False, tuning=None, out=None, dim=-1):
     """outputs = linrec(inputs, coeffs) over the last dim (linrec/impl/cuda/linrec_pipe.cu:16-92).
-    `out`, if given, must have the layout the result would be allocated with."""
-    if tuning is None and inputs.is_cuda:
+    `out`, if given, must have the layout the result would be allocated with.  `dim`: another scan axis (without `out`)."""
+    if tuning is None and inputs.is_cuda and type(dim) is int:
         shape, stride = inputs.shape, inputs.stride()
-        key = (inputs.dtype, inputs.device, shape, stride, coeffs.dtype, coeffs.device, coeffs.shape, coeffs.stride(), reverse)
+        key = (inputs.dtype, inputs.device, shape, stride, coeffs.dtype, coeffs.device, coeffs.shape, coeffs.stride(), reverse, dim)
         table = _repeat_table()
         entry = table.get(key, False)
         if entry is False:
-            _validate(inputs, coeffs, names=("inputs", "coeffs"))
-            entry = _remember(table, key, _repeatable(inputs, coeffs), inputs, False, reverse)
+            x, c = _last(dim, inputs, coeffs)
+            _validate(x, c, names=("inputs", "coeffs"))
+            entry = _remember(table, key, _repeatable(x, c), x, False, reverse)
         if entry is not None:
             px, pc = inputs.data_ptr(), coeffs.data_ptr()
             if not (px | pc) & 15:
@@ -660,21 +678,23 @@ def fwd(inputs, coeffs, reverse=False, tuning=None, out=None):
                     call.in0, call.coef, call.out0 = px, pc, po
                     _repeat_launch(entry, lib().linrec_fwd_call, inputs, "linrec_fwd")
                     return res
-    return _fwd_general(inputs, coeffs, reverse, tuning, out)
+    x, c = _last(dim, inputs, coeffs)
+    return _back(dim, _fwd_general(x, c, reverse, tuning, out))[0]
 
 
-def bwd(d_outputs, coeffs, outputs, reverse=False, tuning=None, out=None):
+def bwd(d_outputs, coeffs, outputs, reverse=False, tuning=None, out=None, dim=-1):
     """(d_inputs, d_coeffs) (linrec/impl/cuda/linrec_pipe.cu:96-174).  The three tensors are brought
     to one memory layout first (the reference instead requires equal strides, linrec_pipe.cu:98)."""
-    if tuning is None and outputs.is_cuda:
+    if tuning is None and outputs.is_cuda and type(dim) is int:
         shape, stride = outputs.shape, outputs.stride()
         key = (outputs.dtype, outputs.device, shape, stride, coeffs.dtype, coeffs.device, coeffs.shape, coeffs.stride(),
-               d_outputs.dtype, d_outputs.device, d_outputs.shape, d_outputs.stride(), reverse, True)
+               d_outputs.dtype, d_outputs.device, d_outputs.shape, d_outputs.stride(), reverse, dim, True)
         table = _repeat_table()
         entry = table.get(key, False)
         if entry is False:
-            _validate(outputs, coeffs, d_outputs, names=("outputs", "coeffs", "d_outputs"))
-            entry = _remember(table, key, _repeatable(outputs, coeffs, d_outputs), outputs, True, reverse)
+            y, c, dy = _last(dim, outputs, coeffs, d_outputs)
+            _validate(y, c, dy, names=("outputs", "coeffs", "d_outputs"))
+            entry = _remember(table, key, _repeatable(y, c, dy), y, True, reverse)
         if entry is not None:
             pd, pc, py = d_outputs.data_ptr(), coeffs.data_ptr(), outputs.data_ptr()
             if not (pd | pc | py) & 15:
@@ -695,7 +715,8 @@ def bwd(d_outputs, coeffs, outputs, reverse=False, tuning=None, out=None):
                     call.in0, call.coef, call.aux, call.out0, call.out1 = pd, pc, py, p0, p1
                     _repeat_launch(entry, lib().linrec_bwd_call, outputs, "linrec_bwd")
                     return dx, dc
-    return _bwd_general(d_outputs, coeffs, outputs, reverse, tuning, out)
+    dy, c, y = _last(dim, d_outputs, coeffs, outputs)
+    return _back(dim, *_bwd_general(dy, c, y, reverse, tuning, out))
 
 
 def _fwd_general(inputs, coeffs, reverse=False, tuning=None, out=None):

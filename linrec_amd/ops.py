@@ -9,6 +9,7 @@ the op is chosen by the dispatcher from the tensors' device, never by a silent f
 from typing import Tuple
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _native
 
@@ -67,18 +68,11 @@ class _LinrecFn(torch.autograd.Function):
     Eager calls go through this class because the Python dispatch of a custom op costs several
     times the kernels' own launch time on small inputs; traced and compiled calls use the operator."""
 
+    # (The scan axis is moved in _native, out of autograd's sight: three views recorded by autograd, and their three
+    # counterparts in the backward, took 40 us of host time a step, as long as the kernels of 2^23 elements.)
     @staticmethod
     def forward(ctx, inputs, coeffs, reverse, dim):
-        if dim == -1:
-            outputs = _native.fwd(inputs, coeffs, reverse)
-        else:
-            # The scan axis is moved here, out of autograd's sight: three views recorded by autograd, and their three
-            # counterparts in the backward, took 40 us of host time a step, as long as the kernels of 2^23 elements.
-            moved = _native.fwd(inputs.transpose(dim, -1), coeffs.transpose(dim, -1), reverse)
-            view = moved.transpose(dim, -1)
-            # (the result itself, not a view of a tensor autograd has not seen)
-            outputs = torch.empty(0, dtype=moved.dtype, device=moved.device).set_(
-                moved.untyped_storage(), view.storage_offset(), view.size(), view.stride())
+        outputs = _native.fwd(inputs, coeffs, reverse, dim=dim)
         ctx.save_for_backward(coeffs, outputs)
         ctx.reverse, ctx.dim = reverse, dim
         return outputs
@@ -87,14 +81,16 @@ class _LinrecFn(torch.autograd.Function):
     @torch.autograd.function.once_differentiable
     def backward(ctx, d_outputs):
         coeffs, outputs = ctx.saved_tensors
-        dim = ctx.dim
-        if dim == -1:
-            d_inputs, d_coeffs = _native.bwd(d_outputs, coeffs, outputs, ctx.reverse)
-        else:
-            d_inputs, d_coeffs = _native.bwd(d_outputs.transpose(dim, -1), coeffs.transpose(dim, -1),
-                                             outputs.transpose(dim, -1), ctx.reverse)
-            d_inputs, d_coeffs = d_inputs.transpose(dim, -1), d_coeffs.transpose(dim, -1)
+        d_inputs, d_coeffs = _native.bwd(d_outputs, coeffs, outputs, ctx.reverse, dim=ctx.dim)
         return d_inputs, d_coeffs, None, None
+
+
+def _nobody_watches(inputs, coeffs):
+    """Nothing would look at an autograd Function around this call: no gradient to record, no forward-mode level open, no
+    function transform, no tracer."""
+    return (not (torch.is_grad_enabled() and (inputs.requires_grad or coeffs.requires_grad))
+            and forward_ad._current_level < 0 and not torch._C._are_functorch_transforms_active()
+            and torch._C._get_tracing_state() is None)
 
 
 def linrec(inputs: torch.Tensor, coeffs: torch.Tensor, reverse: bool = False, *, logc: bool = False,
@@ -119,10 +115,10 @@ def linrec(inputs: torch.Tensor, coeffs: torch.Tensor, reverse: bool = False, *,
         if last:
             return linrec_fwd(inputs, coeffs, reverse)
         return linrec_fwd(inputs.transpose(dim, -1), coeffs.transpose(dim, -1), reverse).transpose(dim, -1)
-    if last or (torch.is_grad_enabled() and (inputs.requires_grad or coeffs.requires_grad)):
-        return _LinrecFn.apply(inputs, coeffs, reverse, -1 if last else dim)
-    # (nothing to record: the views are cheaper here, bf16 1 x 4096 x 2048 forward 14.4 us against 16.2 inside)
-    return _LinrecFn.apply(inputs.transpose(dim, -1), coeffs.transpose(dim, -1), reverse, -1).transpose(dim, -1)
+    dim = -1 if last else dim
+    if _nobody_watches(inputs, coeffs):  # (inference: the Function's own bookkeeping is a quarter of a small call)
+        return _native.fwd(inputs, coeffs, reverse, dim=dim)
+    return _LinrecFn.apply(inputs, coeffs, reverse, dim)
 
 
 # The reference exports three variants of the same function (ops.py:60,81,101); here one set of
