@@ -117,7 +117,7 @@ typedef struct linrec_plan {
   int32_t carry;          /* 1 if tiles of a row are chained through the workspace; COLUMN: lane groups per wave
                              of the block form (1 or 2), 0 for the plain column kernels */
   int32_t tiles_per_row;  /* COLUMN block form: steps of the walk along the scan axis; SEGMENT: segments */
-  int32_t tasks;          /* tiles per workgroup (look-back kernels), else 1 */
+  int32_t tasks;          /* tiles per workgroup (look-back kernels), whole rows per workgroup (packed tiles), else 1 */
   int32_t tail_rows;      /* rows at the end of the tensor that a second launch, planned for them alone, serves
                              (0: one launch serves all rows) */
   int64_t grid;           /* workgroups */

@@ -2,6 +2,7 @@
 #include <hip/hip_runtime.h>
 
 #include "tile_kernel.hpp"
+#include "packed_kernel.hpp"
 #include "stream_kernel.hpp"
 #include "team_kernel.hpp"
 #include "sweep_kernel.hpp"

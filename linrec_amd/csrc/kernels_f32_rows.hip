@@ -3,6 +3,7 @@
 
 #include "tile_kernel.hpp"
 #include "chain_kernel.hpp"
+#include "packed_kernel.hpp"
 #include "kernel_table.hpp"
 
 LINREC_KERNEL_GROUP(kernels_f32_rows,
@@ -13,6 +14,8 @@ LINREC_KERNEL_GROUP(kernels_f32_rows,
     TILE_(F32, 2, 1, 4, 0), TILE_(F32, 2, 2, 4, 0), TILE_(F32, 2, 4, 4, 0), TILE_(F32, 4, 1, 4, 0),
     TILE_(F32, 4, 2, 4, 0), TILE_(F32, 16, 2, 4, 0), TILE_(F32, 4, 4, 4, 0), TILE_(F32, 4, 8, 4, 0),
     TILE_(F32, 8, 2, 4, 0), TILE_(F32, 8, 4, 4, 0), TILE_(F32, 16, 4, 4, 0),
+    // several rows to a workgroup
+    PACKED_(F32, 4, 2, 4), PACKED_(F32, 8, 2, 4), PACKED_(F32, 16, 2, 4),
     // rows chained over several workgroups by look-back
     TILE_(F32, 1, 4, 4, 1), TILE_(F32, 4, 2, 4, 1), TILE_(F32, 4, 4, 4, 1), TILE_(F32, 4, 8, 4, 1),
     TILE_(F32, 8, 4, 4, 1), TILE_(F32, 8, 8, 4, 1), TILE_(F32, 16, 4, 4, 1),

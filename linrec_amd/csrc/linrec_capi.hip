@@ -867,6 +867,75 @@ Problem tail_problem(const Problem& q, int64_t tail_rows) {
   return t;
 }
 
+// Several whole rows to a workgroup (packed_kernel.hpp) in the place of the flat kernels and of one row to a workgroup;
+// `row_slots`, `tile_slots`: what a row takes and what one row to a workgroup would have (0: the flat kernels' rows).
+//
+// From 2^22 elements on (on 256 CUs); with fewer, workgroups of four waves are too few (2^21, against the other kernels,
+// us: bf16 700 forward / backward 5.7 / 8.1 against 5.2 / 7.6; 2^22 7.1 / 10.0 against 7.8 / 11.6).  Geometric means of the
+// gain over 30 lengths, forward / backward in workgroups of 4, 8 and 16 waves: fp32 2^22 1.10 / 1.09, 1.04 / 1.06, 0.93 /
+// 0.99; 2^24 1.12 / 1.06, 1.10 / 1.05, 1.06 / 1.06; 2^25 1.09 / 1.02, 1.09 / 1.01, 1.07 / 1.04; bf16 2^22 1.17 / 1.17, 1.11 / 1.10, 0.94
+// / 0.72; 2^25 1.25 / 1.11, 1.23 / 1.13, 1.17 / 0.92.  So four waves, from 2^25 on eight, and sixteen for the fp32 backward;
+// more where that many hold less than two rows, or leave a fifth of the lanes idle (bf16 2^25 x 1401 backward 67.5 in
+// four waves, 64.6 in eight, 67.4 with one row to a workgroup; 3001 in eight 67.3 against 65.5).
+// Not rows that fill their own workgroup (fp32 2^25, 256 elements: 62.6 / 108.6 against 61.1 / 105.5), nor the backward of
+// large tensors where one slot to a lane does (1001: 117.9 against 112.9; bf16 2001: 62.9 against 61.1; at 2^23 1001 30.9
+// against 32.0), nor the large backward of a few floats (5: 116.1 against 113.8).
+bool packed_plan(const Problem& q, int fv, int mode, int desc, int64_t row_slots, int64_t tile_slots, linrec_plan_t* out) {
+  if (q.base_mis < 0 || q.elem_stride != 1 || q.numseq < 2 || q.row_stride != q.seqlen || q.batched() || q.seqlen < fv) return false;
+  const bool half = q.dtype != LINREC_DTYPE_F32;
+  const int64_t elements = q.numseq * q.seqlen;
+  if (elements < 16384 * q.cus) return false;
+  const bool ragged = q.base_mis > 0 || q.seqlen % fv != 0;  // workgroups start and end inside a slot
+  if (tile_slots > 0 && !ragged && row_slots == tile_slots) return false;
+  if (q.is_bwd && elements >= 65536 * q.cus && tile_slots > 64 && tile_slots <= 256 && row_slots * 100 >= tile_slots * 98) return false;
+  const bool large = elements >= 131072 * q.cus;
+  if (q.is_bwd && !half && large && q.seqlen < 16) return false;
+  for (int waves = !large || (half && !q.is_bwd) ? 4 : half || !q.is_bwd ? 8 : 16; waves <= (half || !q.is_bwd ? 8 : 16); waves *= 2) {
+    const int64_t room = int64_t(waves) * 2 * 64 * fv;
+    const int64_t rows = (room - (ragged ? fv - 1 : 0)) / q.seqlen;
+    if (rows < 2 || rows * q.seqlen * 5 < room * 4) continue;
+    const int id = find_kernel(q.dtype, LINREC_FAMILY_TILE, waves, 2, fv, mode, desc, 4);
+    if (id < 0 || ceil_div(q.numseq, rows) > 2147483647LL) return false;
+    out->family = LINREC_FAMILY_TILE;
+    out->waves = waves; out->slots = 2; out->vec = fv; out->carry = 0;
+    out->tiles_per_row = 1;
+    out->tasks = int32_t(rows);
+    out->grid = ceil_div(q.numseq, rows);
+    out->block = 64 * waves;
+    out->kernel_id = id;
+    out->workspace_bytes = 0;
+    return true;
+  }
+  return false;
+}
+
+// Waves and slots of the tile that holds a row of `max_slots` slots whole, or where none does, of the look-back chain
+// (returns true).
+// Few slots per lane win wherever a row still fits (measured at 2^25 elements, forward:
+// 256-element rows w1 s1 60 us, 1024 w4 s1 63 us against w1 s4 64 us, 2048 w4 s2 63 us
+// against w1 s8 65 us, 4096 w4 s4 and w8 s2 62 us, 8192 w16 s2 63 us against w4 s8 65 us); rows that
+// fill their tile only partly prefer more waves to more slots (3000 elements: w8 s2 72 / 120 us
+// against w4 s4 76 / 132 us).
+// A row that fills little more than half of such a tile leaves every other wave idle from the start;
+// fp32 rows in the lower part of a bucket take half the waves and twice the slots (516 elements:
+// w2 s2 74 / 123 us against w4 s1 86 / 131 us; 260 elements: w1 s2 72 / 137 us against w2 s1 85 / 136 us;
+// from three quarters of the tile on the wider workgroup wins: 800 elements 68 / 112 against 73 / 116 us).
+bool tile_geometry(int64_t max_slots, bool half, int* waves, int* slots) {
+  int w, s;
+  bool chain = false;
+  if (max_slots <= 64) { w = 1; s = 1; }
+  else if (max_slots <= 128) { w = 2; s = 1; if (!half && max_slots <= 80) { w = 1; s = 2; } }
+  else if (max_slots <= 256) { w = 4; s = 1; if (!half && max_slots <= 192) { w = 2; s = 2; } }
+  else if (max_slots <= 512) { w = 4; s = 2; }
+  else if (max_slots <= 1024) { w = 8; s = 2; }
+  else if (max_slots <= 2048) { w = 16; s = 2; }
+  else if (max_slots <= 4096 && !half) { w = 16; s = 4; }
+  else { w = 8; s = half ? 4 : 8; chain = true; }
+  *waves = w;
+  *slots = s;
+  return chain;
+}
+
 int make_plan(const Problem& q, const linrec_tuning_t* tune, linrec_plan_t* out) {
   std::memset(out, 0, sizeof(*out));
   out->kernel_id = -1;
@@ -936,6 +1005,11 @@ int make_plan(const Problem& q, const linrec_tuning_t* tune, linrec_plan_t* out)
             family = LINREC_FAMILY_TILE;
         }
         else if (q.numseq >= (half ? (q.is_bwd ? kTeamMinRowsHalfBwd : kTeamMinRowsHalfFwd) : kTeamMinRows)) family = LINREC_FAMILY_TEAM;
+      }
+      if (family == LINREC_FAMILY_FLAT && packed_plan(q, fv, mode, desc, full_slots, 0, out)) return LINREC_OK;
+      if (family == LINREC_FAMILY_TILE) {
+        int w, s;
+        if (!tile_geometry(full_slots, half, &w, &s) && packed_plan(q, fv, mode, desc, full_slots, int64_t(w) * s * 64, out)) return LINREC_OK;
       }
       // 16-bit storage, many rows of exactly two of the stream kernel's tiles (16384 elements): one workgroup of
       // 8 waves that walks the row beats one tile of 16 waves (bf16 2048 x 16384 34.1 / 57.0 against 36.4 / 59.7 us,
@@ -1177,24 +1251,7 @@ int make_plan(const Problem& q, const linrec_tuning_t* tune, linrec_plan_t* out)
       waves = 4; slots = 4;
       carry = max_slots > 4 * 4 * 64 ? 1 : 0;
     } else {
-      carry = 0;
-      // Few slots per lane win wherever a row still fits (measured at 2^25 elements, forward:
-      // 256-element rows w1 s1 60 us, 1024 w4 s1 63 us against w1 s4 64 us, 2048 w4 s2 63 us
-      // against w1 s8 65 us, 4096 w4 s4 and w8 s2 62 us, 8192 w16 s2 63 us against w4 s8 65 us); rows that
-      // fill their tile only partly prefer more waves to more slots (3000 elements: w8 s2 72 / 120 us
-      // against w4 s4 76 / 132 us).
-      // A row that fills little more than half of such a tile leaves every other wave idle from the start;
-      // fp32 rows in the lower part of a bucket take half the waves and twice the slots (516 elements:
-      // w2 s2 74 / 123 us against w4 s1 86 / 131 us; 260 elements: w1 s2 72 / 137 us against w2 s1 85 / 136 us;
-      // from three quarters of the tile on the wider workgroup wins: 800 elements 68 / 112 against 73 / 116 us).
-      if (max_slots <= 64) { waves = 1; slots = 1; }
-      else if (max_slots <= 128) { waves = 2; slots = 1; if (!half && max_slots <= 80) { waves = 1; slots = 2; } }
-      else if (max_slots <= 256) { waves = 4; slots = 1; if (!half && max_slots <= 192) { waves = 2; slots = 2; } }
-      else if (max_slots <= 512) { waves = 4; slots = 2; }
-      else if (max_slots <= 1024) { waves = 8; slots = 2; }
-      else if (max_slots <= 2048) { waves = 16; slots = 2; }
-      else if (max_slots <= 4096 && !half) { waves = 16; slots = 4; }
-      else { waves = 8; slots = half ? 4 : 8; carry = 1; }
+      carry = tile_geometry(max_slots, half, &waves, &slots) ? 1 : 0;
       // Few rows of a few thousand elements: split them so that the whole chip has work.
       if (!carry && max_slots > 1024 && q.numseq < q.at(kSplitBelowRows)) { waves = 4; slots = half ? 2 : 4; carry = 1; }
     }
