@@ -39,14 +39,24 @@ KernelGroup kernels_bf16_cols();
 #define TILE_ALL_DIRS(TT, DT, PFX, NW, S, VEC, CARRY)                                          \
   TILE_ENTRY(TT, DT, PFX, NW, S, VEC, MODE_FWD, 0, CARRY), TILE_ENTRY(TT, DT, PFX, NW, S, VEC, MODE_FWD, 1, CARRY), \
   TILE_ENTRY(TT, DT, PFX, NW, S, VEC, MODE_BWD, 0, CARRY), TILE_ENTRY(TT, DT, PFX, NW, S, VEC, MODE_BWD, 1, CARRY)
+// ... whose waves at a row's ends mask late (`carry` column 5, and 6 with look-back)
+#define TILE_ENDS_ENTRY(TT, DT, PFX, NW, S, VEC, MODE, DESC, CARRY)                            \
+  {PFX "tile_ends_w" #NW "_s" #S "_v" #VEC "_" #MODE "_" #DESC "_" #CARRY,                     \
+   (const void*)&linrec::tile_kernel<TT, NW, S, VEC, linrec::MODE, DESC != 0, CARRY != 0, true>, DT, \
+   LINREC_FAMILY_TILE, NW, S, VEC, linrec::MODE, DESC, 5 + CARRY}
+#define TILE_ENDS_ALL_DIRS(TT, DT, PFX, NW, S, VEC, CARRY)                                     \
+  TILE_ENDS_ENTRY(TT, DT, PFX, NW, S, VEC, MODE_FWD, 0, CARRY), TILE_ENDS_ENTRY(TT, DT, PFX, NW, S, VEC, MODE_FWD, 1, CARRY), \
+  TILE_ENDS_ENTRY(TT, DT, PFX, NW, S, VEC, MODE_BWD, 0, CARRY), TILE_ENDS_ENTRY(TT, DT, PFX, NW, S, VEC, MODE_BWD, 1, CARRY)
 // several whole rows to a workgroup (`carry` column 4)
 #define PACKED_ENTRY(TT, DT, PFX, NW, S, VEC, MODE, DESC)                                      \
   {PFX "packed_w" #NW "_s" #S "_" #MODE "_" #DESC,                                             \
    (const void*)&linrec::packed_kernel<TT, NW, S, VEC, linrec::MODE, DESC != 0>, DT, LINREC_FAMILY_TILE, \
    NW, S, VEC, linrec::MODE, DESC, 4}
+#define PACKED_BWD_DIRS(TT, DT, PFX, NW, S, VEC)                                               \
+  PACKED_ENTRY(TT, DT, PFX, NW, S, VEC, MODE_BWD, 0), PACKED_ENTRY(TT, DT, PFX, NW, S, VEC, MODE_BWD, 1)
 #define PACKED_ALL_DIRS(TT, DT, PFX, NW, S, VEC)                                               \
   PACKED_ENTRY(TT, DT, PFX, NW, S, VEC, MODE_FWD, 0), PACKED_ENTRY(TT, DT, PFX, NW, S, VEC, MODE_FWD, 1), \
-  PACKED_ENTRY(TT, DT, PFX, NW, S, VEC, MODE_BWD, 0), PACKED_ENTRY(TT, DT, PFX, NW, S, VEC, MODE_BWD, 1)
+  PACKED_BWD_DIRS(TT, DT, PFX, NW, S, VEC)
 #define CHAIN_ENTRY(TT, DT, PFX, NW, S, VEC, MODE, DESC)                                       \
   {PFX "chain_w" #NW "_s" #S "_v" #VEC "_" #MODE "_" #DESC,                                    \
    (const void*)&linrec::chain_kernel<TT, NW, S, VEC, linrec::MODE, DESC != 0>, DT, LINREC_FAMILY_TILE, \
@@ -196,6 +206,8 @@ KernelGroup kernels_bf16_cols();
 #define GROUP_(...) GROUP_ALL_DIRS(__VA_ARGS__)
 #define FLAT_(...) FLAT_ALL_DIRS(__VA_ARGS__)
 #define PACKED_(...) PACKED_ALL_DIRS(__VA_ARGS__)
+#define PACKED_BWD_(...) PACKED_BWD_DIRS(__VA_ARGS__)
+#define TILE_ENDS_(...) TILE_ENDS_ALL_DIRS(__VA_ARGS__)
 #define SEGMENT_(...) SEGMENT_ALL_DIRS(__VA_ARGS__)
 #define COLDRIFT_FWD_(...) COLDRIFT_FWD_DIRS(__VA_ARGS__)
 #define COLDRIFT_BWD_(...) COLDRIFT_BWD_DIRS(__VA_ARGS__)
@@ -216,7 +228,9 @@ KernelGroup kernels_bf16_cols();
 #define HALF_ROW_KERNELS(TY)                                                                    \
   TILE_(TY, 1, 1, 8, 0), TILE_(TY, 2, 1, 8, 0), TILE_(TY, 4, 1, 8, 0), TILE_(TY, 4, 2, 8, 0),   \
   TILE_(TY, 8, 2, 8, 0), TILE_(TY, 16, 2, 8, 0), TILE_(TY, 4, 2, 8, 1), TILE_(TY, 8, 4, 8, 1),  \
-  PACKED_(TY, 4, 2, 8), PACKED_(TY, 8, 2, 8), PACKED_(TY, 16, 2, 8),                            \
+  TILE_ENDS_(TY, 1, 1, 8, 0), TILE_ENDS_(TY, 2, 1, 8, 0), TILE_ENDS_(TY, 4, 1, 8, 0), TILE_ENDS_(TY, 4, 2, 8, 0), \
+  TILE_ENDS_(TY, 8, 2, 8, 0), TILE_ENDS_(TY, 16, 2, 8, 0), TILE_ENDS_(TY, 4, 2, 8, 1), TILE_ENDS_(TY, 8, 4, 8, 1), \
+  PACKED_(TY, 4, 2, 8), PACKED_(TY, 8, 2, 8),                                                   \
   TILE_(TY, 4, 4, 1, 0), TILE_(TY, 4, 4, 1, 1), STREAM_(TY, 8, 2, 8), TEAM_(TY, 8, 2, 8),       \
   TEAM_FWD_(TY, 8, 4, 8), SWEEP_(TY, 8, 2, 8), DRIFT_FWD_(TY, 8, 1, 8),                            \
   DRIFT_FWD_(TY, 16, 1, 8), DRIFT_BWD_(TY, 16, 1, 8), DRIFT_FWD_(TY, 16, 2, 8),                     \

@@ -884,7 +884,8 @@ bool packed_plan(const Problem& q, int fv, int mode, int desc, int64_t row_slots
   if (q.base_mis < 0 || q.elem_stride != 1 || q.numseq < 2 || q.row_stride != q.seqlen || q.batched() || q.seqlen < fv) return false;
   const bool half = q.dtype != LINREC_DTYPE_F32;
   const int64_t elements = q.numseq * q.seqlen;
-  if (elements < 16384 * q.cus) return false;
+  // (tensors of 2^31 elements and more, far beyond what was measured, stay with the kernels they had)
+  if (elements < 16384 * q.cus || elements > 2147483647LL) return false;
   const bool ragged = q.base_mis > 0 || q.seqlen % fv != 0;  // workgroups start and end inside a slot
   if (tile_slots > 0 && !ragged && row_slots == tile_slots) return false;
   if (q.is_bwd && elements >= 65536 * q.cus && tile_slots > 64 && tile_slots <= 256 && row_slots * 100 >= tile_slots * 98) return false;
@@ -907,6 +908,21 @@ bool packed_plan(const Problem& q, int fv, int mode, int desc, int64_t row_slots
     return true;
   }
   return false;
+}
+
+// The form of the tile kernels whose waves at a row's ends mask late (tile_kernel.hpp, ENDS), for `tiles` workgroups.
+// Rows that start or end inside a slot: everywhere (figures there) but in the fp32 backward of wide workgroups that fill
+// half to all of the chip once, where loads and stores of all waves then come in two blocks (2^21 elements in rows of
+// 2049 10.7 against 10.0 us, 3001 10.3 against 10.0, 5001 11.2 against 10.8).
+// Rows of whole slots: 16-bit storage only, whose loads the compiler then spreads better, below a quarter of such a round
+// and from two rounds (one slot to a lane) or four (two) on: bf16 2^21 elements in rows of 4096 4.2 / 5.2 against 4.8 / 6.5 us,
+// 2^24 in rows of 2048 18.4 / 28.7 against 19.3 / 31.7, 2^26 63.5 / 105.8 against 65.3 / 112.4; but 2^23 in rows of 4096, one round, 10.2 /
+// 16.3 against 9.3 / 14.1 (the backward's registers leave seven waves to a SIMD instead of eight).  fp32 2^21 in rows of
+// 3000 6.8 / 9.9 against 6.7 / 8.9.
+bool late_masks_pay(const Problem& q, bool half, bool whole_slots, int64_t tiles, int waves, int slots, int carry) {
+  const int64_t eighths = tiles * waves * 8 / (32 * q.cus);  // of the waves that are on the chip at once
+  if (!whole_slots) return !(q.is_bwd && !half && slots == 2 && waves >= 8 && eighths >= 4 && eighths <= 8);
+  return half && !carry && (eighths <= 2 || eighths >= (slots == 1 ? 16 : 32));
 }
 
 // Waves and slots of the tile that holds a row of `max_slots` slots whole, or where none does, of the look-back chain
@@ -1270,7 +1286,11 @@ int make_plan(const Problem& q, const linrec_tuning_t* tune, linrec_plan_t* out)
     const int64_t row_groups = ceil_div(q.numseq, tasks);
     tasks = int(ceil_div(q.numseq, row_groups));
     // kernel-table code for the carry column: 0 single tile, 1 one tile per workgroup, 2 several
-    const int id = find_kernel(q.dtype, LINREC_FAMILY_TILE, waves, slots, vec, mode, desc, carry ? (tasks > 1 ? 2 : 1) : 0);
+    // (codes 5 and 6: the waves at a row's ends mask late, where that form is compiled and pays)
+    int id = -1;
+    if (tasks == 1 && vec > 1 && late_masks_pay(q, half, rows_on_slots && q.seqlen % fv == 0, row_groups * tiles_per_row, waves, slots, carry))
+      id = find_kernel(q.dtype, LINREC_FAMILY_TILE, waves, slots, vec, mode, desc, carry ? 6 : 5);
+    if (id < 0) id = find_kernel(q.dtype, LINREC_FAMILY_TILE, waves, slots, vec, mode, desc, carry ? (tasks > 1 ? 2 : 1) : 0);
     if (id < 0) return LINREC_E_UNSUPPORTED;
     const int64_t tiles = row_groups * tiles_per_row;  // workgroups
     if (q.numseq * tiles_per_row > 2147483647LL) return LINREC_E_TOO_LARGE;

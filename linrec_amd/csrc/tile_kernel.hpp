@@ -172,8 +172,14 @@ __device__ __forceinline__ void signal_tile_done_end(const TileArgs& p, long lon
   __hip_atomic_store(&p.ws->seq, next_seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-template <typename T, int NW, int S, int VEC, int MODE, bool DESC, bool CARRY>
+// ENDS: a wave that holds an end of its row issues all its loads as whole slots and masks them afterwards (tile_load_edge);
+// without it such a wave looks at every slot and waits for one load after the other where slots lie partly in the row.
+// For rows that start or end inside a slot, forward / backward in us, without and with: fp32 2^23 elements in rows of 1001
+// 20.2 / 32.3 and 18.8 / 31.0, 3001 20.6 / 34.0 and 18.9 / 31.6, 2^18 in rows of 2001 4.6 / 5.7 and 3.6 / 4.3; bf16 2^25 in rows of 5001 40.0 /
+// 70.7 and 35.2 / 59.6, 2^21 of 3001 6.2 / 8.6 and 5.2 / 6.6.
+template <typename T, int NW, int S, int VEC, int MODE, bool DESC, bool CARRY, bool ENDS = false>
 __global__ __launch_bounds__(64 * NW) void tile_kernel(TileArgs p) {
+  static_assert(!ENDS || VEC > 1, "whole slots");
   constexpr int WAVE_SLOTS = S * 64;
   constexpr int TILE_SLOTS = NW * WAVE_SLOTS;
   __shared__ float sh_a[NW];
@@ -212,6 +218,16 @@ __global__ __launch_bounds__(64 * NW) void tile_kernel(TileArgs p) {
   TileData<S, VEC, MODE> d;
   if (interior) {
     tile_load<S, VEC, MODE, DESC, true>(d, q, rv, u_wave, lane, row_start);
+  } else if constexpr (ENDS) {
+    tile_load_edge<S, VEC, MODE, DESC>(d, q, rv, u_wave, lane);
+    tile_mask<S, VEC, MODE, DESC>(d, rv, u_wave, lane);
+    if constexpr (MODE == MODE_FWD) {
+      // the coefficient of the row's first element in scan order takes no part
+      const int first = DESC ? rv.nslots * VEC - rv.hi : rv.lo;
+#pragma unroll
+      for (int i = 0; i < VEC; ++i)
+        if (row_start && lane == 0 && i == first) d.cs[0][i] = 0.0f;
+    }
   } else {
     tile_load<S, VEC, MODE, DESC, false>(d, q, rv, u_wave, lane, row_start);
   }
