@@ -7,8 +7,10 @@
 // (linrec/impl/cuda/linrec_pipe.cuh:8-143), which also keeps a row inside one block; the tile
 // scan, the register double buffer and the addressing differ.
 //
-// Structure of a row: tiles [0, t_lo) and [t_hi, ntiles) touch a row end and take the predicated
-// path without prefetch; the tiles in between are interior for every wave of the workgroup and run
+// Structure of a row: tiles [0, t_lo) and [t_hi, ntiles) touch a row end: they are loaded as whole slots and masked when
+// their turn has come (a partial last tile's loads stay in flight while the tile before it is scanned; looking at every slot
+// as it arrived cost bf16 2^25 elements in rows of 20001 48.9 / 79.7 us forward / backward where this takes 39.7 / 67.1, fp32 2^23
+// in rows of 10001 22.9 / 37.9 and 21.9 / 35.8); the tiles in between are interior for every wave of the workgroup and run
 // the pipelined loop, whose body is straight-line code so that the wait before scanning tile t
 // leaves the loads of tile t+1 outstanding.
 #pragma once
@@ -87,10 +89,25 @@ __global__ __launch_bounds__(64 * NW) void stream_kernel(TileArgs p) {
     carry = has_carry ? fmaf(carry, total.a, total.b) : total.b;
     has_carry = true;
   };
+  // Its loads, as whole slots, and the masks once its turn has come (tile_load_edge).
+  auto edge_load = [&](int t, TileData<S, VEC, MODE>& d) {
+    tile_load_edge<S, VEC, MODE, DESC>(d, q, rv, t * TILE_SLOTS + wave * WAVE_SLOTS, lane);
+  };
+  auto edge_mask = [&](int t, TileData<S, VEC, MODE>& d) {
+    tile_mask<S, VEC, MODE, DESC>(d, rv, t * TILE_SLOTS + wave * WAVE_SLOTS, lane);
+    if constexpr (MODE == MODE_FWD) {
+      // the coefficient of the row's first element in scan order takes no part
+      const int first = DESC ? rv.nslots * VEC - rv.hi : rv.lo;
+#pragma unroll
+      for (int i = 0; i < VEC; ++i)
+        if (t == 0 && wave == 0 && lane == 0 && i == first) d.cs[0][i] = 0.0f;
+    }
+  };
   // The same, loaded and processed on the spot.
   auto edge_tile = [&](int t) {
     TileData<S, VEC, MODE> d;
-    tile_load<S, VEC, MODE, DESC, false>(d, q, rv, t * TILE_SLOTS + wave * WAVE_SLOTS, lane, t == 0 && wave == 0);
+    edge_load(t, d);
+    edge_mask(t, d);
     edge_finish(t, d);
   };
 
@@ -142,8 +159,9 @@ __global__ __launch_bounds__(64 * NW) void stream_kernel(TileArgs p) {
       // a partial tile ends the row: its loads go out before the last interior tile is processed, so
       // that rows of two or three tiles overlap anything at all (3355 x 10000 backward: 186 -> 123 us)
       TileData<S, VEC, MODE> last;
-      tile_load<S, VEC, MODE, DESC, false>(last, q, rv, t_hi * TILE_SLOTS + wave * WAVE_SLOTS, lane, false);
+      edge_load(t_hi, last);
       interior_tile(t_hi - 1, cur);
+      edge_mask(t_hi, last);
       edge_finish(t_hi, last);
       t_hi = ntiles;  // (at most one partial tile follows the interior ones)
     } else {

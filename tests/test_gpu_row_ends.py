@@ -76,3 +76,25 @@ def test_many_rows_in_the_widest_tiles_and_16_bit_rows_of_whole_slots(dtype, row
     dx_t, dc_t = oracle.bwd(_f64(dy), _f64(c), _f64(y), reverse)
     check_close(dx, dx_t, "d_inputs", tol)
     check_close(dc, dc_t, "d_coeffs", tol)
+
+
+@pytest.mark.parametrize("reverse", [False, True])
+@pytest.mark.parametrize("dtype,L,gap", [(torch.float32, 8201, 0), (torch.float32, 8195, 2), (torch.float32, 12287, 1), (torch.float32, 16384, 1),
+                                         (torch.bfloat16, 16387, 0), (torch.bfloat16, 17000, 0), (torch.bfloat16, 24575, 3)])
+def test_one_workgroup_walks_rows_that_end_inside_a_tile(dtype, L, gap, reverse):
+    """Rows of one to three whole tiles and a last one of a slot, of part of its slots, or of all but an element."""
+    from linrec_amd import _native as nat
+    tol = TOL_NORMWISE if dtype == torch.float32 else 1.05 * 2.0 ** -8
+    rows = 300
+    g = torch.Generator().manual_seed(L)
+    x, dy = (torch.randn(rows, L + gap, generator=g).to(dtype)[:, :L] for _ in range(2))
+    c = (torch.rand(rows, L + gap, generator=g) * 1.9 - 0.95).to(dtype)[:, :L]
+    xd, cd, dyd = (torch.empty(rows, L + gap, dtype=dtype, device="cuda:0")[:, :L].copy_(t) for t in (x, c, dy))
+    assert "stream" in nat.kernel_table()[nat.plan(xd, reverse)["kernel_id"]]
+    y = nat.fwd(xd, cd, reverse)
+    dx, dc = nat.bwd(dyd, cd, y, reverse)
+    torch.cuda.synchronize()
+    check_close(y, oracle.fwd(_f64(x), _f64(c), reverse), "outputs", tol)
+    dx_t, dc_t = oracle.bwd(_f64(dy), _f64(c), _f64(y), reverse)
+    check_close(dx, dx_t, "d_inputs", tol)
+    check_close(dc, dc_t, "d_coeffs", tol)
