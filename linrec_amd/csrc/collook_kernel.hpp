@@ -51,10 +51,12 @@
 #include <type_traits>
 
 #include "coldrift_kernel.hpp"  // ColDriftArgs, Held
+#include "lookback_lanes.hpp"
 
 namespace linrec {
 
-constexpr int PHASE_LOOKBACK = 3;  // the kernel table's code beside PHASE_REDUCE and PHASE_APPLY
+constexpr int PHASE_LOOKBACK = 3;         // the kernel table's codes beside PHASE_REDUCE and PHASE_APPLY:
+constexpr int PHASE_LOOKBACK_SHARED = 4;  // ... where a batch's rows are not a multiple of the rows of a lane
 
 // VEC adjacent rows of one position by one access that need not be aligned to more than an element.
 template <typename T, int VEC>
@@ -99,10 +101,27 @@ __device__ __forceinline__ void st_any(T* p, const Lanes<VEC>& r) {
   }
 }
 
+// The same for rows `first` (at least 1, the same for all lanes) and up only.
+template <int VEC, typename T>
+__device__ __forceinline__ void st_from(T* p, const Lanes<VEC>& r, unsigned first) {
+  static_assert(VEC == 2 || VEC == 4, "rows left out: one, or one to three");
+  if constexpr (VEC == 2) {
+    st_any<1>(p + 1, Lanes<1>{{r.v[1]}});
+  } else {
+    if (first & 1u) st_any<1>(p + first, Lanes<1>{{first == 1u ? r.v[1] : r.v[3]}});
+    if (first < 3u) st_any<2>(p + 2, Lanes<2>{{r.v[2], r.v[3]}});
+  }
+}
+
+// SHARED: a batch's last lane shares rows with the lane before it and leaves them to that one (lookback_lanes.hpp).  A kernel
+// of its own: with both kinds of stores in one, fp32 16 x 2048 x 512 backward, which has no such lane, took 64.6 us
+// instead of 62.5.  Which rows a lane leaves out is the same for all lanes that do, so the branches are scalar (a mask per
+// row and lane: fp32 23 x 25862 x 77 forward 160 us, where this takes 148; bf16 2 x 125567 x 222 107 / 184 and 98 / 165).
 // (of args.chain: tasks = blocks of lanes, num_tiles = workgroups; of args.col: lanes_per_segment = lanes of a segment)
-template <typename T, int VEC, int U, int NW, int MODE, bool DESC>
+template <typename T, int VEC, int U, int NW, int MODE, bool DESC, bool SHARED = false>
 __global__ __launch_bounds__(64 * NW) void collook_kernel(ColDriftArgs args) {
   static_assert(VEC <= NW, "a wave per row of a lane looks back");
+  static_assert(!SHARED || VEC > 1, "a lane of one row shares none");
   const ColumnArgs& p = args.col;
   const TileArgs& ch = args.chain;
   constexpr int RPB = 64 * VEC;  // rows of a block
@@ -137,19 +156,15 @@ __global__ __launch_bounds__(64 * NW) void collook_kernel(ColDriftArgs args) {
       block = int(id - unsigned(k) * nb);
     }
   }
-  // Lanes are numbered batch by batch; where a batch's rows are not a multiple of VEC its last lane starts early and
-  // shares rows with the one before it (both compute and store them).
   unsigned lane_no = unsigned(block) * 64u + unsigned(lane);  // (the planner keeps lanes and rows of a segment below 2^31)
   const bool active = lane_no < unsigned(p.lanes_per_segment);
   if (!active) lane_no = unsigned(p.lanes_per_segment) - 1u;  // lanes beyond the last row read the last rows again and store nothing
   const unsigned rows = unsigned(p.rows_per_batch < p.numseq ? p.rows_per_batch : p.numseq);
-  const unsigned lanes = (rows + unsigned(VEC) - 1u) / unsigned(VEC);
-  const unsigned batch = p.rows_per_batch < p.numseq ? lane_no / lanes : 0u;
-  unsigned row = (lane_no - batch * lanes) * unsigned(VEC);
-  if (row > rows - unsigned(VEC)) row = rows - unsigned(VEC);
+  const LaneRows held = lookback_lane_rows(lane_no, rows, unsigned(VEC), p.rows_per_batch < p.numseq);
+  const unsigned own_from = lookback_own_from(rows, unsigned(VEC));  // (a scalar)
   // A wave's accesses are a scalar address plus 32 bits per lane (the planner sees to it that a block's rows span
   // less than 2^31 bytes): 64-bit addresses per lane took 30 to 40 registers, and with them a workgroup per CU.
-  const long long base = (long long)batch * p.batch_stride + (long long)row * p.row_stride;
+  const long long base = (long long)held.batch * p.batch_stride + (long long)held.row * p.row_stride;
   const long long wbase = (long long)(uint32_t)__builtin_amdgcn_readfirstlane(int(base)) |
                           ((long long)__builtin_amdgcn_readfirstlane(int(base >> 32)) << 32);
   const uint32_t lane_bytes = uint32_t(base - wbase) * uint32_t(sizeof(T));
@@ -172,9 +187,18 @@ __global__ __launch_bounds__(64 * NW) void collook_kernel(ColDriftArgs args) {
   const int n0 = k * STEP + wave * U;
   // positions a whole number of 128-byte lines apart: no line is wanted twice
   const bool on_lines = p.elem_stride * (long long)sizeof(T) % 128 == 0;
-  // FULL: all positions of the segment exist and, for the backward, so does the last one's successor.
-  auto segment = [&](auto full_tag, auto stream_tag) __attribute__((always_inline)) {
-    constexpr bool FULL = decltype(full_tag)::value, STREAM = decltype(stream_tag)::value;
+  // FULL: all positions of the segment exist and, for the backward, so does the last one's successor.  OWN: some of the
+  // block's lanes store part of their rows only.
+  auto segment = [&](auto full_tag, auto stream_tag, auto own_tag) __attribute__((always_inline)) {
+    constexpr bool FULL = decltype(full_tag)::value, STREAM = decltype(stream_tag)::value, OWN = decltype(own_tag)::value;
+    auto store = [&](T* to, const Lanes<VEC>& r) __attribute__((always_inline)) {
+      if constexpr (OWN) {
+        if (held.own != 0) st_from<VEC>(to, r, own_from);
+        else st_any<VEC>(to, r);
+      } else {
+        st_any<VEC>(to, r);
+      }
+    };
     Batch bt;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -342,7 +366,7 @@ __global__ __launch_bounds__(64 * NW) void collook_kernel(ColDriftArgs args) {
         if constexpr (MODE == 0) {
 #pragma unroll
           for (int e = 0; e < VEC; ++e) val.v[e] = n == 0 ? x.v[e] : fmaf(val.v[e], c.v[e], x.v[e]);
-          if (active) st_any<VEC>(at(out0, l), val);
+          if (active) store(at(out0, l), val);
         } else {
           const Lanes<VEC> yn = widen(held_again(bt.yn[u]));
           Lanes<VEC> dx, dc;
@@ -353,17 +377,25 @@ __global__ __launch_bounds__(64 * NW) void collook_kernel(ColDriftArgs args) {
             val.v[e] = dx.v[e] * c.v[e];
           }
           if (active) {
-            st_any<VEC>(at(out0, l), dx);
-            st_any<VEC>(at(out1, l), dc);
+            store(at(out0, l), dx);
+            store(at(out1, l), dc);
           }
         }
       }
     }
   };
   const bool full = (k + 1) * (long long)STEP <= (NEED_Y ? L - 1 : L);
-  if (full && on_lines) segment(std::true_type{}, std::true_type{});
-  else if (full) segment(std::true_type{}, std::false_type{});
-  else segment(std::false_type{}, std::false_type{});
+  if constexpr (SHARED) {
+    // (the waves of a workgroup hold the same lanes, so they all take the same form)
+    const bool own = __ballot(active && held.own != 0) != 0;
+    if (full && !own) segment(std::true_type{}, std::false_type{}, std::false_type{});
+    else if (full) segment(std::true_type{}, std::false_type{}, std::true_type{});
+    else segment(std::false_type{}, std::false_type{}, std::true_type{});
+  } else {
+    if (full && on_lines) segment(std::true_type{}, std::true_type{}, std::false_type{});
+    else if (full) segment(std::true_type{}, std::false_type{}, std::false_type{});
+    else segment(std::false_type{}, std::false_type{}, std::false_type{});
+  }
 
   // (the look-back waves are past the last barrier: no descriptor of this launch is touched by this workgroup again)
   if (threadIdx.x == 0) {

@@ -181,6 +181,17 @@ KernelGroup kernels_bf16_cols();
   {PFX "segment_lookback_w" #NW "_v" #VEC "_u" #U "_" #MODE "_" #DESC,                         \
    (const void*)&linrec::collook_kernel<TT, VEC, U, NW, linrec::MODE, DESC != 0>, DT,          \
    LINREC_FAMILY_SEGMENT, NW, U, VEC, linrec::MODE, DESC, linrec::PHASE_LOOKBACK}
+#define COLLOOK_SHARED_ENTRY(TT, DT, PFX, NW, VEC, U, MODE, DESC)                              \
+  {PFX "segment_lookback_shared_w" #NW "_v" #VEC "_u" #U "_" #MODE "_" #DESC,                  \
+   (const void*)&linrec::collook_kernel<TT, VEC, U, NW, linrec::MODE, DESC != 0, true>, DT,    \
+   LINREC_FAMILY_SEGMENT, NW, U, VEC, linrec::MODE, DESC, linrec::PHASE_LOOKBACK_SHARED}
+// (of several rows to a lane, both forms)
+#define COLLOOK_WIDE_FWD_DIRS(TT, DT, PFX, NW, VEC, U)                                         \
+  COLLOOK_FWD_DIRS(TT, DT, PFX, NW, VEC, U),                                                   \
+  COLLOOK_SHARED_ENTRY(TT, DT, PFX, NW, VEC, U, MODE_FWD, 0), COLLOOK_SHARED_ENTRY(TT, DT, PFX, NW, VEC, U, MODE_FWD, 1)
+#define COLLOOK_WIDE_BWD_DIRS(TT, DT, PFX, NW, VEC, U)                                         \
+  COLLOOK_BWD_DIRS(TT, DT, PFX, NW, VEC, U),                                                   \
+  COLLOOK_SHARED_ENTRY(TT, DT, PFX, NW, VEC, U, MODE_BWD, 0), COLLOOK_SHARED_ENTRY(TT, DT, PFX, NW, VEC, U, MODE_BWD, 1)
 #define COLLOOK_FWD_DIRS(TT, DT, PFX, NW, VEC, U)                                              \
   COLLOOK_ENTRY(TT, DT, PFX, NW, VEC, U, MODE_FWD, 0), COLLOOK_ENTRY(TT, DT, PFX, NW, VEC, U, MODE_FWD, 1)
 #define COLLOOK_BWD_DIRS(TT, DT, PFX, NW, VEC, U)                                              \
@@ -213,6 +224,8 @@ KernelGroup kernels_bf16_cols();
 #define COLDRIFT_BWD_(...) COLDRIFT_BWD_DIRS(__VA_ARGS__)
 #define COLLOOK_FWD_(...) COLLOOK_FWD_DIRS(__VA_ARGS__)
 #define COLLOOK_BWD_(...) COLLOOK_BWD_DIRS(__VA_ARGS__)
+#define COLLOOK_WIDE_FWD_(...) COLLOOK_WIDE_FWD_DIRS(__VA_ARGS__)
+#define COLLOOK_WIDE_BWD_(...) COLLOOK_WIDE_BWD_DIRS(__VA_ARGS__)
 #define COLBLOCK_FWD_(...) COLBLOCK_FWD_DIRS(__VA_ARGS__)
 #define COLBLOCK_BWD_(...) COLBLOCK_BWD_DIRS(__VA_ARGS__)
 
@@ -241,7 +254,8 @@ KernelGroup kernels_bf16_cols();
   SEGMENT_(TY, 4, 8), SEGMENT_(TY, 2, 8), SEGMENT_(TY, 1, 8),                                   \
   COLBLOCK_FWD_(TY, 2, 8, 1), COLBLOCK_BWD_(TY, 2, 4, 1), COLBLOCK_FWD_(TY, 2, 8, 2), COLBLOCK_BWD_(TY, 2, 4, 2), \
   COLDRIFT_FWD_(TY, 16, 2, 8), COLDRIFT_BWD_(TY, 8, 2, 16), COLDRIFT_FWD_(TY, 8, 2, 16), COLDRIFT_BWD_(TY, 16, 2, 4), \
-  COLLOOK_NARROW_KERNELS(TY), COLLOOK_FWD_(TY, 16, 2, 16), COLLOOK_BWD_(TY, 16, 2, 16), COLLOOK_FWD_(TY, 16, 4, 16), COLLOOK_BWD_(TY, 16, 4, 16)
+  COLLOOK_NARROW_KERNELS(TY), COLLOOK_WIDE_FWD_(TY, 16, 2, 16), COLLOOK_WIDE_BWD_(TY, 16, 2, 16), \
+  COLLOOK_WIDE_FWD_(TY, 16, 4, 16), COLLOOK_WIDE_BWD_(TY, 16, 4, 16)
 
 #define LINREC_KERNEL_GROUP(NAME, ...)                                                          \
   namespace linrec {                                                                            \

@@ -33,5 +33,6 @@ LINREC_KERNEL_GROUP(kernels_f32_cols,
     // 4096 x 16384 forward 187 against 157 us, 2048 x 16384 124 against 85.3 us, 8192 x 4096 89.6 against 82.7 us)
     COLDRIFT_FWD_(F32, 16, 1, 8), COLDRIFT_BWD_(F32, 16, 1, 4), COLDRIFT_FWD_(F32, 8, 1, 16), COLDRIFT_BWD_(F32, 8, 1, 16),
     // segments in one launch, chained by look-back
-    COLLOOK_NARROW_KERNELS(F32), COLLOOK_FWD_(F32, 16, 2, 16), COLLOOK_FWD_(F32, 16, 4, 8), COLLOOK_BWD_(F32, 16, 2, 8), COLLOOK_BWD_(F32, 16, 4, 8)
+    COLLOOK_NARROW_KERNELS(F32), COLLOOK_WIDE_FWD_(F32, 16, 2, 16), COLLOOK_WIDE_FWD_(F32, 16, 4, 8), COLLOOK_WIDE_BWD_(F32, 16, 2, 8),
+    COLLOOK_WIDE_BWD_(F32, 16, 4, 8)
 )

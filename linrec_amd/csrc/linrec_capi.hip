@@ -62,7 +62,7 @@ int find_kernel(int dtype, int family, int waves, int slots, int vec, int mode, 
     const bool waves_matter = family == LINREC_FAMILY_TILE || family == LINREC_FAMILY_STREAM ||
                               family == LINREC_FAMILY_TEAM || family == LINREC_FAMILY_SWEEP || family == LINREC_FAMILY_DRIFT || family == LINREC_FAMILY_GROUP ||
                               family == LINREC_FAMILY_FLAT || family == LINREC_FAMILY_COLDRIFT ||
-                              (family == LINREC_FAMILY_SEGMENT && carry == linrec::PHASE_LOOKBACK);
+                              (family == LINREC_FAMILY_SEGMENT && carry >= linrec::PHASE_LOOKBACK);
     if (k.dtype == dtype && k.family == family && k.slots == slots && k.vec == vec && k.mode == mode &&
         k.desc == desc && k.carry == carry && (!waves_matter || k.waves == waves))
       return i;
@@ -642,9 +642,13 @@ bool coldrift_applies(const Problem& q) {
 // The plan of a segmented launch whose segments are chained by look-back (one launch): `waves` waves per workgroup
 // with runs of `depth` positions, `vec` rows to a lane.
 // Lanes of a segment: `vec` adjacent rows each, a batch's last lane overlapping the one before it where the rows of a batch
-// are not a multiple of `vec`.
+// are not a multiple of `vec` (lookback_lanes.hpp).
 int64_t lookback_lanes(const Problem& q, int64_t vec) {
   return q.batched() ? q.numseq / q.rows_per_batch * ceil_div(q.rows_per_batch, vec) : ceil_div(q.numseq, vec);
+}
+// The form of the kernels: where lanes share rows, each row has to be left to one of them.
+int lookback_form(const Problem& q, int64_t vec) {
+  return (q.batched() ? q.rows_per_batch : q.numseq) % vec ? linrec::PHASE_LOOKBACK_SHARED : linrec::PHASE_LOOKBACK;
 }
 // Segments dealt out at a time (collook_kernel.hpp): eight where that is as good or better, whole groups of which there are
 // at least two.  Forward / backward in us, eight against one: off the 128-byte lines fp32 8326 x 4022 (time x channels) 91.6 /
@@ -668,7 +672,7 @@ int lookback_segments_plan(const Problem& q, int vec, int waves, int depth, int 
     if (q.row_stride > bound / rows || (q.batched() && q.batch_stride > bound / 2 / (rows / rpb + 2)) || q.row_stride * rows > bound / 2)
       return LINREC_E_UNSUPPORTED;
   }
-  const int id = find_kernel(q.dtype, LINREC_FAMILY_SEGMENT, waves, depth, vec, mode, desc, linrec::PHASE_LOOKBACK);
+  const int id = find_kernel(q.dtype, LINREC_FAMILY_SEGMENT, waves, depth, vec, mode, desc, lookback_form(q, vec));
   if (id < 0) return LINREC_E_UNSUPPORTED;
   const int64_t rows_per_block = int64_t(64) * vec;
   const int64_t blocks = ceil_div(lookback_lanes(q, vec), 64);
@@ -1616,7 +1620,7 @@ int launch(const linrec_plan_t& plan, const Problem& q, const void* in0, const v
   if (plan.family == LINREC_FAMILY_SEGMENT && plan.carry == 1) {
     const int64_t rows_per_block = int64_t(64) * k.vec, lanes = lookback_lanes(q, k.vec);
     const int64_t blocks = ceil_div(lanes, 64);
-    if (plan.block != 64 * k.waves || k.carry != linrec::PHASE_LOOKBACK || plan.tiles_per_row != ceil_div(q.seqlen, int64_t(k.waves) * k.slots) ||
+    if (plan.block != 64 * k.waves || k.carry != lookback_form(q, k.vec) || plan.tiles_per_row != ceil_div(q.seqlen, int64_t(k.waves) * k.slots) ||
         plan.grid != blocks * plan.tiles_per_row)
       return LINREC_E_INVALID;  // (what the kernel is compiled for)
     if (!workspace || (reinterpret_cast<uintptr_t>(workspace) & 15u) || workspace_bytes < plan.workspace_bytes)
