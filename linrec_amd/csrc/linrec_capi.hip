@@ -319,6 +319,13 @@ int half_drift_slots_for(const Problem& q, int fv) {
   }
   return 0;
 }
+// Slots a row takes where rows start wherever they do: one more than its length asks for unless all start on a slot.
+bool rows_start_on_slots(const Problem& q, int fv) { return q.base_mis == 0 && (q.row_stride % fv == 0 || q.numseq == 1); }
+int64_t slots_of_a_row(const Problem& q, int fv) { return ceil_div(q.seqlen + (rows_start_on_slots(q, fv) ? 0 : fv - 1), fv); }
+// Tiles of `tile` elements that a row takes in a drift launch, the partial ones included: what its workspace, its teams
+// and its walk are counted in.
+int64_t drift_tiles_per_row(const Problem& q, int fv, int64_t tile) { return ceil_div(slots_of_a_row(q, fv) * fv, tile); }
+
 // Rows that start or end inside a slot.
 bool drift_skewed(const Problem& q, int fv) {
   return q.base_mis > 0 || (q.numseq > 1 && q.row_stride % fv != 0) || q.seqlen % fv != 0;
@@ -370,7 +377,8 @@ int drift_slots_for(const Problem& q, int fv) {
     if (ragged && (half || s != (q.is_bwd ? 2 : 4))) continue;
     if (skewed && !drift_skewed_pays(q)) continue;
     const int64_t tiles_per_row = q.seqlen / tile;  // (full ones)
-    const int64_t team = drift_team_size(q, tiles_per_row + ragged, 8, q.cus, ragged);
+    const int64_t all_tiles = drift_tiles_per_row(q, fv, tile);
+    const int64_t team = drift_team_size(q, all_tiles, 8, q.cus, ragged);
     // the forward's tiles of 8192 elements: as many tiles a row as the generated table says, and from its number of
     // rows on also rows of two tiles in teams of two (us, against one workgroup per row: 2048 x 16384 66.2 against 69.3,
     // 4096 x 16384 128.9 against 138.8; but 600 x 16384 22.6 against 22.1, 1024 x 16384 34.5 against 35.0)
@@ -378,7 +386,7 @@ int drift_slots_for(const Problem& q, int fv) {
                                 : q.numseq >= q.at(kT_drift_fwd_two_tiles_min_rows) ? 2 : kT_drift_fwd_min_tiles_per_row;
     if (tiles_per_row < least_tiles || team < least_tiles) continue;
     // (a caller that can only give so much workspace is served by the kernels that need less)
-    if (q.workspace_cap && linrec_workspace_bytes_for_tiles(q.numseq * (tiles_per_row + ragged)) > q.workspace_cap) continue;
+    if (q.workspace_cap && linrec_workspace_bytes_for_tiles(q.numseq * all_tiles) > q.workspace_cap) continue;
     // fp32 rows of fewer than eight tiles of 4096 elements: one workgroup per row does as well or better
     // (forward / backward in us: 768 x 16384 27.3 / 46.3 against 32.3 / 47.5, 400 x 24576 22.6 / 36.4 against
     // 26.3 / 39.7, 1000 x 24576 52.2 / 89.3 against 55.7 / 90.3, 1536 x 16384 52.4 / 90.4 against 55.3 / 89.7,
@@ -976,8 +984,8 @@ int make_plan(const Problem& q, const linrec_tuning_t* tune, linrec_plan_t* out)
   const int fv = full_vec_of(q.dtype);        // elements of a 16-byte slot
   const bool half = q.dtype != LINREC_DTYPE_F32;
   // slots a row needs when all rows start on a slot boundary, one more otherwise
-  const bool rows_on_slots = q.base_mis == 0 && (q.row_stride % fv == 0 || q.numseq == 1);
-  const int64_t full_slots = ceil_div(q.seqlen + (rows_on_slots ? 0 : fv - 1), fv);
+  const bool rows_on_slots = rows_start_on_slots(q, fv);
+  const int64_t full_slots = slots_of_a_row(q, fv);
 
   // The gradient scan runs against the forward scan.
   const int desc = (q.reverse != 0) != (q.is_bwd != 0) ? 1 : 0;
@@ -1193,7 +1201,8 @@ int make_plan(const Problem& q, const linrec_tuning_t* tune, linrec_plan_t* out)
     // 43.6, 1024 x 65536 132.2 against 133.8, 16 x 1048576 in teams of 128 37.6 against 38.1 - compiled without
     // the larger teams' code, which does not fit its registers, so those keep 8 waves).
     if (drift && !half && !q.is_bwd && auto_slots == 4 && !(tune && (tune->waves > 0 || tune->slots > 0)) &&
-        drift_team_size(q, ceil_div(q.seqlen, int64_t(8) * 4 * 64 * fv), 8, q.cus, q.seqlen % (int64_t(8) * 4 * 64 * fv) != 0) <= 64) {
+        drift_team_size(q, drift_tiles_per_row(q, fv, int64_t(8) * 4 * 64 * fv), 8, q.cus,
+                        drift_skewed(q, fv) || q.seqlen % (int64_t(8) * 4 * 64 * fv) != 0) <= 64) {
       waves = 16;
       slots = 2;
     }
@@ -1208,7 +1217,7 @@ int make_plan(const Problem& q, const linrec_tuning_t* tune, linrec_plan_t* out)
     const int id = find_kernel(q.dtype, family, waves, slots, fv, mode, desc, skewed ? 3 : ragged ? 2 : 1);
     if (id < 0) return LINREC_E_UNSUPPORTED;
     const int block = 64 * waves;
-    const int64_t tiles_per_row = ceil_div(full_slots * fv, tile_elems);
+    const int64_t tiles_per_row = drift_tiles_per_row(q, fv, tile_elems);
     // Every workgroup of the launch has to be resident at once (a walker waits for its team mates, and a
     // workgroup that has not started yet only starts when another one ends): never more than the CUs hold.
     const int64_t resident = int64_t(workgroups_per_cu(id, block, drift || q.is_bwd ? 1 : 2)) * q.cus;
