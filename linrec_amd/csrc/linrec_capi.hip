@@ -8,6 +8,7 @@
 #include <cstdio>
 #include <cstring>
 #include <mutex>
+#include <utility>
 #include <vector>
 
 #include "../../include/linrec_hip.h"
@@ -56,18 +57,35 @@ const std::vector<KernelEntry> g_kernel_table = [] {
 const KernelEntry* const kKernels = g_kernel_table.data();
 const int kNumKernels = int(g_kernel_table.size());
 
-int find_kernel(int dtype, int family, int waves, int slots, int vec, int mode, int desc, int carry) {
+// What an entry is looked up by, in one word; 0 where a caller's tuning asks for more than any entry has.
+uint64_t kernel_key(int dtype, int family, int waves, int slots, int vec, int mode, int desc, int carry) {
+  const bool waves_matter = family == LINREC_FAMILY_TILE || family == LINREC_FAMILY_STREAM ||
+                            family == LINREC_FAMILY_TEAM || family == LINREC_FAMILY_SWEEP || family == LINREC_FAMILY_DRIFT || family == LINREC_FAMILY_GROUP ||
+                            family == LINREC_FAMILY_FLAT || family == LINREC_FAMILY_COLDRIFT ||
+                            (family == LINREC_FAMILY_SEGMENT && carry >= linrec::PHASE_LOOKBACK);
+  uint64_t key = 1;
+  for (int part : {dtype, family, carry, mode, desc, vec, slots, waves_matter ? waves : 0}) {
+    if (part < 0 || part > 127) return 0;
+    key = key << 7 | uint64_t(part);
+  }
+  return key;
+}
+// The table in the order of these words (a walk through its more than seven hundred entries took as long as the rest of a
+// plan: bf16 8 x 4096 x 1024 forward 1.7 us, 0.2 with the words).  Of equal entries the first counts.
+const std::vector<std::pair<uint64_t, int>> g_kernel_index = [] {
+  std::vector<std::pair<uint64_t, int>> all;
   for (int i = 0; i < kNumKernels; ++i) {
     const KernelEntry& k = kKernels[i];
-    const bool waves_matter = family == LINREC_FAMILY_TILE || family == LINREC_FAMILY_STREAM ||
-                              family == LINREC_FAMILY_TEAM || family == LINREC_FAMILY_SWEEP || family == LINREC_FAMILY_DRIFT || family == LINREC_FAMILY_GROUP ||
-                              family == LINREC_FAMILY_FLAT || family == LINREC_FAMILY_COLDRIFT ||
-                              (family == LINREC_FAMILY_SEGMENT && carry >= linrec::PHASE_LOOKBACK);
-    if (k.dtype == dtype && k.family == family && k.slots == slots && k.vec == vec && k.mode == mode &&
-        k.desc == desc && k.carry == carry && (!waves_matter || k.waves == waves))
-      return i;
+    all.emplace_back(kernel_key(k.dtype, k.family, k.waves, k.slots, k.vec, k.mode, k.desc, k.carry), i);
   }
-  return -1;
+  std::sort(all.begin(), all.end());
+  return all;
+}();
+
+int find_kernel(int dtype, int family, int waves, int slots, int vec, int mode, int desc, int carry) {
+  const uint64_t key = kernel_key(dtype, family, waves, slots, vec, mode, desc, carry);
+  const auto it = std::lower_bound(g_kernel_index.begin(), g_kernel_index.end(), std::make_pair(key, 0));
+  return key != 0 && it != g_kernel_index.end() && it->first == key ? it->second : -1;
 }
 
 // ---- the device ------------------------------------------------------------------------------
@@ -668,32 +686,35 @@ int64_t lookback_segments_at_once(const Problem& q, int64_t blocks, int64_t segm
   const bool on_lines = q.elem_stride * elem_size_of(q.dtype) % 128 == 0;
   return segments >= 16 && (on_lines ? q.is_bwd && blocks >= 4 : blocks >= 2) ? 8 : 1;
 }
-int lookback_segments_plan(const Problem& q, int vec, int waves, int depth, int mode, int desc, linrec_plan_t* out) {
+// Workgroups of such a launch, without a look at the kernel table; negative: LINREC_E_UNSUPPORTED or LINREC_E_TOO_LARGE.
+int64_t lookback_segments_grid(const Problem& q, int vec, int waves, int depth) {
   if (vec < 1 || colblock_rows_per_lane(q, 1) != 1) return LINREC_E_UNSUPPORTED;
   const int64_t rpb = q.batched() ? q.rows_per_batch : q.numseq;
   if (vec > 1 && (q.row_stride != 1 || rpb < vec)) return LINREC_E_UNSUPPORTED;
+  const int64_t rows_per_block = int64_t(64) * vec;
   // (a lane's offset from its wave's first row is 32 bits of bytes: strides forward, a block's rows within 2^31 bytes)
-  {
-    const int64_t rows = 64 * int64_t(vec);
-    if (q.row_stride < 0 || (q.batched() && q.batch_stride < rpb * q.row_stride)) return LINREC_E_UNSUPPORTED;
-    const int64_t bound = (int64_t(1) << 31) / elem_size_of(q.dtype);
-    if (q.row_stride > bound / rows || (q.batched() && q.batch_stride > bound / 2 / (rows / rpb + 2)) || q.row_stride * rows > bound / 2)
-      return LINREC_E_UNSUPPORTED;
-  }
+  if (q.row_stride < 0 || (q.batched() && q.batch_stride < rpb * q.row_stride)) return LINREC_E_UNSUPPORTED;
+  const int64_t bound = (int64_t(1) << 31) / elem_size_of(q.dtype);
+  if (q.row_stride > bound / rows_per_block || (q.batched() && q.batch_stride > bound / 2 / (rows_per_block / rpb + 2)) ||
+      q.row_stride * rows_per_block > bound / 2)
+    return LINREC_E_UNSUPPORTED;
+  const int64_t grid = ceil_div(lookback_lanes(q, vec), 64) * ceil_div(q.seqlen, int64_t(waves) * depth);
+  return grid * rows_per_block > 2147483647LL ? LINREC_E_TOO_LARGE : grid;
+}
+int lookback_segments_plan(const Problem& q, int vec, int waves, int depth, int mode, int desc, linrec_plan_t* out) {
+  const int64_t grid = lookback_segments_grid(q, vec, waves, depth);
+  if (grid == LINREC_E_UNSUPPORTED) return LINREC_E_UNSUPPORTED;
   const int id = find_kernel(q.dtype, LINREC_FAMILY_SEGMENT, waves, depth, vec, mode, desc, lookback_form(q, vec));
   if (id < 0) return LINREC_E_UNSUPPORTED;
-  const int64_t rows_per_block = int64_t(64) * vec;
-  const int64_t blocks = ceil_div(lookback_lanes(q, vec), 64);
-  const int64_t segments = ceil_div(q.seqlen, int64_t(waves) * depth);
-  if (blocks * segments * rows_per_block > 2147483647LL) return LINREC_E_TOO_LARGE;
+  if (grid < 0) return int(grid);
   out->family = LINREC_FAMILY_SEGMENT;
   out->waves = waves; out->slots = depth; out->vec = vec; out->carry = 1;
-  out->tiles_per_row = int32_t(segments);
+  out->tiles_per_row = int32_t(ceil_div(q.seqlen, int64_t(waves) * depth));
   out->tasks = waves * depth;
-  out->grid = blocks * segments;
+  out->grid = grid;
   out->block = 64 * waves;
   out->kernel_id = id;
-  out->workspace_bytes = linrec_workspace_bytes_for_tiles(blocks * segments * rows_per_block);
+  out->workspace_bytes = linrec_workspace_bytes_for_tiles(grid * 64 * vec);
   return LINREC_OK;
 }
 
@@ -808,28 +829,30 @@ bool lookback_segments_choose(const Problem& q, int family, int colblock, int mo
   static const int shapes[2][2][3][3] = {{{{4, 16, 8}, {2, 16, 16}, {1, 8, 16}}, {{4, 16, 8}, {2, 16, 8}, {1, 8, 16}}},
                                          {{{4, 16, 16}, {2, 16, 16}, {1, 8, 16}}, {{4, 16, 16}, {2, 16, 16}, {1, 8, 16}}}};
   const int(*s)[3] = shapes[half][q.is_bwd != 0];
-  linrec_plan_t p[3];
+  // (the rules below only look at the workgroups; a plan of each geometry took bf16 8 x 4096 x 1024 from 1.7 / 0.8 to 2.4 /
+  // 1.9 us of host time a call, forward / backward)
+  int64_t grids[3];
   bool fits[3];
   for (int i = 0; i < 3; ++i) {
-    std::memset(&p[i], 0, sizeof(p[i]));
-    fits[i] = lookback_segments_plan(q, s[i][0], s[i][1], s[i][2], mode, desc, &p[i]) == LINREC_OK;
+    grids[i] = lookback_segments_grid(q, s[i][0], s[i][1], s[i][2]);
+    fits[i] = grids[i] >= 0;
     if (s[i][0] == 1) continue;
     const int64_t lanes = ceil_div(lookback_lanes(q, s[i][0]), 64) * 64;  // of a segment, with and without a row
     if (q.numseq * 2 <= lanes * s[i][0] || (q.batched() && channels < 24)) fits[i] = false;
   }
   auto round_and_a_bit = [&](int64_t grid, int64_t sixteenths) { return grid > q.cus && grid * 16 <= q.cus * (16 + sixteenths); };
   auto enough = [&](int i) {  // workgroups
-    const int64_t grid = p[i].grid;
+    const int64_t grid = grids[i];
     if (s[i][0] == 1) return true;
-    if (s[i][0] == 4) return grid * 16 >= q.cus * (fits[1] && round_and_a_bit(p[1].grid, 5) ? 9 : 10);
+    if (s[i][0] == 4) return grid * 16 >= q.cus * (fits[1] && round_and_a_bit(grids[1], 5) ? 9 : 10);
     if (q.is_bwd) return grid * 16 >= (half ? 9 : 10) * q.cus;
-    if (half) return grid * 16 >= (q.seqlen > 4096 ? 7 : 4) * q.cus && p[2].grid >= q.cus;
+    if (half) return grid * 16 >= (q.seqlen > 4096 ? 7 : 4) * q.cus && grids[2] >= q.cus;
     return grid * 128 >= (on_lines || q.seqlen > 2048 ? 68 : 44) * q.cus;
   };
   for (int i = 0, kept = 0; i < 3; ++i) {
     if (!fits[i]) continue;
     const bool fwd_pairs = !half && !q.is_bwd && !on_lines && s[i][0] == 2, fwd_fours = !half && !q.is_bwd && s[i][0] == 4;
-    if (fwd_fours && (on_lines || q.numseq < q.at(1536) || p[i].grid < 2 * q.cus)) continue;
+    if (fwd_fours && (on_lines || q.numseq < q.at(1536) || grids[i] < 2 * q.cus)) continue;
     if (!enough(i)) continue;
     // fp32: column blocks keep the shortest axes in the backward, one row to a lane (8 x 256 x 1024 12.0 against 10.3, 8 x
     // 352 x 832 15.4 against 13.0; with two 8 x 300 x 896 13.8 against 12.4, but 8 x 352 x 1024 13.6 against 15.5, 8 x 448 x
@@ -847,19 +870,23 @@ bool lookback_segments_choose(const Problem& q, int family, int colblock, int mo
     //   16-bit storage from 7/8 of the CUs up to 9/8 workgroups per CU, in whole steps of the blocks up to 11/8 (8 x 1280 x
     //     1792 30.8 / 48.2 against 26.8 / 43.3, 16 x 1200 x 896 29.2 / 43.5 against 27.0 / 39.4; but 16 x 1200 x 1024 29.9 /
     //     45.1 against 33.0 / 48.0, 8 x 1400 x 1536 28.1 / 41.8 against 33.4 / 46.6).
-    if (!kept++ && colblock == 2 && on_lines && p[i].waves == 16 && p[i].grid > q.cus) {
+    if (!kept++ && colblock == 2 && on_lines && s[i][1] == 16 && grids[i] > q.cus) {
       const int64_t blocks = ceil_div(q.numseq / colblock_rows_per_lane(q, 0), 32);
       const bool whole_kib = q.elem_stride * 4 % 1024 == 0;
       const bool fills = blocks * 16 >= (half ? 14 : s[i][0] <= 2 && whole_kib ? 13 : 11) * q.cus;
       const int64_t up_to = half ? (q.seqlen % 128 == 0 ? 11 : 9) : s[i][0] <= 2 ? (whole_kib ? 12 : 14) : whole_kib ? 0 : 12;
-      if (fills && p[i].grid * 8 < up_to * q.cus) return false;
+      if (fills && grids[i] * 8 < up_to * q.cus) return false;
     }
-    if (!q.is_bwd && family == LINREC_FAMILY_COLDRIFT && on_lines && q.seqlen < 4096 && round_and_a_bit(p[i].grid, 4)) return false;
-    if (s[i][0] > 1 && !q.is_bwd && !(half && on_lines) && round_and_a_bit(p[i].grid, 4)) continue;
-    if (fwd_pairs && (q.seqlen > 1920 && p[2].grid >= (on_slots ? 3 : 2) * q.cus)) continue;
+    if (!q.is_bwd && family == LINREC_FAMILY_COLDRIFT && on_lines && q.seqlen < 4096 && round_and_a_bit(grids[i], 4)) return false;
+    if (s[i][0] > 1 && !q.is_bwd && !(half && on_lines) && round_and_a_bit(grids[i], 4)) continue;
+    if (fwd_pairs && (q.seqlen > 1920 && grids[2] >= (on_slots ? 3 : 2) * q.cus)) continue;
     // (a caller that can only give so much workspace is served by the kernels that need less)
-    if (q.workspace_cap && p[i].workspace_bytes > q.workspace_cap) return false;
-    *out = p[i];
+    linrec_plan_t p;
+    std::memset(&p, 0, sizeof(p));
+    p.kernel_id = -1;
+    if (lookback_segments_plan(q, s[i][0], s[i][1], s[i][2], mode, desc, &p) != LINREC_OK) return false;
+    if (q.workspace_cap && p.workspace_bytes > q.workspace_cap) return false;
+    *out = p;
     return true;
   }
   return false;
