@@ -359,7 +359,7 @@ bool drift_skewed(const Problem& q, int fv) {
 // 33554431 75.8 against 82.3, 4 x 8388609 77.2 against 83.0).
 bool drift_skewed_pays(const Problem& q) {
   if (q.is_bwd) return q.numseq <= q.at(2560) || q.seqlen < kT_stream_max_len;
-  return q.numseq >= q.at(20) ? q.numseq < q.cus : q.numseq < kT_team_min_rows && q.numseq * q.seqlen >= 12 * 8192 * q.cus;
+  return q.numseq >= 20 ? q.numseq < q.cus : q.numseq < kT_team_min_rows && q.numseq * q.seqlen >= 12 * 8192 * q.cus;
 }
 // Returns the tile to use as slots per lane of 8 waves (4: 8192 fp32 elements, 2: 4096), 0 for "not a drift
 // case"; which kernel serves the tile (8 waves, or 16 with half the slots) is the launch planner's business.

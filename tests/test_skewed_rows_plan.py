@@ -63,16 +63,3 @@ def test_rows_of_as_many_tiles_take_the_same_launch():
                 assert [a[k] for k in keys] == [b[k] for k in keys], (rows, tiles, a, b)
                 seen.add((a["waves"], a["tasks"] > 64))
     assert {(16, False), (8, True)} <= seen, seen
-
-
-def test_the_rows_of_the_forward_s_teams_follow_the_compute_units():
-    """A quarter of the rows on a quarter of the compute units: the same work for each, and teams on both."""
-    for rows in (24, 40, 100, 192):
-        for length in (262145, 524289, 1048577):
-            families = []
-            for part in (1, 4):
-                nat.set_compute_units(256 // part)
-                p = nat.Plan()
-                assert nat.lib().linrec_plan(0, None, rows // part, length, length, 1, 0, 0, None, ctypes.byref(p)) == 0
-                families.append(p.family)
-            assert families == [nat.FAMILY_DRIFT] * 2, (rows, length, families)
