@@ -1,0 +1,39 @@
+"""How many rows a lane of the look-back segments takes (planner only, for 256 compute units)."""
+import ctypes
+
+import pytest
+
+from linrec_amd import _native as nat
+
+F32, F16, BF16 = 0, 1, 2
+
+
+@pytest.fixture(autouse=True)
+def full_part():
+    old = nat.set_compute_units(256)
+    yield
+    nat.set_compute_units(old)
+
+
+def rows_of_a_lane(dtype, batch, time, channels, is_bwd):
+    """0: not served by look-back segments."""
+    p = nat.Plan()
+    assert nat.lib().linrec_plan_batched(dtype, None, batch, channels, time, time * channels, 1, channels, 0, int(is_bwd), None,
+                                         ctypes.byref(p)) == 0
+    return p.vec if p.family == nat.FAMILY_SEGMENT and p.carry == 1 else 0
+
+
+@pytest.mark.parametrize("dtype", [F32, F16, BF16])
+@pytest.mark.parametrize("is_bwd", [False, True])
+def test_lanes_of_narrow_batches_take_rows_that_start_on_an_access(dtype, is_bwd):
+    """(of fewer than 64 channels, 80 in 16-bit storage)"""
+    least, seen = 64 if dtype == F32 else 80, set()
+    for channels in (24, 25, 26, 28, 29, 37, 42, 48, 50, 55, 58, 60, 63, 65, 66, 75, 79, 81, 90, 98, 150, 222):
+        for batch, time in ((3, 40000), (6, 50000), (17, 17000), (115, 4000), (320, 750)):
+            vec = rows_of_a_lane(dtype, batch, time, channels, is_bwd)
+            if channels < least:
+                assert vec == 0 or channels % vec == 0, (batch, time, channels, vec)
+            elif vec > 1 and channels % vec:
+                seen.add(vec)
+    assert 4 in seen, seen
+    assert rows_of_a_lane(dtype, 2, 262144, 64, is_bwd) == 2  # (positions that start on lines)
