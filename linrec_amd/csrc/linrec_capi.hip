@@ -750,10 +750,14 @@ int lookback_segments_plan(const Problem& q, int vec, int waves, int depth, int 
 // 13.7).  Drawn closer, `enough`:
 //   four rows: nine sixteenths of the CUs where two rows would make a little more than one round (bf16 1880 x 4704 forward 152
 //     workgroups 16.3, 296 of two rows 21.8; fp32 6 x 256 x 3058 backward 144 23.8, 288 31.0);
-//   two rows, forward: little more than half (fp32 2048 x 2048 128 workgroups 14.5, 512 of one row 15.2; 10005 x 192 x 2 120 18.4,
-//     474 15.7), off the lines and on axes of up to 2048 positions a third (fp32 778 x 4051 128 12.9, 448 14.9, 441 x 5810 92
-//     13.0, 364 14.0); 16-bit storage from a quarter on where one row makes a workgroup for each CU (7 x 256 x 1664 91 8.8, 364
-//     10.9; 300 x 4096 64 10.6, 192 7.7), on axes beyond 4096 from seven sixteenths (26869 x 103 105 15.6, 420 13.8).
+//   two rows, forward: fp32 five eighths as above (42 x 1560 x 64 147 workgroups 16.0, 546 of one row 14.2; 2 x 4100 x 512 136 16.8,
+//     528 14.5; 2 x 12000 x 192 141 19.1, 564 16.5; 16 x 1560 x 192 168 16.1, 624 16.3), off the lines and on axes of up to 2048 positions a
+//     third (778 x 4051 128 12.9, 448 14.9, 441 x 5810 92 13.0, 364 14.0); 16-bit storage where one row makes two workgroups for each
+//     CU (11 x 300 x 512 88 10.9, 264 8.7; 4 x 900 x 512 64 10.9, 256 8.9; 15 x 900 x 192 92 11.1, 360 10.7; 6 x 3000 x 192 108 12.4, 432 11.6;
+//     8 x 3000 x 192 144 12.4, 576 13.0), five for four where the axis is whole segments of two rows but for a few positions
+//     or off the lines (16 x 2048 x 64 64 9.6, 256 9.5; 7 x 2048 x 192 88 9.9, 336 10.9; 9 x 2048 x 192 112 10.1, 432 11.6; 10 x 4100 x 64 85
+//     10.6, 330 11.1; 3 x 900 x 1000 96 11.0, 376 12.2), and on axes beyond 4096 from seven sixteenths of the CUs (26869 x 103 105
+//     15.6, 420 13.8).
 // A forward whose workgroups are a little more than one round (up to five quarters of the CUs) takes the next narrower
 // access (fp32 3 x 35605 x 59 280 workgroups of two rows 36.3, 837 of one 26.7; 33112 x 148 28.0 and 21.9; bf16 8192 x 2049 four rows
 // 39.0, two 35.3), 16-bit storage on whole lines excepted (8 x 1400 x 1536 four rows 25.4, two 29.8).
@@ -852,8 +856,8 @@ bool lookback_segments_choose(const Problem& q, int family, int colblock, int mo
     if (s[i][0] == 1) return true;
     if (s[i][0] == 4) return grid * 16 >= q.cus * (fits[1] && round_and_a_bit(grids[1], 5) ? 9 : 10);
     if (q.is_bwd) return grid * 16 >= (half ? 9 : 10) * q.cus;
-    if (half) return grid * 16 >= (q.seqlen > 4096 ? 7 : 4) * q.cus && grids[2] >= q.cus;
-    return grid * 128 >= (on_lines || q.seqlen > 2048 ? 68 : 44) * q.cus;
+    if (half) return grid * 16 >= (q.seqlen > 4096 ? 7 : 4) * q.cus && grids[2] * 4 >= (on_lines && q.seqlen % 256 >= 16 ? 8 : 5) * q.cus;
+    return grid * 128 >= (on_lines || q.seqlen > 2048 ? 80 : 44) * q.cus;
   };
   for (int i = 0, kept = 0; i < 3; ++i) {
     if (!fits[i]) continue;

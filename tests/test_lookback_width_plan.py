@@ -37,3 +37,15 @@ def test_lanes_of_narrow_batches_take_rows_that_start_on_an_access(dtype, is_bwd
                 seen.add(vec)
     assert 4 in seen, seen
     assert rows_of_a_lane(dtype, 2, 262144, 64, is_bwd) == 2  # (positions that start on lines)
+
+
+def test_a_forward_that_leaves_much_of_the_chip_idle_takes_one_row_to_a_lane():
+    """Two rows to a lane from five eighths of the compute units on, in 16-bit storage where one row would make two workgroups
+    for each, five for four where the axis is whole segments of 256 positions."""
+    for batch, time, channels, want in [(42, 1560, 64, 1), (2, 4100, 512, 1), (2, 12000, 192, 1), (8, 8842, 64, 1), (16, 1560, 192, 2),
+                                        (48, 1560, 64, 2), (20, 4100, 64, 2)]:
+        assert rows_of_a_lane(F32, batch, time, channels, False) == want, (batch, time, channels)
+    for batch, time, channels, want in [(11, 342, 512, 1), (4, 900, 512, 1), (12, 2730, 64, 1), (2, 2000, 512, 1), (7, 1560, 192, 1),
+                                        (9, 2048, 192, 2), (7, 2048, 192, 2), (15, 900, 192, 1), (10, 4100, 64, 1), (16, 4100, 64, 2), (5, 1560, 512, 2), (6, 3000, 192, 1), (8, 3000, 192, 2)]:
+        for dtype in (F16, BF16):
+            assert rows_of_a_lane(dtype, batch, time, channels, False) == want, (batch, time, channels)
