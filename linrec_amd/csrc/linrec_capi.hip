@@ -926,7 +926,12 @@ Problem tail_problem(const Problem& q, int64_t tail_rows) {
 // / 0.72; 2^25 1.25 / 1.11, 1.23 / 1.13, 1.17 / 0.92.  So four waves, from 2^25 on eight, and sixteen for the fp32 backward;
 // more where that many hold less than two rows, or leave a fifth of the lanes idle (bf16 2^25 x 1401 backward 67.5 in
 // four waves, 64.6 in eight, 67.4 with one row to a workgroup; 3001 in eight 67.3 against 65.5).
-// Not rows that fill their own workgroup (fp32 2^25, 256 elements: 62.6 / 108.6 against 61.1 / 105.5), nor the backward of
+// Not rows of whole slots that fill most of their own workgroup, whose loads need no masks either way (geometric means
+// against one row to a workgroup, forward / backward, by how much of it is filled: 16-bit storage half 0.92 / 0.98, five
+// eighths 0.99 / 1.03, 11/16 1.03 / 1.08, three quarters 1.05 / 1.05, 7/8 1.02 / 1.05, bf16 1944 x 3392 9.5 against 8.2, backward 3728 x 1792 15.8
+// against 13.4; fp32 three quarters to all 0.99 / 0.99 with single lengths up to 1.12, 1584 backward 2^23 31.2 against 27.8; of
+// less than 1.5 times the least size 9/16 and more 1.04); nor in the 16-bit backward rows off the slots from 7/8 on (1.06 against
+// the form of the tile kernels that masks late; the forward 1.01).  Nor the backward of
 // large tensors where one slot to a lane does (1001: 117.9 against 112.9; bf16 2001: 62.9 against 61.1; at 2^23 1001 30.9
 // against 32.0), nor the large backward of a few floats (5: 116.1 against 113.8).
 bool packed_plan(const Problem& q, int fv, int mode, int desc, int64_t row_slots, int64_t tile_slots, linrec_plan_t* out) {
@@ -936,7 +941,10 @@ bool packed_plan(const Problem& q, int fv, int mode, int desc, int64_t row_slots
   // (tensors of 2^31 elements and more, far beyond what was measured, stay with the kernels they had)
   if (elements < 16384 * q.cus || elements > 2147483647LL) return false;
   const bool ragged = q.base_mis > 0 || q.seqlen % fv != 0;  // workgroups start and end inside a slot
-  if (tile_slots > 0 && !ragged && row_slots == tile_slots) return false;
+  if (tile_slots > 0 && (!ragged || (half && q.is_bwd))) {
+    const int sixteenths = ragged ? 14 : half ? (q.is_bwd ? 10 : 11) : elements < 24576 * q.cus ? 9 : 12;
+    if (row_slots * 16 >= tile_slots * sixteenths) return false;
+  }
   if (q.is_bwd && elements >= 65536 * q.cus && tile_slots > 64 && tile_slots <= 256 && row_slots * 100 >= tile_slots * 98) return false;
   const bool large = elements >= 131072 * q.cus;
   if (q.is_bwd && !half && large && q.seqlen < 16) return false;

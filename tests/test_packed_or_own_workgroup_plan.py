@@ -1,0 +1,54 @@
+"""Which dense short rows are packed and which keep a workgroup of their own (planner only, for 256 compute units)."""
+import ctypes
+
+import pytest
+
+from linrec_amd import _native as nat
+
+F32, F16, BF16 = 0, 1, 2
+
+
+@pytest.fixture(autouse=True)
+def full_part():
+    old = nat.set_compute_units(256)
+    yield
+    nat.set_compute_units(old)
+
+
+def packed(dtype, rows, length, is_bwd):
+    p = nat.Plan()
+    assert nat.lib().linrec_plan(dtype, None, rows, length, length, 1, 0, int(is_bwd), None, ctypes.byref(p)) == 0
+    return "packed" in nat.kernel_table()[p.kernel_id]
+
+
+@pytest.mark.parametrize("dtype", [F16, BF16])
+def test_16_bit_rows_of_whole_slots_that_fill_their_workgroup(dtype):
+    """(a workgroup of one row holds 512, 1024, 2048 or 4096 elements)"""
+    for is_bwd, least in ((False, 11), (True, 10)):
+        for room in (512, 1024, 2048, 4096):
+            for sixteenths in range(9, 17):
+                for rows in ((1 << 22) // room * 3 // 2, (1 << 24) // room, (1 << 26) // room):
+                    length = room * sixteenths // 16
+                    if rows * length >= 1 << 22:
+                        assert packed(dtype, rows, length, is_bwd) == (sixteenths < least), (is_bwd, rows, length)
+    assert not packed(dtype, 1944, 3392, False) and not packed(dtype, 3728, 1792, True)
+
+
+@pytest.mark.parametrize("dtype", [F16, BF16])
+def test_16_bit_backward_of_rows_off_the_slots(dtype):
+    for room in (1024, 2048, 4096):
+        for rows in ((1 << 23) // room, (1 << 26) // room):
+            assert packed(dtype, rows, room * 13 // 16 + 1, True) and packed(dtype, rows, room * 15 // 16 + 1, False), (rows, room)
+            assert not packed(dtype, rows, room * 15 // 16 + 1, True), (rows, room)
+
+
+@pytest.mark.parametrize("is_bwd", [False, True])
+def test_single_precision_rows_of_whole_slots(is_bwd):
+    for room in (512, 1024, 2048, 4096):
+        for rows in ((1 << 23) // room * 3 // 2, (1 << 26) // room):
+            if room < 4096:  # (two rows have to fit)
+                assert packed(F32, rows, room * 11 // 16, is_bwd), (rows, room)
+            assert not packed(F32, rows, room * 13 // 16, is_bwd), (rows, room)
+        length = room * 10 // 16
+        assert not packed(F32, (1 << 22) // length + 1, length, is_bwd), room  # little work
+    assert not packed(F32, 4849, 1584, True) and not packed(F32, 22657, 192, False)
