@@ -46,7 +46,7 @@ def test_16_bit_backward_of_rows_off_the_slots(dtype):
 def test_single_precision_rows_of_whole_slots(is_bwd):
     for room in (512, 1024, 2048, 4096):
         for rows in ((1 << 23) // room * 3 // 2, (1 << 26) // room):
-            if room < 4096:  # (two rows have to fit)
+            if room < 2048:  # (whole rows have to fill four fifths of a workgroup)
                 assert packed(F32, rows, room * 11 // 16, is_bwd), (rows, room)
             assert not packed(F32, rows, room * 13 // 16, is_bwd), (rows, room)
         length = room * 10 // 16
