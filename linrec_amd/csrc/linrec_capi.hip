@@ -970,7 +970,13 @@ bool packed_plan(const Problem& q, int fv, int mode, int desc, int64_t row_slots
 // The form of the tile kernels whose waves at a row's ends mask late (tile_kernel.hpp, ENDS), for `tiles` workgroups.
 // Rows that start or end inside a slot: everywhere (figures there) but in the fp32 backward of wide workgroups that fill
 // half to all of the chip once, where loads and stores of all waves then come in two blocks (2^21 elements in rows of
-// 2049 10.7 against 10.0 us, 3001 10.3 against 10.0, 5001 11.2 against 10.8).
+// 2049 10.7 against 10.0 us, 3001 10.3 against 10.0, 5001 11.2 against 10.8; of two waves from six eighths on, 3065 x 549 8.7
+// against 8.1); and the backward of two slots to a lane in 16-bit storage, which takes 72 to 74 registers where the other form
+// takes 62 to 64, so that a SIMD holds six or seven of its waves instead of eight: where half to all of the chip is filled once
+// (bf16 559 x 7138 11.0 against 9.5, 1217 x 4084 11.9 against 10.8; below that and beyond, 0.72 to 0.95), and in workgroups of sixteen
+// waves, of which a CU then holds one instead of two, everywhere beyond that in bf16 (2910 x 9843 64.0 against 57.2, 2478 x 8192 49.7
+// against 44.1; fp16, whose other form spends more on its conversions, gains there: 0.89).  bf16 forward, sixteen waves, half to three
+// quarters of the chip: 1.04.
 // Rows of whole slots: 16-bit storage only, whose loads the compiler then spreads better, below a quarter of such a round
 // and from two rounds (one slot to a lane) or four (two) on: bf16 2^21 elements in rows of 4096 4.2 / 5.2 against 4.8 / 6.5 us,
 // 2^24 in rows of 2048 18.4 / 28.7 against 19.3 / 31.7, 2^26 63.5 / 105.8 against 65.3 / 112.4; but 2^23 in rows of 4096, one round, 10.2 /
@@ -978,7 +984,12 @@ bool packed_plan(const Problem& q, int fv, int mode, int desc, int64_t row_slots
 // 3000 6.8 / 9.9 against 6.7 / 8.9.
 bool late_masks_pay(const Problem& q, bool half, bool whole_slots, int64_t tiles, int waves, int slots, int carry) {
   const int64_t eighths = tiles * waves * 8 / (32 * q.cus);  // of the waves that are on the chip at once
-  if (!whole_slots) return !(q.is_bwd && !half && slots == 2 && waves >= 8 && eighths >= 4 && eighths <= 8);
+  const bool bf16 = q.dtype == LINREC_DTYPE_BF16;
+  if (half && slots == 2 && !carry && eighths >= 4) {
+    if (q.is_bwd && waves >= 4 && (eighths <= (bf16 ? 7 : 5) || (bf16 && waves == 16))) return false;
+    if (!q.is_bwd && bf16 && waves == 16 && eighths <= 5) return false;
+  }
+  if (!whole_slots) return !(q.is_bwd && !half && slots == 2 && (waves >= 8 ? eighths >= 4 && eighths <= 8 : waves == 2 && (eighths == 6 || eighths == 7)));
   return half && !carry && (eighths <= 2 || eighths >= (slots == 1 ? 16 : 32));
 }
 
