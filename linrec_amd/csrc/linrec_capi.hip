@@ -970,7 +970,7 @@ bool packed_plan(const Problem& q, int fv, int mode, int desc, int64_t row_slots
 // The form of the tile kernels whose waves at a row's ends mask late (tile_kernel.hpp, ENDS), for `tiles` workgroups.
 // Rows that start or end inside a slot: everywhere (figures there) but in the fp32 backward of wide workgroups that fill
 // half to all of the chip once, where loads and stores of all waves then come in two blocks (2^21 elements in rows of
-// 2049 10.7 against 10.0 us, 3001 10.3 against 10.0, 5001 11.2 against 10.8; of two waves from six eighths on, 3065 x 549 8.7
+// 2049 10.7 against 10.0 us, 3001 10.3 against 10.0, 5001 11.2 against 10.8; of two waves from five eighths on, 3065 x 549 8.7
 // against 8.1); and the backward of two slots to a lane in 16-bit storage, which takes 72 to 74 registers where the other form
 // takes 62 to 64, so that a SIMD holds six or seven of its waves instead of eight: where half to all of the chip is filled once
 // (bf16 559 x 7138 11.0 against 9.5, 1217 x 4084 11.9 against 10.8; below that and beyond, 0.72 to 0.95), and in workgroups of sixteen
@@ -989,7 +989,7 @@ bool late_masks_pay(const Problem& q, bool half, bool whole_slots, int64_t tiles
     if (q.is_bwd && waves >= 4 && (eighths <= (bf16 ? 7 : 5) || (bf16 && waves == 16))) return false;
     if (!q.is_bwd && bf16 && waves == 16 && eighths <= 5) return false;
   }
-  if (!whole_slots) return !(q.is_bwd && !half && slots == 2 && (waves >= 8 ? eighths >= 4 && eighths <= 8 : waves == 2 && (eighths == 6 || eighths == 7)));
+  if (!whole_slots) return !(q.is_bwd && !half && slots == 2 && (waves >= 8 ? eighths >= 4 && eighths <= 8 : waves == 2 && eighths >= 5 && eighths <= 7));
   return half && !carry && (eighths <= 2 || eighths >= (slots == 1 ? 16 : 32));
 }
 
