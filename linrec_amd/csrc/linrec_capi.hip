@@ -760,7 +760,9 @@ int lookback_segments_plan(const Problem& q, int vec, int waves, int depth, int 
 //     15.6, 420 13.8).
 // A forward whose workgroups are a little more than one round (up to five quarters of the CUs) takes the next narrower
 // access (fp32 3 x 35605 x 59 280 workgroups of two rows 36.3, 837 of one 26.7; 33112 x 148 28.0 and 21.9; bf16 8192 x 2049 four rows
-// 39.0, two 35.3), 16-bit storage on whole lines excepted (8 x 1400 x 1536 four rows 25.4, two 29.8).
+// 39.0, two 35.3), 16-bit storage on whole lines excepted (8 x 1400 x 1536 four rows 25.4, two 29.8), and on whole lines up
+// to 33/32 of the CUs (4 x 13107 x 160 260 workgroups of two rows 23.2, 1030 of one 26.2, 2 x 21845 x 192 258 23.9, 1026 26.1; but 5 x
+// 22595 x 64 267 39.0, 885 30.9; bf16 10 x 13130 x 64 156 of four rows 19.4, 260 of two 16.7).
 // The fp32 forward off the lines: two rows are no better than one from three rounds of workgroups on (30 x 1024 x 1500 135
 // against 122, 2 x 125567 x 222 166 against 156, 8192 x 1025 32.8 against 29.6; 8326 x 4022 91.6 against 93.1), four are from
 // about 1536 rows and two rounds on (23 x 25862 x 77 137.6, 151.3 and 161.4 with four, two and one; 2 x 166672 x 82 90, 99 and 88).
@@ -851,10 +853,13 @@ bool lookback_segments_choose(const Problem& q, int family, int colblock, int mo
     if (q.numseq * 2 <= lanes * s[i][0] || (q.batched() && channels < (aligned ? 24 : half ? 80 : 64))) fits[i] = false;
   }
   auto round_and_a_bit = [&](int64_t grid, int64_t sixteenths) { return grid > q.cus && grid * 16 <= q.cus * (16 + sixteenths); };
+  auto leaves_much_idle = [&](int64_t grid, int64_t sixteenths) {
+    return round_and_a_bit(grid, sixteenths) && (q.is_bwd || !on_lines || grid * 32 > q.cus * 33);
+  };
   auto enough = [&](int i) {  // workgroups
     const int64_t grid = grids[i];
     if (s[i][0] == 1) return true;
-    if (s[i][0] == 4) return grid * 16 >= q.cus * (fits[1] && round_and_a_bit(grids[1], 5) ? 9 : 10);
+    if (s[i][0] == 4) return grid * 16 >= q.cus * (fits[1] && leaves_much_idle(grids[1], 5) ? 9 : 10);
     if (q.is_bwd) return grid * 16 >= (half ? 9 : 10) * q.cus;
     if (half) return grid * 16 >= (q.seqlen > 4096 ? 7 : 4) * q.cus && grids[2] * 4 >= (on_lines && q.seqlen % 256 >= 16 ? 8 : 5) * q.cus;
     return grid * 128 >= (on_lines || q.seqlen > 2048 ? 80 : 44) * q.cus;
@@ -888,7 +893,7 @@ bool lookback_segments_choose(const Problem& q, int family, int colblock, int mo
       if (fills && grids[i] * 8 < up_to * q.cus) return false;
     }
     if (!q.is_bwd && family == LINREC_FAMILY_COLDRIFT && on_lines && q.seqlen < 4096 && round_and_a_bit(grids[i], 4)) return false;
-    if (s[i][0] > 1 && !q.is_bwd && !(half && on_lines) && round_and_a_bit(grids[i], 4)) continue;
+    if (s[i][0] > 1 && !q.is_bwd && !(half && on_lines) && leaves_much_idle(grids[i], 4)) continue;
     if (fwd_pairs && (q.seqlen > 1920 && grids[2] >= (on_slots ? 3 : 2) * q.cus)) continue;
     // (a caller that can only give so much workspace is served by the kernels that need less)
     linrec_plan_t p;

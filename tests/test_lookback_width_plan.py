@@ -49,3 +49,12 @@ def test_a_forward_that_leaves_much_of_the_chip_idle_takes_one_row_to_a_lane():
                                         (9, 2048, 192, 2), (7, 2048, 192, 2), (15, 900, 192, 1), (10, 4100, 64, 1), (16, 4100, 64, 2), (5, 1560, 512, 2), (6, 3000, 192, 1), (8, 3000, 192, 2)]:
         for dtype in (F16, BF16):
             assert rows_of_a_lane(dtype, batch, time, channels, False) == want, (batch, time, channels)
+
+
+def test_a_forward_on_whole_lines_that_makes_hardly_more_than_one_round():
+    """(of workgroups, up to 33/32 of the compute units, is not told from one that makes a round)"""
+    for batch, time, channels, want in [(4, 13107, 160, 2), (2, 13107, 320, 2), (2, 21845, 192, 2), (5, 22595, 64, 1), (3, 34342, 64, 1),
+                                        (2, 17718, 256, 1)]:
+        assert rows_of_a_lane(F32, batch, time, channels, False) == want, (batch, time, channels)
+    for batch, time, channels, want in [(10, 13130, 64, 2), (14, 9272, 64, 2), (10, 7379, 128, 4), (15, 1040, 512, 4)]:
+        assert rows_of_a_lane(BF16, batch, time, channels, False) == want, (batch, time, channels)
