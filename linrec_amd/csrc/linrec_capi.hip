@@ -760,7 +760,9 @@ int lookback_segments_plan(const Problem& q, int vec, int waves, int depth, int 
 //     15.6, 420 13.8).
 // A forward whose workgroups are a little more than one round (up to five quarters of the CUs) takes the next narrower
 // access (fp32 3 x 35605 x 59 280 workgroups of two rows 36.3, 837 of one 26.7; 33112 x 148 28.0 and 21.9; bf16 8192 x 2049 four rows
-// 39.0, two 35.3), 16-bit storage on whole lines excepted (8 x 1400 x 1536 four rows 25.4, two 29.8), and on whole lines up
+// 39.0, two 35.3), 16-bit storage on whole lines excepted (8 x 1400 x 1536 four rows 25.4, two 29.8) and four
+// rows of an even number of channels (8 x 1323 x 1584 29.3, two 34.3; 29 x 1079 x 564 35.0, 40.9; 17 of 20 shapes within 3 % or
+// better, of an odd number 0.91 to 0.97), and on whole lines up
 // to 33/32 of the CUs (4 x 13107 x 160 260 workgroups of two rows 23.2, 1030 of one 26.2, 2 x 21845 x 192 258 23.9, 1026 26.1; but 5 x
 // 22595 x 64 267 39.0, 885 30.9; bf16 10 x 13130 x 64 156 of four rows 19.4, 260 of two 16.7).
 // The fp32 forward off the lines: two rows are no better than one from three rounds of workgroups on (30 x 1024 x 1500 135
@@ -893,7 +895,7 @@ bool lookback_segments_choose(const Problem& q, int family, int colblock, int mo
       if (fills && grids[i] * 8 < up_to * q.cus) return false;
     }
     if (!q.is_bwd && family == LINREC_FAMILY_COLDRIFT && on_lines && q.seqlen < 4096 && round_and_a_bit(grids[i], 4)) return false;
-    if (s[i][0] > 1 && !q.is_bwd && !(half && on_lines) && leaves_much_idle(grids[i], 4)) continue;
+    if (s[i][0] > 1 && !q.is_bwd && !(half && (on_lines || (s[i][0] == 4 && q.elem_stride % 2 == 0))) && leaves_much_idle(grids[i], 4)) continue;
     if (fwd_pairs && (q.seqlen > 1920 && grids[2] >= (on_slots ? 3 : 2) * q.cus)) continue;
     // (a caller that can only give so much workspace is served by the kernels that need less)
     linrec_plan_t p;

@@ -58,7 +58,8 @@ def test_lanes_that_share_rows_take_the_kernels_that_know(dtype):
     try:
         seen = set()
         for batch, time, channels in [(8, 4096, 1024), (8, 4096, 1025), (8, 4096, 1026), (8, 4096, 1027), (23, 5000, 77), (4, 4096, 700),
-                                      (1, 11944, 2809), (1, 8326, 4022), (2, 40000, 222), (8, 4096, 175), (5, 777, 1001)]:
+                                      (1, 11944, 2809), (1, 8326, 4022), (2, 40000, 222), (8, 4096, 175), (5, 777, 1001),
+                                      (7, 2048, 192)]:
             for is_bwd in (0, 1):
                 p = nat.Plan()
                 if batch > 1:

@@ -58,3 +58,11 @@ def test_a_forward_on_whole_lines_that_makes_hardly_more_than_one_round():
         assert rows_of_a_lane(F32, batch, time, channels, False) == want, (batch, time, channels)
     for batch, time, channels, want in [(10, 13130, 64, 2), (14, 9272, 64, 2), (10, 7379, 128, 4), (15, 1040, 512, 4)]:
         assert rows_of_a_lane(BF16, batch, time, channels, False) == want, (batch, time, channels)
+
+
+@pytest.mark.parametrize("dtype", [F16, BF16])
+def test_16_bit_forwards_a_little_beyond_one_round_keep_four_rows(dtype):
+    """(of an even number of channels)"""
+    for batch, time, channels, want in [(8, 1323, 1584, 4), (29, 1079, 564, 4), (3, 1310, 4268, 4), (48, 3120, 112, 4), (34, 1277, 472, 4),
+                                        (8, 1275, 1812, 4), (5, 5584, 675, 2), (4, 38189, 121, 2)]:
+        assert rows_of_a_lane(dtype, batch, time, channels, False) == want, (batch, time, channels)
