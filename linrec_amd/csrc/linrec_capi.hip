@@ -766,7 +766,9 @@ int lookback_segments_plan(const Problem& q, int vec, int waves, int depth, int 
 // to 33/32 of the CUs (4 x 13107 x 160 260 workgroups of two rows 23.2, 1030 of one 26.2, 2 x 21845 x 192 258 23.9, 1026 26.1; but 5 x
 // 22595 x 64 267 39.0, 885 30.9; bf16 10 x 13130 x 64 156 of four rows 19.4, 260 of two 16.7).
 // The fp32 forward off the lines: two rows are no better than one from three rounds of workgroups on (30 x 1024 x 1500 135
-// against 122, 2 x 125567 x 222 166 against 156, 8192 x 1025 32.8 against 29.6; 8326 x 4022 91.6 against 93.1), four are from
+// against 122, 2 x 125567 x 222 166 against 156, 8192 x 1025 32.8 against 29.6; 8326 x 4022 91.6 against 93.1; but rows on 16 bytes
+// that make three quarters to all of one round 24 x 1980 x 144 216 workgroups 19.6 against 22.9, 6 x 5535 x 208 220 20.6 against 23.8,
+// 7 x 2883 x 328 21.7 against 24.1), four are from
 // about 1536 rows and two rounds on (23 x 25862 x 77 137.6, 151.3 and 161.4 with four, two and one; 2 x 166672 x 82 90, 99 and 88).
 // More than one row to a lane needs rows for more than half of its lanes, or the accesses and descriptors are mostly
 // padding (fp32 2 x 262144 x 32: 78 / 131 with two rows to a lane in the forward and four in the backward, 57 / 78 with one, 78 /
@@ -896,7 +898,8 @@ bool lookback_segments_choose(const Problem& q, int family, int colblock, int mo
     }
     if (!q.is_bwd && family == LINREC_FAMILY_COLDRIFT && on_lines && q.seqlen < 4096 && round_and_a_bit(grids[i], 4)) return false;
     if (s[i][0] > 1 && !q.is_bwd && !(half && (on_lines || (s[i][0] == 4 && q.elem_stride % 2 == 0))) && leaves_much_idle(grids[i], 4)) continue;
-    if (fwd_pairs && (q.seqlen > 1920 && grids[2] >= (on_slots ? 3 : 2) * q.cus)) continue;
+    const bool fills_a_round = on_slots && channels >= 64 && grids[i] * 4 >= 3 * q.cus && grids[i] <= q.cus;
+    if (fwd_pairs && !fills_a_round && (q.seqlen > 1920 && grids[2] >= (on_slots ? 3 : 2) * q.cus)) continue;
     // (a caller that can only give so much workspace is served by the kernels that need less)
     linrec_plan_t p;
     std::memset(&p, 0, sizeof(p));

@@ -66,3 +66,10 @@ def test_16_bit_forwards_a_little_beyond_one_round_keep_four_rows(dtype):
     for batch, time, channels, want in [(8, 1323, 1584, 4), (29, 1079, 564, 4), (3, 1310, 4268, 4), (48, 3120, 112, 4), (34, 1277, 472, 4),
                                         (8, 1275, 1812, 4), (5, 5584, 675, 2), (4, 38189, 121, 2)]:
         assert rows_of_a_lane(dtype, batch, time, channels, False) == want, (batch, time, channels)
+
+
+def test_single_precision_pairs_that_fill_one_round():
+    """Rows that start on 16 bytes but not on a line: two to a lane where that makes three quarters of a round to a whole one."""
+    for batch, time, channels, want in [(24, 1980, 144, 2), (6, 5535, 208, 2), (7, 2883, 328, 2), (2, 3912, 784, 2), (2, 3826, 912, 2),
+                                        (34, 2416, 80, 2), (8, 19774, 36, 1), (11, 7742, 104, 1), (4, 5961, 360, 1), (9, 4646, 100, 1)]:
+        assert rows_of_a_lane(F32, batch, time, channels, False) == want, (batch, time, channels)
