@@ -768,7 +768,9 @@ int lookback_segments_plan(const Problem& q, int vec, int waves, int depth, int 
 // The fp32 forward off the lines: two rows are no better than one from three rounds of workgroups on (30 x 1024 x 1500 135
 // against 122, 2 x 125567 x 222 166 against 156, 8192 x 1025 32.8 against 29.6; 8326 x 4022 91.6 against 93.1; but rows on 16 bytes
 // that make three quarters to all of one round 24 x 1980 x 144 216 workgroups 19.6 against 22.9, 6 x 5535 x 208 220 20.6 against 23.8,
-// 7 x 2883 x 328 21.7 against 24.1), four are from
+// 7 x 2883 x 328 21.7 against 24.1, and up to 1024 rows in batches of an even number of channels that waste no lanes of two rows
+// 2 x 611013 x 54 188 against 225, 3 x 368823 x 30 123 against 137, 8 x 57222 x 126 183 against 194; 2 x 97138 x 172 and 4 x 170534 x 24
+// the same, with half the lanes wasted 2 x 256555 x 76 0.85, 8 x 258805 x 24 0.81), four are from
 // about 1536 rows and two rounds on (23 x 25862 x 77 137.6, 151.3 and 161.4 with four, two and one; 2 x 166672 x 82 90, 99 and 88).
 // More than one row to a lane needs rows for more than half of its lanes, or the accesses and descriptors are mostly
 // padding (fp32 2 x 262144 x 32: 78 / 131 with two rows to a lane in the forward and four in the backward, 57 / 78 with one, 78 /
@@ -899,7 +901,8 @@ bool lookback_segments_choose(const Problem& q, int family, int colblock, int mo
     if (!q.is_bwd && family == LINREC_FAMILY_COLDRIFT && on_lines && q.seqlen < 4096 && round_and_a_bit(grids[i], 4)) return false;
     if (s[i][0] > 1 && !q.is_bwd && !(half && (on_lines || (s[i][0] == 4 && q.elem_stride % 2 == 0))) && leaves_much_idle(grids[i], 4)) continue;
     const bool fills_a_round = on_slots && channels >= 64 && grids[i] * 4 >= 3 * q.cus && grids[i] <= q.cus;
-    if (fwd_pairs && !fills_a_round && (q.seqlen > 1920 && grids[2] >= (on_slots ? 3 : 2) * q.cus)) continue;
+    const bool few_blocks = q.batched() && channels % 2 == 0 && q.numseq <= q.at(1024) && grids[i] > q.cus && grids[2] * 10 >= grids[i] * 39;
+    if (fwd_pairs && !fills_a_round && !few_blocks && (q.seqlen > 1920 && grids[2] >= (on_slots ? 3 : 2) * q.cus)) continue;
     // (a caller that can only give so much workspace is served by the kernels that need less)
     linrec_plan_t p;
     std::memset(&p, 0, sizeof(p));

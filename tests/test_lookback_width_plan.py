@@ -73,3 +73,11 @@ def test_single_precision_pairs_that_fill_one_round():
     for batch, time, channels, want in [(24, 1980, 144, 2), (6, 5535, 208, 2), (7, 2883, 328, 2), (2, 3912, 784, 2), (2, 3826, 912, 2),
                                         (34, 2416, 80, 2), (8, 19774, 36, 1), (11, 7742, 104, 1), (4, 5961, 360, 1), (9, 4646, 100, 1)]:
         assert rows_of_a_lane(F32, batch, time, channels, False) == want, (batch, time, channels)
+
+
+def test_single_precision_pairs_of_few_rows():
+    """Up to 1024 rows of an even number of channels, where one row to a lane would take four times the workgroups."""
+    for batch, time, channels, want in [(2, 611013, 54, 2), (2, 659408, 42, 2), (2, 390360, 42, 2), (3, 368823, 30, 2), (2, 176680, 126, 2),
+                                        (8, 57222, 126, 2), (3, 690000, 24, 2), (2, 256555, 76, 1), (8, 258805, 24, 1), (3, 103563, 27, 1),
+                                        (17, 36332, 24, 1)]:
+        assert rows_of_a_lane(F32, batch, time, channels, False) == want, (batch, time, channels)
