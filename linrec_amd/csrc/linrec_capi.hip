@@ -777,7 +777,8 @@ int lookback_segments_plan(const Problem& q, int vec, int waves, int depth, int 
 // 102 in three launches; bf16 2 x 262144 x 16 72 / 93, 48 / 58 and 50 / 76), and lanes that lie next to each other: batches of at
 // least 24 channels (fp32 500 x 2000 x 8 42 / 92, 42 / 99 and 30 / 65 with two, four and one; bf16 8 x 262144 x 16 127 / 206,
 // 106 / 161 and 147 / 264 in three launches).  Lanes whose rows do not start on the size of an access, or lie in two batches, take a
-// line more for every batch that a wave spans: at least 64 channels, 80 in 16-bit storage (12 million elements, one row to a
+// line more for every batch that a wave spans: at least 64 channels, 80 in 16-bit storage and for four rows in the fp32
+// backward (28 x 3768 x 74 two rows 51.9, four 56.7, 4 x 214903 x 66 374, 407, 27 x 25043 x 66 306, 331; 12 million elements, one row to a
 // lane / two / four, and what accesses to whole slots had taken, backward: bf16 461 x 1000 x 26 68 / 75 / 107, 87, 324 x 1000 x 37 64 /
 // 81 / 86, 78, 206 x 1000 x 58 60 / 60 / 64, 66, 160 x 1000 x 75 62 / 64 / 67, 80, 133 x 1000 x 90 61 / 56 / 53, 62, fp32 461 x 1000 x 26
 // 90 / 87 / 130, 108, 324 x 1000 x 37 95 / 103 / 116, 120, 240 x 1000 x 50 90 / 78 / 92, 92, 181 x 1000 x 66 95 / 79 / 87, 92; forward bf16
@@ -856,7 +857,7 @@ bool lookback_segments_choose(const Problem& q, int family, int colblock, int mo
     if (s[i][0] == 1) continue;
     const int64_t lanes = ceil_div(lookback_lanes(q, s[i][0]), 64) * 64;  // of a segment, with and without a row
     const bool aligned = colblock_rows_per_lane(q, s[i][0]) == s[i][0];  // (never across a batch, on the size of the access)
-    if (q.numseq * 2 <= lanes * s[i][0] || (q.batched() && channels < (aligned ? 24 : half ? 80 : 64))) fits[i] = false;
+    if (q.numseq * 2 <= lanes * s[i][0] || (q.batched() && channels < (aligned ? 24 : half || (q.is_bwd && s[i][0] == 4) ? 80 : 64))) fits[i] = false;
   }
   auto round_and_a_bit = [&](int64_t grid, int64_t sixteenths) { return grid > q.cus && grid * 16 <= q.cus * (16 + sixteenths); };
   auto leaves_much_idle = [&](int64_t grid, int64_t sixteenths) {

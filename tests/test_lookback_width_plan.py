@@ -81,3 +81,9 @@ def test_single_precision_pairs_of_few_rows():
                                         (8, 57222, 126, 2), (3, 690000, 24, 2), (2, 256555, 76, 1), (8, 258805, 24, 1), (3, 103563, 27, 1),
                                         (17, 36332, 24, 1)]:
         assert rows_of_a_lane(F32, batch, time, channels, False) == want, (batch, time, channels)
+
+
+def test_single_precision_backwards_of_64_to_80_channels_take_pairs():
+    for batch, time, channels in [(28, 3768, 74), (4, 214903, 66), (55, 1955, 78), (56, 2269, 66), (27, 25043, 66), (7, 17119, 70)]:
+        assert rows_of_a_lane(F32, batch, time, channels, True) == 2, (batch, time, channels)
+    assert rows_of_a_lane(F32, 28, 3768, 72, True) == 4 and rows_of_a_lane(F32, 28, 3768, 82, True) == 4
