@@ -904,6 +904,12 @@ bool lookback_segments_choose(const Problem& q, int family, int colblock, int mo
     const bool fills_a_round = on_slots && channels >= 64 && grids[i] * 4 >= 3 * q.cus && grids[i] <= q.cus;
     const bool few_blocks = q.batched() && channels % 2 == 0 && q.numseq <= q.at(1024) && grids[i] > q.cus && grids[2] * 10 >= grids[i] * 39;
     if (fwd_pairs && !fills_a_round && !few_blocks && (q.seqlen > 1920 && grids[2] >= (on_slots ? 3 : 2) * q.cus)) continue;
+    // Column drift teams keep 16-bit backwards of single matrices of less than 4096 rows that fill most of the chip in one round,
+    // where the segments would take two rows to a lane or make a little more than one round (4864 x 3772 59.0 against
+    // 51.5, 4894 x 3540 56.4 against 48.6, 2048 x 3676 26.0 against 23.4; but 9131 x 4036 0.92, 3390 x 3812 0.90).
+    if (!q.batched() && half && q.is_bwd && family == LINREC_FAMILY_COLDRIFT && q.numseq < q.at(4096) &&
+        (s[i][0] == 2 || round_and_a_bit(grids[i], 2)))
+      return false;
     // (a caller that can only give so much workspace is served by the kernels that need less)
     linrec_plan_t p;
     std::memset(&p, 0, sizeof(p));

@@ -23,6 +23,12 @@ def rows_of_a_lane(dtype, batch, time, channels, is_bwd):
     return p.vec if p.family == nat.FAMILY_SEGMENT and p.carry == 1 else 0
 
 
+def rows_of_a_lane_of_one_matrix(dtype, time, channels, is_bwd):
+    p = nat.Plan()
+    assert nat.lib().linrec_plan(dtype, None, channels, time, 1, channels, 0, int(is_bwd), None, ctypes.byref(p)) == 0
+    return p.vec if p.family == nat.FAMILY_SEGMENT and p.carry == 1 else 0
+
+
 @pytest.mark.parametrize("dtype", [F32, F16, BF16])
 @pytest.mark.parametrize("is_bwd", [False, True])
 def test_lanes_of_narrow_batches_take_rows_that_start_on_an_access(dtype, is_bwd):
@@ -87,3 +93,10 @@ def test_single_precision_backwards_of_64_to_80_channels_take_pairs():
     for batch, time, channels in [(28, 3768, 74), (4, 214903, 66), (55, 1955, 78), (56, 2269, 66), (27, 25043, 66), (7, 17119, 70)]:
         assert rows_of_a_lane(F32, batch, time, channels, True) == 2, (batch, time, channels)
     assert rows_of_a_lane(F32, 28, 3768, 72, True) == 4 and rows_of_a_lane(F32, 28, 3768, 82, True) == 4
+
+
+@pytest.mark.parametrize("dtype", [F16, BF16])
+def test_16_bit_backwards_of_one_matrix_that_drift_teams_serve_in_one_round(dtype):
+    for time, channels, want in [(4864, 3772, 0), (4894, 3540, 0), (2048, 3676, 0), (3390, 3812, 4), (8895, 3772, 4), (9131, 4036, 4),
+                                 (2368, 7084, 4)]:
+        assert rows_of_a_lane_of_one_matrix(dtype, time, channels, True) == want, (time, channels)
