@@ -833,9 +833,10 @@ bool lookback_segments_choose(const Problem& q, int family, int colblock, int mo
     // against 74 / 140)
     const bool many = !on_slots && q.numseq > q.at(32768) && q.numseq <= q.at(65536);
     if (family == LINREC_FAMILY_COLUMN && !many && (!colblock || !half || q.seqlen <= 1024)) return false;
-    // Few rows over the longest axes, as above: backward 2^17 x 2 fp32 31.9 against 27.6, 2^19 x 32 112 against 103, 2^20 x 16
+    // Few rows over the longest axes, as above: 495094 x 16 bf16 forward 68.3 against 56.8, fp32 backward 99.7 against 85.9, 429270 x
+    // 12 60.5 against 54.2 (415453 x 32 the same); backward 2^17 x 2 fp32 31.9 against 27.6, 2^19 x 32 112 against 103, 2^20 x 16
     // bf16 143 / 185 against 87 / 125.
-    if (q.numseq < 64 && q.seqlen >= (q.numseq <= 8 ? 131072 : 524288)) return false;
+    if (q.numseq < 64 && q.seqlen >= (q.numseq <= 8 ? 131072 : q.numseq <= 16 ? 425984 : 524288)) return false;
   }
   if (!q.is_bwd && colblock && q.seqlen < (on_lines ? 1024 : 704)) return false;
   if (half && q.is_bwd && colblock == 2 && q.seqlen < (on_lines || channels < 32 ? 352 : 264)) return false;

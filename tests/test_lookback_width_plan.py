@@ -100,3 +100,13 @@ def test_16_bit_backwards_of_one_matrix_that_drift_teams_serve_in_one_round(dtyp
     for time, channels, want in [(4864, 3772, 0), (4894, 3540, 0), (2048, 3676, 0), (3390, 3812, 4), (8895, 3772, 4), (9131, 4036, 4),
                                  (2368, 7084, 4)]:
         assert rows_of_a_lane_of_one_matrix(dtype, time, channels, True) == want, (time, channels)
+
+
+@pytest.mark.parametrize("dtype", [F32, F16, BF16])
+def test_sixteen_rows_of_one_matrix_over_the_longest_axes(dtype):
+    for time, channels, is_bwd, want in [(495094, 16, True, 0), (482545, 16, True, 0), (440210, 12, True, 0), (430000, 9, True, 0),
+                                         (415453, 32, True, 1), (400000, 16, True, 1), (400000, 12, True, 1)]:
+        assert rows_of_a_lane_of_one_matrix(dtype, time, channels, is_bwd) == want, (time, channels)
+    if dtype != F32:
+        for time, channels in [(495094, 16), (440210, 12), (429270, 12), (434490, 11)]:
+            assert rows_of_a_lane_of_one_matrix(dtype, time, channels, False) == 0, (time, channels)
