@@ -676,16 +676,6 @@ int64_t lookback_lanes(const Problem& q, int64_t vec) {
 int lookback_form(const Problem& q, int64_t vec) {
   return (q.batched() ? q.rows_per_batch : q.numseq) % vec ? linrec::PHASE_LOOKBACK_SHARED : linrec::PHASE_LOOKBACK;
 }
-// Segments dealt out at a time (collook_kernel.hpp): eight where that is as good or better, whole groups of which there are
-// at least two.  Forward / backward in us, eight against one: off the 128-byte lines fp32 8326 x 4022 (time x channels) 91.6 /
-// 140.7 against 98.0 / 150.2, 2 x 125567 x 222 165.9 / 244 against 172.4 / 251, bf16 8 x 4096 x 700 40.6 / 69.0 against 42.9 /
-// 73.2, but 3 x 1813 x 1464 (eight segments) 33.7 against 28.0; on them fp32 32768 x 1024 79.9 / 122.8 against 82.9 / 129.7,
-// 16 x 2048 x 512 43.6 / 66.8 against 39.5 / 69.5, bf16 32768 x 1024 47.6 / 67.6 against 44.4 / 68.8, of two blocks fp32
-// 16384 x 512 24.2 / 33.9 against 22.3 / 32.6.
-int64_t lookback_segments_at_once(const Problem& q, int64_t blocks, int64_t segments) {
-  const bool on_lines = q.elem_stride * elem_size_of(q.dtype) % 128 == 0;
-  return segments >= 16 && (on_lines ? q.is_bwd && blocks >= 4 : blocks >= 2) ? 8 : 1;
-}
 // Workgroups of such a launch, without a look at the kernel table; negative: LINREC_E_UNSUPPORTED or LINREC_E_TOO_LARGE.
 int64_t lookback_segments_grid(const Problem& q, int vec, int waves, int depth) {
   if (vec < 1 || colblock_rows_per_lane(q, 1) != 1) return LINREC_E_UNSUPPORTED;
@@ -1716,7 +1706,7 @@ int launch(const linrec_plan_t& plan, const Problem& q, const void* in0, const v
     linrec::ColDriftArgs d{};
     d.col = a;
     d.col.lanes_per_segment = lanes;
-    d.chain.row_groups = lookback_segments_at_once(q, blocks, plan.tiles_per_row);
+    d.chain.row_groups = linrec::lookback_segments_at_once(q.elem_stride * elem_size_of(q.dtype) % 128 == 0, q.is_bwd, q.dtype != LINREC_DTYPE_F32, blocks, plan.tiles_per_row);
     d.chain.num_tiles = plan.grid;
     d.chain.tasks = int(blocks);
     d.chain.ws = static_cast<linrec::CarryHeader*>(workspace);

@@ -52,6 +52,24 @@ def test_every_row_is_stored_by_one_lane(program, vec):
                 assert got.returncode == 0, (batches, rows, vec, got.returncode, got.stdout)
 
 
+AT_ONCE = r"""
+#include "lookback_lanes.hpp"
+using linrec::lookback_segments_at_once;
+constexpr bool LINES = true, BWD = true, HALF = true;
+static_assert(lookback_segments_at_once(LINES, BWD, HALF, 33, 16) == 1, "16-bit backwards of many blocks take one segment after the other");
+static_assert(lookback_segments_at_once(LINES, BWD, HALF, 16, 100) == 1 && lookback_segments_at_once(LINES, BWD, HALF, 15, 100) == 8);
+static_assert(lookback_segments_at_once(LINES, BWD, HALF, 4, 16) == 8 && lookback_segments_at_once(LINES, BWD, HALF, 3, 16) == 1);
+static_assert(lookback_segments_at_once(LINES, BWD, !HALF, 33, 16) == 8 && lookback_segments_at_once(LINES, !BWD, !HALF, 33, 16) == 1);
+static_assert(lookback_segments_at_once(!LINES, BWD, HALF, 33, 16) == 8 && lookback_segments_at_once(!LINES, !BWD, HALF, 2, 16) == 8);
+static_assert(lookback_segments_at_once(!LINES, BWD, HALF, 33, 15) == 1 && lookback_segments_at_once(!LINES, BWD, HALF, 1, 100) == 1);
+"""
+
+
+def test_segments_dealt_out_at_a_time(tmp_path):
+    (tmp_path / "at_once.cpp").write_text(AT_ONCE)
+    subprocess.run(["g++", "-std=c++17", "-fsyntax-only", "-I", CSRC, str(tmp_path / "at_once.cpp")], check=True)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 def test_lanes_that_share_rows_take_the_kernels_that_know(dtype):
     old = nat.set_compute_units(256)
