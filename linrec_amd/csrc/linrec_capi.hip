@@ -942,7 +942,9 @@ Problem tail_problem(const Problem& q, int64_t tail_rows) {
 // eighths 0.99 / 1.03, 11/16 1.03 / 1.08, three quarters 1.05 / 1.05, 7/8 1.02 / 1.05, bf16 1944 x 3392 9.5 against 8.2, backward 3728 x 1792 15.8
 // against 13.4; fp32 three quarters to all 0.99 / 0.99 with single lengths up to 1.12, 1584 backward 2^23 31.2 against 27.8; of
 // less than 1.5 times the least size 9/16 and more 1.04); nor in the 16-bit backward rows off the slots from 7/8 on (1.06 against
-// the form of the tile kernels that masks late; the forward 1.01).  Nor the backward of
+// the form of the tile kernels that masks late; the forward 1.01).  Nor where workgroups of eight waves make about one round in
+// 16-bit storage (forward from one round to ten eighths 1.02, f16 2430 x 3524 13.2 against 12.3; backward from six to nine eighths 1.03,
+// 1707 x 3436 16.5 against 12.7, 1908 x 3325 16.5 against 13.5; less and more 0.86 to 0.98).  Nor the backward of
 // large tensors where one slot to a lane does (1001: 117.9 against 112.9; bf16 2001: 62.9 against 61.1; at 2^23 1001 30.9
 // against 32.0), nor the large backward of a few floats (5: 116.1 against 113.8).
 bool packed_plan(const Problem& q, int fv, int mode, int desc, int64_t row_slots, int64_t tile_slots, linrec_plan_t* out) {
@@ -965,6 +967,10 @@ bool packed_plan(const Problem& q, int fv, int mode, int desc, int64_t row_slots
     if (rows < 2 || rows * q.seqlen * 5 < room * 4) continue;
     const int id = find_kernel(q.dtype, LINREC_FAMILY_TILE, waves, 2, fv, mode, desc, 4);
     if (id < 0 || ceil_div(q.numseq, rows) > 2147483647LL) return false;
+    // 16-bit storage, eight waves: about one round of workgroups (of which a CU holds four, in the backward, whose 69
+    // registers are too many for that, three) or a few more
+    const int64_t eighths = ceil_div(q.numseq, rows) * waves * 8 / (32 * q.cus);
+    if (half && tile_slots > 0 && waves == 8 && eighths >= (q.is_bwd ? 6 : 8) && eighths <= (q.is_bwd ? 8 : 9)) return false;
     out->family = LINREC_FAMILY_TILE;
     out->waves = waves; out->slots = 2; out->vec = fv; out->carry = 0;
     out->tiles_per_row = 1;

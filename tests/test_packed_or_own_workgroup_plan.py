@@ -37,7 +37,7 @@ def test_16_bit_rows_of_whole_slots_that_fill_their_workgroup(dtype):
 @pytest.mark.parametrize("dtype", [F16, BF16])
 def test_16_bit_backward_of_rows_off_the_slots(dtype):
     for room in (1024, 2048, 4096):
-        for rows in ((1 << 23) // room, (1 << 26) // room):
+        for rows in ((1 << 24) // room, (1 << 26) // room):
             assert packed(dtype, rows, room * 13 // 16 + 1, True) and packed(dtype, rows, room * 15 // 16 + 1, False), (rows, room)
             assert not packed(dtype, rows, room * 15 // 16 + 1, True), (rows, room)
 
@@ -52,3 +52,12 @@ def test_single_precision_rows_of_whole_slots(is_bwd):
         length = room * 10 // 16
         assert not packed(F32, (1 << 22) // length + 1, length, is_bwd), room  # little work
     assert not packed(F32, 4849, 1584, True) and not packed(F32, 22657, 192, False)
+
+
+@pytest.mark.parametrize("dtype", [F16, BF16])
+def test_16_bit_workgroups_of_eight_waves_that_make_about_one_round(dtype):
+    """(a compute unit holds four of them, three in the backward)"""
+    for rows, length, is_bwd in [(1707, 3436, True), (1908, 3325, True), (1698, 3353, True), (2200, 3524, False), (2430, 3524, False)]:
+        assert not packed(dtype, rows, length, is_bwd), (rows, length)
+    for rows, length, is_bwd in [(1300, 3436, True), (4000, 3325, True), (1300, 3427, False), (6000, 3427, False)]:
+        assert packed(dtype, rows, length, is_bwd), (rows, length)
