@@ -946,7 +946,10 @@ Problem tail_problem(const Problem& q, int64_t tail_rows) {
 // 16-bit storage (forward from one round to ten eighths 1.02, f16 2430 x 3524 13.2 against 12.3; backward from six to nine eighths 1.03,
 // 1707 x 3436 16.5 against 12.7, 1908 x 3325 16.5 against 13.5; less and more 0.86 to 0.98).  Nor the backward of
 // large tensors where one slot to a lane does (1001: 117.9 against 112.9; bf16 2001: 62.9 against 61.1; at 2^23 1001 30.9
-// against 32.0), nor the large backward of a few floats (5: 116.1 against 113.8).
+// against 32.0), nor the large backward of a few floats (5: 116.1 against 113.8), nor the fp32
+// backward of a scan that ran in reverse, whose flat kernels read rows in ascending order (less than 16 floats 1.04 in the geometric
+// mean, 9 x 3728270 124.0 against 115.3; less than 64 from 2^23 elements on 1.03, 35 x 1232460 162.5 against 153.0, before that 1.00;
+// in descending order 0.92 and 0.89).
 bool packed_plan(const Problem& q, int fv, int mode, int desc, int64_t row_slots, int64_t tile_slots, linrec_plan_t* out) {
   if (q.base_mis < 0 || q.elem_stride != 1 || q.numseq < 2 || q.row_stride != q.seqlen || q.batched() || q.seqlen < fv) return false;
   const bool half = q.dtype != LINREC_DTYPE_F32;
@@ -961,6 +964,7 @@ bool packed_plan(const Problem& q, int fv, int mode, int desc, int64_t row_slots
   if (q.is_bwd && elements >= 65536 * q.cus && tile_slots > 64 && tile_slots <= 256 && row_slots * 100 >= tile_slots * 98) return false;
   const bool large = elements >= 131072 * q.cus;
   if (q.is_bwd && !half && large && q.seqlen < 16) return false;
+  if (q.is_bwd && !half && tile_slots == 0 && !desc && q.seqlen < (elements < 32768 * q.cus ? 16 : 64)) return false;
   for (int waves = !large || (half && !q.is_bwd) ? 4 : half || !q.is_bwd ? 8 : 16; waves <= (half || !q.is_bwd ? 8 : 16); waves *= 2) {
     const int64_t room = int64_t(waves) * 2 * 64 * fv;
     const int64_t rows = (room - (ragged ? fv - 1 : 0)) / q.seqlen;

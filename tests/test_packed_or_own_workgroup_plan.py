@@ -15,9 +15,9 @@ def full_part():
     nat.set_compute_units(old)
 
 
-def packed(dtype, rows, length, is_bwd):
+def packed(dtype, rows, length, is_bwd, reverse=0):
     p = nat.Plan()
-    assert nat.lib().linrec_plan(dtype, None, rows, length, length, 1, 0, int(is_bwd), None, ctypes.byref(p)) == 0
+    assert nat.lib().linrec_plan(dtype, None, rows, length, length, 1, reverse, int(is_bwd), None, ctypes.byref(p)) == 0
     return "packed" in nat.kernel_table()[p.kernel_id]
 
 
@@ -61,3 +61,16 @@ def test_16_bit_workgroups_of_eight_waves_that_make_about_one_round(dtype):
         assert not packed(dtype, rows, length, is_bwd), (rows, length)
     for rows, length, is_bwd in [(1300, 3436, True), (4000, 3325, True), (1300, 3427, False), (6000, 3427, False)]:
         assert packed(dtype, rows, length, is_bwd), (rows, length)
+
+
+def test_single_precision_backward_of_short_rows_that_ran_in_reverse():
+    """(its scan runs in ascending order, in which the flat kernels are ahead)"""
+    for length in (5, 7, 9, 13, 15, 21, 35, 45, 63):
+        for elements in (1 << 22, 1 << 23, 1 << 24, 30 << 20):
+            rows = elements // length + 1
+            flat = length < 16 or elements > 1 << 22
+            assert packed(F32, rows, length, True, reverse=1) == (not flat), (rows, length)
+            assert packed(F32, rows, length, True, reverse=0) and packed(F32, rows, length, False, reverse=1), (rows, length)
+            if length > 8:
+                assert packed(BF16, rows, length, True, reverse=1), (rows, length)
+    assert packed(F32, (1 << 24) // 101, 101, True, reverse=1)
