@@ -396,7 +396,7 @@ int drift_slots_for(const Problem& q, int fv) {
     if (skewed && !drift_skewed_pays(q)) continue;
     const int64_t tiles_per_row = q.seqlen / tile;  // (full ones)
     const int64_t all_tiles = drift_tiles_per_row(q, fv, tile);
-    const int64_t team = drift_team_size(q, all_tiles, 8, q.cus, ragged);
+    const int64_t team = drift_team_size(q, tiles_per_row + ragged, 8, q.cus, ragged);  // (the launch's own goes by all its tiles)
     // the forward's tiles of 8192 elements: as many tiles a row as the generated table says, and from its number of
     // rows on also rows of two tiles in teams of two (us, against one workgroup per row: 2048 x 16384 66.2 against 69.3,
     // 4096 x 16384 128.9 against 138.8; but 600 x 16384 22.6 against 22.1, 1024 x 16384 34.5 against 35.0)

@@ -63,3 +63,13 @@ def test_rows_of_as_many_tiles_take_the_same_launch():
                 assert [a[k] for k in keys] == [b[k] for k in keys], (rows, tiles, a, b)
                 seen.add((a["waves"], a["tasks"] > 64))
     assert {(16, False), (8, True)} <= seen, seen
+
+
+def test_a_tile_more_does_not_send_rows_elsewhere():
+    """Whether drift teams serve rows at any phase is decided by the length alone; their teams may be smaller than four where
+    the last slot's tile leaves them nothing better."""
+    for cus, rows, length, stride in [(6, 4, 57342, 57343), (6, 4, 57341, 57343), (256, 171, 57342, 57343), (256, 300, 65541, 65541)]:
+        nat.set_compute_units(cus)
+        p = nat.Plan()
+        assert nat.lib().linrec_plan(0, None, rows, length, stride, 1, 0, 1, None, ctypes.byref(p)) == 0
+        assert "drift_skewed" in nat.kernel_table()[p.kernel_id], (cus, rows, length)
