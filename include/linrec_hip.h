@@ -79,7 +79,9 @@ extern "C" {
                                   The planner's picks are the 16-wave ones, and 8 x 4 forward for fp32 teams beyond 64.
                                   Rows must be whole tiles; rows of whole 16-byte slots may end in a partial tile
                                   (fp32 forward 16 x 2 and 8 x 4, backward 16 x 1; 16-bit storage forward 16 x 2,
-                                  backward 8 x 2), and their teams need not divide the tiles of a row */
+                                  backward 8 x 2), and their teams need not divide the tiles of a row.
+                                  fp32 rows that start or end inside a slot take forms of the same geometries by
+                                  the planner's choice only: a caller who names the family is refused them */
 
 #define LINREC_FAMILY_COLDRIFT 11 /* as COLUMN in its block form for a few hundred to a few thousand rows: teams
                                    of workgroups share a block of rows and take its steps along the scan axis in

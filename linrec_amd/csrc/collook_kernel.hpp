@@ -20,7 +20,7 @@
 // through the caches, and eight segments are dealt out at a time so that the blocks of a segment run on one XCD and
 // find the border lines in its L2 (memory-only, 16640 x 4022, 8 bytes to a lane: 101.7 us as before, 93 with cached loads,
 // 85 with both; where positions start on lines cached loads cost 4 %).  That order also serves backwards on whole
-// lines (fp32 32768 x 1024 123 us instead of 130, 16384 x 4096 233 instead of 247), not forwards (16 x 2048 x 512 43.6
+// lines (fp32 32768 x 1024 123 us instead of 130, 16384 x 4096 233 instead of 247; not 16-bit ones of many blocks), not forwards (16 x 2048 x 512 43.6
 // instead of 39.5).
 //
 // Measured (medians of launches replayed from a graph over several buffer sets, forward / backward): bf16 1 x 4096 x 2048
@@ -185,7 +185,8 @@ __global__ __launch_bounds__(64 * NW) void collook_kernel(ColDriftArgs args) {
     Held<T, VEC> x[U], c[U], yn[NEED_Y ? U : 1];
   };
   const int n0 = k * STEP + wave * U;
-  // positions a whole number of 128-byte lines apart: no line is wanted twice
+  // positions a whole number of 128-byte lines apart: no line is wanted twice if the base starts on one too (what torch allocates
+  // does; a view that does not reads its border lines twice, as it would without this)
   const bool on_lines = p.elem_stride * (long long)sizeof(T) % 128 == 0;
   // FULL: all positions of the segment exist and, for the backward, so does the last one's successor.  OWN: some of the
   // block's lanes store part of their rows only.

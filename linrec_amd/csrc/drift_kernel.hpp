@@ -40,13 +40,14 @@ namespace linrec {
 // one and two steps from now) and the tiles of loaded data change roles without a register being copied.
 // PF: tiles of loads in flight ahead of the scan (1 or 2); WPE: waves per SIMD the compiler is to allow for;
 // WIDE: teams of more than 64 are served (the forward with 16 waves of two slots has no registers for that).
-// RAGGED: rows of whole slots whose last tile is a partial one (K = tiles of a row, the last one counted): that
-// tile takes the loads and stores that look at every slot, the others stay as they are; the team need not divide K,
+// RAGGED: rows of whole slots whose last tile is a partial one (K = tiles of a row, the last one counted): its loads look
+// at every slot (the fp32 backward's are whole slots, masked when the tile's turn has come), and so do its stores, the
+// other tiles stay as they are; the team need not divide K,
 // and the walk's start moves on by K % M tiles in every row, so that neither the partial tiles nor the longer walks
 // all fall to the same team mates.
 // SKEWED (fp32, with RAGGED): rows that start or end inside a slot, each at its own phase (RowView per row).  The waves
-// that hold a row's first or last slot take the loads and stores that look at every slot, all others whole slots as
-// before; a row's last tile may hold no slot of it at all, and is the identity then.  335 x 100001 backward 120.4 us, 5.6
+// that hold a row's first or last slot mask what they loaded as whole slots when its turn has come and store slot by
+// slot, all others whole slots as before; a row's last tile may hold no slot of it at all, and is the identity then.  335 x 100001 backward 120.4 us, 5.6
 // TB/s, where look-back tiles of 16384 elements take 135.5 (one workgroup per CU and its waits); 100 x 250001 57.3 / 91.3
 // where one team per row takes 66.6 / 105.8.  Rows that start on a slot (335 x 100000 73.7 / 115.7) move the same bytes: what
 // is left is the launch shape's, see above.
@@ -70,7 +71,7 @@ __global__ __launch_bounds__(64 * NW, WPE) void drift_kernel(TileArgs p) {
   const int lane = threadIdx.x & 63;
   const int wave = NW == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int M = p.tasks;          // team size; divides K unless RAGGED
-  const int K = p.tiles_per_row;  // every row is exactly K full tiles
+  const int K = p.tiles_per_row;  // every row is exactly K full tiles, the last one partial or empty where RAGGED
   const int teams = int(p.row_groups);  // the grid is teams * M workgroups
   const int team = int(blockIdx.x) / M;
   const int j = int(blockIdx.x) - team * M;

@@ -1,5 +1,4 @@
-// Packed tiles: dense rows (no gaps between them) of more than a wave's worth of elements, several whole rows to a
-// workgroup.  One row to a workgroup leaves the lanes between the row's end and the tile's idle (a row of 333 floats
+// Packed tiles: dense rows (no gaps between them) of a slot and more, several whole rows to a workgroup.  One row to a workgroup leaves the lanes between the row's end and the tile's idle (a row of 333 floats
 // takes 84 or 85 slots of 128), and rows that are not whole slots make every wave look at every slot.  Here a workgroup
 // takes `tasks` consecutive rows as one array: slots are whole except the first and the last of the workgroup, all
 // lanes but those of the last row's remainder have work, and the scan is cut at the row starts.

@@ -63,7 +63,7 @@ __global__ __launch_bounds__(64 * NW) void stream_kernel(TileArgs p) {
 #define LINREC_ROW_STAMP(i, v) do { } while (0)
 #endif
 
-  // A tile with ragged or missing slots, already in registers (loaded through the predicated path).
+  // A tile with ragged or missing slots, already in registers and masked.
   auto edge_finish = [&](int t, const TileData<S, VEC, MODE>& d) {
     const int u_wave = t * TILE_SLOTS + wave * WAVE_SLOTS;
     TileScan<S, VEC> r;

@@ -176,7 +176,8 @@ __device__ __forceinline__ void signal_tile_done_end(const TileArgs& p, long lon
 // without it such a wave looks at every slot and waits for one load after the other where slots lie partly in the row.
 // For rows that start or end inside a slot, forward / backward in us, without and with: fp32 2^23 elements in rows of 1001
 // 20.2 / 32.3 and 18.8 / 31.0, 3001 20.6 / 34.0 and 18.9 / 31.6, 2^18 in rows of 2001 4.6 / 5.7 and 3.6 / 4.3; bf16 2^25 in rows of 5001 40.0 /
-// 70.7 and 35.2 / 59.6, 2^21 of 3001 6.2 / 8.6 and 5.2 / 6.6.
+// 70.7 and 35.2 / 59.6, 2^21 of 3001 6.2 / 8.6 and 5.2 / 6.6.  In the 16-bit backward of two slots to a lane it takes 72 to 74
+// registers instead of 62 to 64 (held to 64 it spills 16 to 20 of them): the planner knows where that costs more (late_masks_pay).
 template <typename T, int NW, int S, int VEC, int MODE, bool DESC, bool CARRY, bool ENDS = false>
 __global__ __launch_bounds__(64 * NW) void tile_kernel(TileArgs p) {
   static_assert(!ENDS || VEC > 1, "whole slots");

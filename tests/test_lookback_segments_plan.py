@@ -133,6 +133,33 @@ def test_a_lane_is_less_than_2_31_bytes_from_its_wave(dtype, channels):
     assert wide is not None and not chained(wide)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("is_bwd", [False, True])
+def test_the_same_where_lanes_share_rows(dtype, is_bwd):
+    """Channels that are no multiple of the rows of a lane, which the planner alone takes: a batch's last lane starts early.
+    The first batch stride beyond the bound is served otherwise."""
+    size, time, seen = torch.empty(0, dtype=dtype).element_size(), 4096, set()
+    for batch, channels in ((8, 1025), (8, 1026), (8, 2809), (8, 222), (40, 83), (64, 101)):
+        def wide(stride):
+            p = plan(dtype, batch, time, channels, is_bwd, batch_stride=stride)
+            return p["vec"] if p is not None and chained(p) and channels % p["vec"] else 0
+        low = time * channels
+        if not wide(low):
+            continue
+        vec, high = wide(low), 1 << 40
+        while high - low > 1:  # (the stride alone does not change the rows of a lane but where one is refused)
+            mid = (low + high) // 2
+            low, high = (mid, high) if wide(mid) == vec else (low, mid)
+        lanes = -(-channels // vec)
+        offset = lambda lane: lane // lanes * low + min(lane % lanes * vec, channels - vec)
+        blocks = range(0, batch * lanes, 64)
+        worst = max((offset(min(b + 64, batch * lanes) - 1) - offset(b) + vec) * size for b in blocks)
+        assert worst < 1 << 31, (batch, channels, vec, low, worst)
+        assert lanes >= 64 or worst > 1 << 28, (batch, channels, vec, low, worst)
+        seen.add(vec)
+    assert 4 in seen, seen
+
+
 def test_strides_that_run_backwards_or_batches_that_overlap_are_refused():
     tuning = nat.Tuning(S, 1, 16, 1, 8)
     assert plan(torch.float32, 4, 4096, 64, tuning=tuning) is not None

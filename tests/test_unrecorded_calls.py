@@ -42,10 +42,10 @@ def test_a_traced_call_is_not_a_constant():
     original = ops._nobody_watches
     try:
         ops._nobody_watches = lambda a, b: seen.append(original(a, b)) or seen[-1]
-        try:
-            torch.jit.trace(lambda a, b: linrec_amd.linrec(a, b), (x, c), check_trace=False)
-        except Exception:
-            pass  # (whether the tracer takes an autograd Function is torch's business)
+        traced = torch.jit.trace(lambda a, b: linrec_amd.linrec(a, b), (x, c), check_trace=False)
     finally:
         ops._nobody_watches = original
     assert seen and not any(seen)
+    assert any("_LinrecFn" in str(n) for n in traced.graph.nodes()), traced.graph
+    other, c2 = torch.randn_like(x), torch.rand_like(c)
+    assert torch.equal(traced(other, c2), linrec_amd.linrec(other, c2)) and not torch.equal(traced(other, c2), traced(x, c))
