@@ -26,13 +26,14 @@ constexpr LaneRows lookback_lane_rows(unsigned lane_no, unsigned rows, unsigned 
 // Segments dealt out at a time (collook_kernel.hpp): eight where that is as good or better, whole groups of which there are
 // at least two.  Forward / backward in us, eight against one: off the 128-byte lines fp32 8326 x 4022 (time x channels) 91.6 /
 // 140.7 against 98.0 / 150.2, 2 x 125567 x 222 165.9 / 244 against 172.4 / 251, bf16 8 x 4096 x 700 40.6 / 69.0 against 42.9 /
-// 73.2, but 3 x 1813 x 1464 (eight segments) 33.7 against 28.0; on them fp32 32768 x 1024 79.9 / 122.8 against 82.9 / 129.7,
-// 16 x 2048 x 512 43.6 / 66.8 against 39.5 / 69.5, bf16 32768 x 1024 47.6 / 67.6 against 44.4 / 68.8, of two blocks fp32
-// 16384 x 512 24.2 / 33.9 against 22.3 / 32.6; the 16-bit backward of sixteen blocks and more 1.09 in the geometric mean up to one
-// and a half rounds of workgroups and 1.02 beyond (fp16 2 x 3859 x 4160 71.1 against 62.0).
+// 73.2, in the geometric means of 1100 shapes 0.92 / 0.97 in fp32 and 0.94 / 0.93 in 16-bit storage, but 3 x 1813 x 1464 (eight
+// segments) 33.7 against 28.0.  On lines only the fp32 backward of many segments in a few blocks gains (32768 x 1024 122.8 against
+// 129.7, 0.99 in the mean of such shapes); the others lose the look-back's own locality, a block's segments being on one XCD when
+// its number alone decides that: 16 x 2048 x 512 backward 73.7 against 70.2, fp16 2 x 3859 x 4160 71.1 against 62.0, up to one and
+// a half rounds of workgroups 1.05 to 1.12 in the means; forward 1.02.
 constexpr long long lookback_segments_at_once(bool on_lines, bool is_bwd, bool half, long long blocks, long long segments) {
-  const bool eight = on_lines ? is_bwd && blocks >= 4 && !(half && blocks >= 16) : blocks >= 2;
-  return segments >= 16 && eight ? 8 : 1;
+  const bool eight = on_lines ? is_bwd && !half && blocks >= 4 && segments >= 100 : blocks >= 2 && segments >= 16;
+  return eight ? 8 : 1;
 }
 
 }  // namespace linrec
