@@ -19,16 +19,16 @@
 // 16 bytes get the same widths as the others.  The line at the border of two blocks is wanted by both: such launches load
 // through the caches, and eight segments are dealt out at a time so that the blocks of a segment run on one XCD and
 // find the border lines in its L2 (memory-only, 16640 x 4022, 8 bytes to a lane: 101.7 us as before, 93 with cached loads,
-// 85 with both; where positions start on lines cached loads cost 4 %).  That order also serves backwards on whole
-// lines (fp32 32768 x 1024 123 us instead of 130, 16384 x 4096 233 instead of 247; not 16-bit ones of many blocks), not forwards (16 x 2048 x 512 43.6
-// instead of 39.5).
+// 85 with both; where positions start on lines cached loads cost 4 %).  On whole lines
+// that order serves some fp32 backwards only (32768 x 1024 123 us instead of 130, 16384 x 4096 233 instead of 247; lookback_lanes.hpp),
+// not forwards (16 x 2048 x 512 43.6 instead of 39.5).
 //
 // Measured (medians of launches replayed from a graph over several buffer sets, forward / backward): bf16 1 x 4096 x 2048
 // (batch x time x channels) 15.1 / 22.0 us, 3.3 / 3.8 TB/s, where the three launches take 28.1 / 37.4; 8 x 4096 x 1024
 // 42.1 / 64.9 us, 4.8 / 5.2 TB/s, where the column drift kernels take 54.5 / 78.4; fp32 16 x 2048 x 512 39.5 / 66.8 us,
 // 5.1 / 5.0 TB/s, where column blocks / drift take 45.5 / 70.9.  Off the lines, with narrow aligned accesses in the order
-// of the segments before / now: fp32 2 x 125567 x 222 184 / 325 before, 166 / 244 now, bf16 131 / 227 and 90 / 149, 8 x 4096 x 175
-// 20.7 / 34.5 and 13.2 / 23.4, fp32 30 x 1024 x 1500 141 / 215 and 135 / 198.  What is left to the rate of a plain stream is
+// of the segments before / now: fp32 2 x 125567 x 222 189 / 329 before, 158 / 265 now, bf16 131 / 233 and 97 / 167, 8 x 4096 x 175
+// 20.0 / 35.3 and 13.0 / 24.3, fp32 30 x 1024 x 1500 137 / 203 and 126 / 206.  What is left to the rate of a plain stream is
 // the width of the accesses (bf16 8 x 4096 x 1024 with two rows to a lane instead of four 48.4 / 75.6 us, with one in eight
 // waves 52.9 / 82.8) and the one workgroup per CU, whose loads and stores do not overlap: a memory-only launch of this
 // shape takes 79 us for fp32 32768 x 1024 forward where small workgroups take 63, but smaller segments pay more for the

@@ -58,11 +58,12 @@ using linrec::lookback_segments_at_once;
 constexpr bool LINES = true, BWD = true, HALF = true;
 static_assert(lookback_segments_at_once(LINES, BWD, HALF, 33, 16) == 1 && lookback_segments_at_once(LINES, BWD, HALF, 4, 1000) == 1,
               "16-bit backwards on lines take one segment after the other");
-static_assert(lookback_segments_at_once(LINES, BWD, !HALF, 32, 16) == 1 && lookback_segments_at_once(LINES, BWD, !HALF, 32, 99) == 1,
-              "fp32 backwards on lines of few segments too");
-static_assert(lookback_segments_at_once(LINES, BWD, !HALF, 4, 100) == 8 && lookback_segments_at_once(LINES, BWD, !HALF, 3, 100) == 1);
+static_assert(lookback_segments_at_once(LINES, BWD, !HALF, 17, 100) == 1 && lookback_segments_at_once(LINES, BWD, !HALF, 32, 15) == 1,
+              "fp32 backwards on lines too, but of a multiple of four blocks");
+static_assert(lookback_segments_at_once(LINES, BWD, !HALF, 4, 16) == 8 && lookback_segments_at_once(LINES, BWD, !HALF, 2, 100) == 1);
 static_assert(lookback_segments_at_once(LINES, !BWD, !HALF, 33, 256) == 1 && lookback_segments_at_once(LINES, !BWD, HALF, 33, 256) == 1);
 static_assert(lookback_segments_at_once(!LINES, BWD, HALF, 33, 16) == 8 && lookback_segments_at_once(!LINES, !BWD, HALF, 2, 16) == 8);
+static_assert(lookback_segments_at_once(!LINES, BWD, !HALF, 176, 8) == 8 && lookback_segments_at_once(!LINES, BWD, HALF, 20, 7) == 1);
 static_assert(lookback_segments_at_once(!LINES, !BWD, HALF, 33, 15) == 1 && lookback_segments_at_once(!LINES, BWD, HALF, 1, 100) == 1);
 """
 
