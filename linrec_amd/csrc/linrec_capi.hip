@@ -719,9 +719,9 @@ int lookback_segments_plan(const Problem& q, int vec, int waves, int depth, int 
 //   up to 8192 rows (16-bit storage: 16384): fp32 16 x 2048 x 512 39.5 / 66.8 against 45.5 / 70.9 (column blocks,
 //     column drift), 2 x 8192 x 700 39.9 / 58.4 against 48.9 / 74.1, bf16 8 x 4096 x 1024 42.1 / 64.9 against 54.5 /
 //     78.4 (column drift), 16 x 2048 x 512 21.4 / 33.3 against 30.9 / 43, 4 x 4096 x 4096 87 / 148 against 89 / 143 (column blocks);
-//   more rows: where a position's rows do not start on a 128-byte line, fp32 30 x 1024 x 1500 135 / 198 against
-//     186 / 337, 8 x 1024 x 4097 99 / 145 against 143 / 252, bf16 7 x 4096 x 3500 162 / 281 against 219 / 397, 31 x 600 x 777
-//     33 / 54 against 45 / 83; where it does, the column blocks are as good or better (fp32 4 x 4096 x 4096 146 / 244 against
+//   more rows: where a position's rows do not start on a 128-byte line, fp32 30 x 1024 x 1500 126 / 206 against
+//     186 / 337, 8 x 1024 x 4097 89 / 157 against 143 / 252, bf16 7 x 4096 x 3500 141 / 253 against 219 / 397, 31 x 600 x 777
+//     37 / 54 against 45 / 83; where it does, the column blocks are as good or better (fp32 4 x 4096 x 4096 146 / 244 against
 //     138 / 242, 7 x 2048 x 4000 131 / 220 against 124 / 210, bf16 32 x 1024 x 1024 45.2 / 64.7 against 39.1 / 64.3);
 //   a forward of less than 1024 positions stays with the column blocks where positions start on lines (fp32 8 x 700 x 1024
 //     17.0 against 17.7), of less than 704 elsewhere (fp32 270 x 6544 9.1 against 10.9, 441 x 5810 13.4 against 13.0, 8 x 1001 x
@@ -811,15 +811,15 @@ bool lookback_segments_choose(const Problem& q, int family, int colblock, int mo
     // 28.3 / 35.3, 65536 x 512 44.4 / 68 against 72.5 / 94.8, 23633 x 2216 75.5 / 122.6 against 117.7 / 168.7, 35781 x 49 13.8 /
     // 15.9 against 25.1 / 30.4, fp32 backward 16384 x 512 32.6 against 50.8, 65536 x 512 125 against 160, 4096 x 256 11.8
     // against 16.2, 65536 x 4 19.3 against 23.4.  Where a position's rows do not start on 16 bytes both the three launches
-    // and the teams take narrow accesses, which cost most: fp32 8192 x 1025 29.6 / 44.2 against 53.7 / 79.5, 11944 x 2809
-    // 95.6 / 141 against 125 / 213, 8326 x 4022 91.6 / 140 against 115 / 214, bf16 11944 x 2809 57.9 / 96 against 151 / 227.
+    // and the teams take narrow accesses, which cost most: fp32 8192 x 1025 28.3 / 46.8 against 53.7 / 79.5, 11944 x 2809
+    // 86 / 141 against 125 / 213, 8326 x 4022 86.5 / 139 against 115 / 214, bf16 11944 x 2809 59 / 99 against 151 / 227.
     // The planner's tests fix the rest: the forwards of fp32 matrices, and of 16-bit ones of many rows and more than 8192
     // positions, that start on 16 bytes (fp32 16384 x 512 22.3 against 40.1, bf16 32768 x 1024 44.4 against 67.6), the teams
     // on such matrices (fp32 8192 x 2048 40.0 / 61.8 against 46.6 / 70.7, bf16 16384 x 4096 82 / 127 against 108 / 157), and
     // all column blocks of fp32 or of up to 1024 positions.
     if (family == LINREC_FAMILY_COLDRIFT && on_slots) return false;
     if (family == LINREC_FAMILY_SEGMENT && !q.is_bwd && on_slots && (!half || (q.seqlen > 8192 && on_lines && q.numseq >= q.at(1536)))) return false;
-    // (rows off 16 bytes that are too many for the column blocks: fp32 500 x 60001 83 / 139 against 122 / 221, bf16 46 / 76
+    // (rows off 16 bytes that are too many for the column blocks: fp32 500 x 60001 83 / 139 against 122 / 221, bf16 45 / 80
     // against 74 / 140)
     const bool many = !on_slots && q.numseq > q.at(32768) && q.numseq <= q.at(65536);
     if (family == LINREC_FAMILY_COLUMN && !many && (!colblock || !half || q.seqlen <= 1024)) return false;
