@@ -38,7 +38,10 @@
 // A segment's map multiplies 128 or 256 coefficients, and the look-back composes several: the product can overflow where
 // the recurrence does not (nothing put in yet, or small values that grow and shrink again).  Where what leaves a segment
 // comes out non-finite, its row takes the value that leaves the segment before and goes through the waves' maps of U
-// positions one after the other.
+// positions one after the other.  From the position on at which a row itself is infinite or NaN every segment of its block
+// does, so the segments follow each other about 0.9 us apart: bf16 65536 x 512 with an infinity after an eighth of the
+// positions takes 305 / 311 us (47 / 68 without; 69 / 95 in three launches either way), 588412 x 64 4.0 / 4.1 ms (90 / 117 us; 121 / 169),
+// 4096 x 2048 29 / 36 us (14 / 21).
 //
 // A segment only waits for segments with smaller numbers, which are started first; every wait is bounded, and a
 // lane whose wait runs out computes what enters its row from the row's own data.
